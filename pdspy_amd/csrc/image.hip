@@ -113,7 +113,7 @@ __device__ __forceinline__ float integrate_ray_l(const CamParams &C, Pos p, cons
     uint32_t nzero = 0;
     for (int guard = 0; guard < (1 << 24); ++guard) {
         int kind;
-        float tw = next_wall(C.g, p, kind);
+        float tw = next_wall<1>(C.g, p, kind);
         const float rcell = C.g.rw[p.ir + 1];
         if (p.ir >= 0) {
             ++nseg;
@@ -234,7 +234,7 @@ __device__ __forceinline__ void adjoint_ray(const CamParams &C, float X, float Y
     uint32_t nzero = 0;
     for (int guard = 0; guard < (1 << 24); ++guard) {
         int kind;
-        float tw = next_wall(C.g, p, kind);
+        float tw = next_wall<1>(C.g, p, kind);
         const float rcell = C.g.rw[p.ir + 1];
         if (p.ir >= 0) {
             ++nseg;
@@ -570,7 +570,7 @@ __global__ void k_stars(CamParams C, int nstar, const float *spos, StarArg sflux
     uint32_t nzero = 0;
     for (int guard = 0; guard < (1 << 24) && p.ir < g.nr; ++guard) {
         int kind;
-        float tw = next_wall(g, p, kind);
+        float tw = next_wall<1>(g, p, kind);
         const float rcell = g.rw[p.ir + 1];
         if (p.ir >= 0) tau += C.alpha[cell_index(g, p)] * tw;
         if (cross_wall(g, p, tw, kind)) break;
@@ -587,7 +587,7 @@ __global__ void k_stars(CamParams C, int nstar, const float *spos, StarArg sflux
     nzero = 0;
     for (int guard = 0; guard < (1 << 24) && p.ir < g.nr; ++guard) {
         int kind;
-        float tw = next_wall(g, p, kind);
+        float tw = next_wall<1>(g, p, kind);
         const float rcell = g.rw[p.ir + 1];
         if (p.ir >= 0)
             atomicAdd((u64 *)&g_alpha[cell_index(g, p)],

@@ -28,8 +28,11 @@ __device__ __forceinline__ void philox_block(uint32_t c0, uint32_t c1, uint32_t 
             k0 += 0x9E3779B9u;
             k1 += 0xBB67AE85u;
         }
-        uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
-        uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
+        // one 64-bit product per pair of halves (v_mad_u64_u32): the high and
+        // low words taken separately cost two quarter-rate multiplies each
+        const uint64_t m0 = (uint64_t)0xD2511F53u * c0, m1 = (uint64_t)0xCD9E8D57u * c2;
+        uint32_t hi0 = (uint32_t)(m0 >> 32), lo0 = (uint32_t)m0;
+        uint32_t hi1 = (uint32_t)(m1 >> 32), lo1 = (uint32_t)m1;
         uint32_t n0 = hi1 ^ c1 ^ k0, n2 = hi0 ^ c3 ^ k1;
         c0 = n0;
         c1 = lo1;
@@ -81,6 +84,20 @@ struct DevGrid {
     const float *sp;
 };
 
+// x a + y b with one rounding of the first product less: which of the two a
+// compiler fuses depends on the code around an inlined call, and a packet's
+// whole history on the last bit, so the choice is written out.  XF = 1: x a is
+// the fused one.  (next_wall's XF is the caller's: the thermal packets take 0,
+// the scattering source's 1.)
+template <int XF>
+__device__ __forceinline__ float sum2(float x, float a, float y, float b) {
+    return XF ? fmaf(x, a, y * b) : fmaf(y, b, x * a);
+}
+template <int XF>
+__device__ __forceinline__ double sum2(double x, double a, double y, double b) {
+    return XF ? fma(x, a, y * b) : fma(y, b, x * a);
+}
+
 enum { W_NONE = 0, W_ROUT, W_RIN, W_TLO, W_THI, W_PLO, W_PHI, W_HOLE };
 
 struct Pos {
@@ -107,8 +124,9 @@ __device__ __forceinline__ int search_walls(const float *w, int n, float v) {
     return lo;
 }
 
+template <int XF = 1>
 __device__ __forceinline__ void locate_angles(const DevGrid &g, Pos &p) {
-    float rho = sqrtf(p.x * p.x + p.y * p.y);
+    float rho = sqrtf(sum2<XF>(p.x, p.x, p.y, p.y));
     if (g.mirror) {
         p.hemi = (p.z >= 0.f) ? 1 : -1;
         p.it = search_walls(g.tw, g.nt, atan2f(rho, fabsf(p.z)));
@@ -127,8 +145,9 @@ __device__ __forceinline__ void locate_angles(const DevGrid &g, Pos &p) {
 
 // Cell of the position.  Every index is written once at the end (separate
 // early returns writing different fields would keep Pos out of registers).
+template <int XF = 1>
 __device__ __forceinline__ void locate(const DevGrid &g, Pos &p) {
-    float rr = p.x * p.x + p.y * p.y + p.z * p.z;
+    float rr = fmaf(p.z, p.z, sum2<XF>(p.x, p.x, p.y, p.y));
     const bool hole = rr < g.rw2[0], outside = !hole && rr >= g.rw2[g.nr];
     int ir;
     Pos q = p;
@@ -141,7 +160,7 @@ __device__ __forceinline__ void locate(const DevGrid &g, Pos &p) {
         ir = g.nr;
     } else {
         ir = search_walls(g.rw, g.nr, sqrtf(rr));
-        locate_angles(g, q);
+        locate_angles<XF>(g, q);
     }
     p.ir = ir;
     p.it = q.it;
@@ -157,27 +176,18 @@ __device__ __forceinline__ float sph_out(float b, float rr, float R2) {
     return fmaxf(t, 0.f);
 }
 
-// inner sphere; near-tangent cases (D small against b^2) are re-evaluated in
-// FP64 from the FP32 position so the hit/miss decision is consistent.  A
-// discriminant below -1e-5 (r^2 + R^2), twenty times its FP32 rounding bound,
-// is a miss without that check (most rays moving inwards miss the inner
-// sphere; one lane re-evaluating holds its whole wave).
-__device__ __forceinline__ float sph_in(const Pos &p, float b, float rr, float R2, double Rd) {
-    if (b >= 0.f) return RT_INF;
-    float c = rr - R2;
-    float D = fmaf(b, b, -c);
-    if (D < -1e-5f * (rr + R2)) return RT_INF;
-    if (D < 1e-4f * b * b) {
-        double bd = (double)p.x * p.dx + (double)p.y * p.dy + (double)p.z * p.dz;
-        double rrd = (double)p.x * p.x + (double)p.y * p.y + (double)p.z * p.z;
-        double cd = rrd - Rd * Rd;
-        double Dd = bd * bd - cd;
-        if (Dd < 0.0) return RT_INF;
-        double t = cd / (sqrt(Dd) - bd);
-        return t > 0.0 ? (float)t : 0.f;
-    }
-    float t = c / (sqrtf(D) - b);
-    return fmaxf(t, 0.f);
+// inner sphere, moving inwards (b < 0), where the discriminant is small against
+// b^2: FP64 from the FP32 position, so that hit or miss is decided consistently
+template <int XF>
+__device__ __forceinline__ float sph_in_d(const Pos &p, double Rd) {
+    const double xd = p.x, yd = p.y, zd = p.z;
+    double bd = fma(zd, (double)p.dz, sum2<XF>(xd, (double)p.dx, yd, (double)p.dy));
+    double rrd = fma(zd, zd, sum2<XF>(xd, xd, yd, yd));
+    double cd = fma(-Rd, Rd, rrd);
+    double Dd = fma(bd, bd, -cd);
+    if (Dd < 0.0) return RT_INF;
+    double t = cd / (sqrt(Dd) - bd);
+    return t > 0.0 ? (float)t : 0.f;
 }
 
 // Exit through the cone at polar angle th (folded frame): f = rho^2 cos^2 -
@@ -203,53 +213,61 @@ __device__ __forceinline__ float cone_root(double A, double B, double C, double 
     return (float)t;
 }
 
-__device__ __forceinline__ float cone_hit(float x, float y, float z, float dx, float dy,
-                                          float dz, float rr, float cth, float sth, double cthd,
-                                          double sthd, int req) {
-    float c2 = cth * cth, s2 = sth * sth;
-    float A = (dx * dx + dy * dy) * c2 - dz * dz * s2;
-    float B = (x * dx + y * dy) * c2 - z * dz * s2;
-    float C = (x * x + y * y) * c2 - z * z * s2;
+// what a ray and all cones have in common, in the folded frame
+struct ConeRay {
+    float z, dz, rr;
+    float dd, xd, rho2;     // dx^2 + dy^2, x dx + y dy, x^2 + y^2
+    float dz2, zdz, z2;
+};
+
+// the same in FP64, for the cone of cos/sin cthd, sthd (near tangency)
+template <int XF>
+__device__ __forceinline__ float cone_hit_d(float x, float y, float z, float dx, float dy, float dz,
+                                            double cthd, double sthd, float sreq) {
+    double c2d = cthd * cthd, s2d = sthd * sthd;
+    const double xd = x, yd = y, zd = z, dxd = dx, dyd = dy, dzd = dz;
+    double Ad = fma(sum2<XF>(dxd, dxd, dyd, dyd), c2d, -(dzd * dzd * s2d));
+    double Bd = fma(sum2<XF>(xd, dxd, yd, dyd), c2d, -(zd * dzd * s2d));
+    double Cd = fma(sum2<XF>(xd, xd, yd, yd), c2d, -(zd * zd * s2d));
+    double Dd = fma(Bd, Bd, -(Ad * Cd));
+    // no crossing: f keeps the sign of C along the whole line
+    if (Dd < 0.0) return Cd * sreq > 0.0 ? 0.f : RT_INF;
+    return cone_root(Ad, Bd, Cd, Dd, sreq > 0.f);
+}
+
+// Without branches but for the near-tangent one: a wave's lanes differ in
+// every one of these cases, so each branch was taken by some of them, and a
+// branch on a lone lane costs as much as the ten instructions it skips.
+template <int XF>
+__device__ __forceinline__ float cone_hit(const Pos &p, const ConeRay &q, float cth, float sth,
+                                          const double *cthd, const double *sthd, int req,
+                                          bool there) {
+    const float c2 = cth * cth, s2 = sth * sth;
+    const float A = fmaf(q.dd, c2, -(q.dz2 * s2));
+    const float B = fmaf(q.xd, c2, -(q.zdz * s2));
+    const float C = fmaf(q.rho2, c2, -(q.z2 * s2));
     // a ray lying in the cone (direction and position on it, as a radial ray
     // through the origin along a wall angle): it never leaves through it
-    if (fabsf(A) <= 1e-6f && fabsf(C) <= 1e-6f * (x * x + y * y + z * z)) return RT_INF;
-    float D = B * B - A * C;
+    const bool lies = fabsf(A) <= 1e-6f && fabsf(C) <= 1e-6f * (q.rho2 + q.z2);
+    const float D = fmaf(B, B, -(A * C));
     const float sreq = (float)(cth > 0.f ? req : -req);
-    int want_plus = sreq > 0.f;
-    float t;
-    if (D < -1e-5f * rr) {
-        // no crossing, clear of rounding (|A| <= 1, |B| <= r, |C| <= r^2, so D
-        // is good to a few ulp of r^2): as the FP64 test below would find
-        if (!(C * sreq > 0.f)) return RT_INF;
-        t = 0.f;
-    } else if (D < 1e-4f * B * B) {
-        double c2d = cthd * cthd, s2d = sthd * sthd;
-        double Ad = ((double)dx * dx + (double)dy * dy) * c2d - (double)dz * dz * s2d;
-        double Bd = ((double)x * dx + (double)y * dy) * c2d - (double)z * dz * s2d;
-        double Cd = ((double)x * x + (double)y * y) * c2d - (double)z * z * s2d;
-        double Dd = Bd * Bd - Ad * Cd;
-        if (Dd < 0.0) {
-            // no crossing: f keeps the sign of C along the whole line
-            if (!(Cd * sreq > 0.0)) return RT_INF;
-            t = 0.f;
-        } else {
-            t = cone_root(Ad, Bd, Cd, Dd, want_plus);
-        }
-    } else {
-        float sq = sqrtf(D);
-        if (want_plus)
-            t = (B < 0.f) ? (-B + sq) / A : -C / (B + sq);
-        else
-            t = (B > 0.f) ? -(B + sq) / A : C / (-B + sq);
-    }
-    if (!(t >= 0.f)) {
-        if (!(B * sreq > 0.f)) return RT_INF;
-        t = 0.f;
-    }
-    if (!(t < RT_INF)) return RT_INF;
-    float zh = fmaf(t, dz, z);
-    if (zh * cth < 0.f) return RT_INF;
-    return t;
+    // the root as one quotient: (-B + sq) / A or -C / (B + sq) for the larger,
+    // -(B + sq) / A or C / (-B + sq) for the other
+    const float sq = sqrtf(D);
+    const float s = sreq > 0.f ? B : -B;
+    const bool direct = s < 0.f;   // no cancellation in -B +- sq
+    const float u = sreq > 0.f ? (direct ? -B + sq : -C) : (direct ? -(B + sq) : C);
+    const float v = direct ? A : s + sq;
+    float t = u / v;
+    // no crossing, clear of rounding (|A| <= 1, |B| <= r, |C| <= r^2, so D is
+    // good to a few ulp of r^2): as the FP64 test would find
+    const bool clear = D < -1e-5f * q.rr;
+    t = clear ? (C * sreq > 0.f ? 0.f : RT_INF) : t;
+    if (there && !lies && !clear && D < 1e-4f * B * B)
+        t = cone_hit_d<XF>(p.x, p.y, q.z, p.dx, p.dy, q.dz, *cthd, *sthd, sreq);
+    t = t >= 0.f ? t : (B * sreq > 0.f ? 0.f : RT_INF);
+    const float zh = fmaf(t, q.dz, q.z);
+    return !there || lies || !(t < RT_INF) || zh * cth < 0.f ? RT_INF : t;
 }
 
 // Exit through the phi half-plane (cos ph, sin ph); a crossing just behind
@@ -257,96 +275,88 @@ __device__ __forceinline__ float cone_hit(float x, float y, float z, float dx, f
 // once, as for the cones.
 __device__ __forceinline__ float phi_hit(float x, float y, float dx, float dy, float cph,
                                          float sph, int req) {
-    float g0 = -x * sph + y * cph;
-    float g1 = -dx * sph + dy * cph;
-    if (req < 0 ? !(g1 < 0.f) : !(g1 > 0.f)) return RT_INF;
-    float t = fmaxf(-g0 / g1, 0.f);
+    float g0 = fmaf(y, cph, -(x * sph));
+    float g1 = fmaf(dy, cph, -(dx * sph));
+    const float t = fmaxf(-g0 / g1, 0.f);
     float xh = fmaf(t, dx, x), yh = fmaf(t, dy, y);
-    if (xh * cph + yh * sph < 0.f) return RT_INF;
-    return t;
+    const bool hit = (req < 0 ? g1 < 0.f : g1 > 0.f) && !(fmaf(xh, cph, yh * sph) < 0.f);
+    return hit ? t : RT_INF;
 }
 
 // distance to the next wall of the current cell and which wall it is
+template <int XF>
 __device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &kind) {
-    float rr = p.x * p.x + p.y * p.y + p.z * p.z;
-    float b = p.x * p.dx + p.y * p.dy + p.z * p.dz;
-    if (p.ir < 0) {
-        kind = W_HOLE;
-        return sph_out(b, rr, g.rw2[0]);
+    const bool in = p.ir >= 0;
+    const int i = in ? p.ir : 0, j = p.it;
+    // the walls' words first: one wait for all of them
+    const float R2o = g.rw2[p.ir + 1], R2i = g.rw2[i];
+    const float ctl = g.ct[j], stl = g.st[j], cth = g.ct[j + 1], sth = g.st[j + 1];
+    ConeRay q;
+    q.dd = sum2<XF>(p.dx, p.dx, p.dy, p.dy);
+    q.xd = sum2<XF>(p.x, p.dx, p.y, p.dy);
+    q.rho2 = sum2<XF>(p.x, p.x, p.y, p.y);
+    const float rr = fmaf(p.z, p.z, q.rho2);
+    const float b = fmaf(p.z, p.dz, q.xd);
+    q.rr = rr;
+    q.z = p.hemi > 0 ? p.z : -p.z;
+    q.dz = p.hemi > 0 ? p.dz : -p.dz;
+    q.dz2 = __fmul_rn(q.dz, q.dz);
+    q.zdz = __fmul_rn(q.z, q.dz);
+    q.z2 = __fmul_rn(q.z, q.z);
+    // outer sphere (from the inner hole: its wall)
+    float tb = sph_out(b, rr, R2o);
+    kind = in ? W_ROUT : W_HOLE;
+    // inner sphere.  A discriminant below -1e-5 (r^2 + R^2), twenty times its
+    // FP32 rounding bound, is a miss without the FP64 check
+    {
+        const float c = rr - R2i;
+        const float D = fmaf(b, b, -c);
+        const bool cand = in && b < 0.f && !(D < -1e-5f * (rr + R2i));
+        float t = fmaxf(c / (sqrtf(D) - b), 0.f);
+        if (cand && D < 1e-4f * b * b) t = sph_in_d<XF>(p, g.rwd[i]);
+        const bool hit = cand && t < tb;
+        tb = hit ? t : tb;
+        kind = hit ? W_RIN : kind;
     }
-    float tb = sph_out(b, rr, g.rw2[p.ir + 1]);
-    kind = W_ROUT;
-    float t = sph_in(p, b, rr, g.rw2[p.ir], g.rwd[p.ir]);
-    if (t < tb) {
-        tb = t;
-        kind = W_RIN;
+    // lower cone; the equatorial plane of a full-sphere grid is left upwards
+    // (a crossing behind the position is taken at once)
+    {
+        const bool plane = !g.mirror && ctl == 0.f;
+        float t = cone_hit<XF>(p, q, ctl, stl, g.ctd + j, g.std_ + j, -1, in && j > 0 && !plane);
+        if (!g.mirror && plane && in && j > 0 && p.dz > 0.f) t = fmaxf(-p.z / p.dz, 0.f);
+        const bool hit = t < tb;
+        tb = hit ? t : tb;
+        kind = hit ? W_TLO : kind;
     }
-    float zf = p.hemi > 0 ? p.z : -p.z, dzf = p.hemi > 0 ? p.dz : -p.dz;
-    int j = p.it;
-    if (j > 0) {
-        if (!g.mirror && g.ct[j] == 0.f) {
-            // the equatorial plane, left upwards (a crossing behind the
-            // position is taken at once)
-            if (p.dz > 0.f) {
-                t = fmaxf(-p.z / p.dz, 0.f);
-                if (t < tb) {
-                    tb = t;
-                    kind = W_TLO;
-                }
-            }
-        } else {
-            t = cone_hit(p.x, p.y, zf, p.dx, p.dy, dzf, rr, g.ct[j], g.st[j], g.ctd[j], g.std_[j],
-                         -1);
-            if (t < tb) {
-                tb = t;
-                kind = W_TLO;
-            }
-        }
-    }
-    if (g.mirror && j + 1 == g.nt) {
-        if (dzf < 0.f) {
-            t = fmaxf(-zf / dzf, 0.f);
-            if (t < tb) {
-                tb = t;
-                kind = W_THI;
-            }
-        }
-    } else if (j + 1 < g.nt) {
-        if (!g.mirror && g.ct[j + 1] == 0.f) {
-            if (p.dz < 0.f) {
-                t = fmaxf(-p.z / p.dz, 0.f);
-                if (t < tb) {
-                    tb = t;
-                    kind = W_THI;
-                }
-            }
-        } else {
-            t = cone_hit(p.x, p.y, zf, p.dx, p.dy, dzf, rr, g.ct[j + 1], g.st[j + 1],
-                         g.ctd[j + 1], g.std_[j + 1], +1);
-            if (t < tb) {
-                tb = t;
-                kind = W_THI;
-            }
-        }
+    // upper cone, or the mirror plane under the last row of cells
+    {
+        const bool last = j + 1 == g.nt;
+        const bool plane = !g.mirror && cth == 0.f;
+        float t = cone_hit<XF>(p, q, cth, sth, g.ctd + j + 1, g.std_ + j + 1, +1,
+                               in && !last && !plane);
+        const bool fold = g.mirror ? last && q.dz < 0.f : plane && !last && p.dz < 0.f;
+        const float tp = fmaxf(-q.z / q.dz, 0.f);
+        t = in && fold ? tp : t;
+        const bool hit = t < tb;
+        tb = hit ? t : tb;
+        kind = hit ? W_THI : kind;
     }
     if (g.np > 1) {
-        int k = p.ip;
-        t = phi_hit(p.x, p.y, p.dx, p.dy, g.cp[k], g.sp[k], -1);
-        if (t < tb) {
-            tb = t;
-            kind = W_PLO;
-        }
+        const int k = p.ip;
+        float t = phi_hit(p.x, p.y, p.dx, p.dy, g.cp[k], g.sp[k], -1);
+        bool hit = in && t < tb;
+        tb = hit ? t : tb;
+        kind = hit ? W_PLO : kind;
         t = phi_hit(p.x, p.y, p.dx, p.dy, g.cp[k + 1], g.sp[k + 1], +1);
-        if (t < tb) {
-            tb = t;
-            kind = W_PHI;
-        }
+        hit = in && t < tb;
+        tb = hit ? t : tb;
+        kind = hit ? W_PHI : kind;
     }
     return tb;
 }
 
 __device__ __forceinline__ void snap_radius(Pos &p, float R) {
-    float r = sqrtf(p.x * p.x + p.y * p.y + p.z * p.z);
+    float r = sqrtf(fmaf(p.z, p.z, sum2<1>(p.x, p.x, p.y, p.y)));
     if (r > 0.f) {
         float f = R / r;
         p.x *= f;
@@ -404,7 +414,7 @@ __device__ __forceinline__ bool unstick(const DevGrid &g, Pos &p, float tw, floa
     p.x = fmaf(d, p.dx, p.x);
     p.y = fmaf(d, p.dy, p.y);
     p.z = fmaf(d, p.dz, p.z);
-    locate(g, p);
+    locate<0>(g, p);
     return true;
 }
 
@@ -437,12 +447,14 @@ __device__ __forceinline__ void rotate_dir(float ct, float u2, float &dx, float 
         dy = st * sps;
         dz = (uz > 0.f ? 1.f : -1.f) * ct;
     } else {
-        float s = sqrtf(1.f - uz * uz);
-        dx = st * (ux * uz * cps - uy * sps) / s + ux * ct;
-        dy = st * (uy * uz * cps + ux * sps) / s + uy * ct;
-        dz = -st * cps * s + uz * ct;
+        // (fused as written: which of two products a compiler fuses depends on
+        // the code around an inlined call, and a packet's history on the last bit)
+        float s = sqrtf(fmaf(-uz, uz, 1.f));
+        dx = fmaf(ux, ct, st * fmaf(ux * uz, cps, -(uy * sps)) / s);
+        dy = fmaf(uy, ct, st * fmaf(uy * uz, cps, ux * sps) / s);
+        dz = fmaf(uz, ct, -(st * cps * s));
     }
-    float n = rsqrtf(dx * dx + dy * dy + dz * dz);
+    float n = rsqrtf(fmaf(dz, dz, fmaf(dx, dx, dy * dy)));
     dx *= n;
     dy *= n;
     dz *= n;
@@ -470,28 +482,28 @@ __device__ __forceinline__ void hg_dir(float u1, float u2, float g, float &dx, f
 // |theta - theta_j| <= pi/2 (else the axis, r); phi half-plane at phi_k:
 // |y cos phi_k - x sin phi_k| while |phi - phi_k| <= pi/2 (else rho).
 __device__ __forceinline__ float wall_dist(const DevGrid &g, const Pos &p) {
-    float r = sqrtf(p.x * p.x + p.y * p.y + p.z * p.z);
+    float r = sqrtf(fmaf(p.z, p.z, fmaf(p.x, p.x, p.y * p.y)));
     float d = fminf(r - g.rw[p.ir], g.rw[p.ir + 1] - r);
-    float rho = sqrtf(p.x * p.x + p.y * p.y);
+    float rho = sqrtf(fmaf(p.x, p.x, p.y * p.y));
     float zf = g.mirror ? fabsf(p.z) : p.z;
     int j = p.it;
     if (j > 0) {
-        float sn = rho * g.ct[j] - zf * g.st[j];
-        float cs = zf * g.ct[j] + rho * g.st[j];
+        float sn = fmaf(rho, g.ct[j], -(zf * g.st[j]));
+        float cs = fmaf(zf, g.ct[j], rho * g.st[j]);
         d = fminf(d, cs >= 0.f ? fabsf(sn) : r);
     }
     if (j + 1 < g.nt) {
-        float sn = rho * g.ct[j + 1] - zf * g.st[j + 1];
-        float cs = zf * g.ct[j + 1] + rho * g.st[j + 1];
+        float sn = fmaf(rho, g.ct[j + 1], -(zf * g.st[j + 1]));
+        float cs = fmaf(zf, g.ct[j + 1], rho * g.st[j + 1]);
         d = fminf(d, cs >= 0.f ? fabsf(sn) : r);
     }
     if (g.np > 1) {
         int k = p.ip;
-        float sn = p.y * g.cp[k] - p.x * g.sp[k];
-        float cs = p.x * g.cp[k] + p.y * g.sp[k];
+        float sn = fmaf(p.y, g.cp[k], -(p.x * g.sp[k]));
+        float cs = fmaf(p.x, g.cp[k], p.y * g.sp[k]);
         d = fminf(d, cs >= 0.f ? fabsf(sn) : rho);
-        sn = p.y * g.cp[k + 1] - p.x * g.sp[k + 1];
-        cs = p.x * g.cp[k + 1] + p.y * g.sp[k + 1];
+        sn = fmaf(p.y, g.cp[k + 1], -(p.x * g.sp[k + 1]));
+        cs = fmaf(p.x, g.cp[k + 1], p.y * g.sp[k + 1]);
         d = fminf(d, cs >= 0.f ? fabsf(sn) : rho);
     }
     return d;

@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(256) k_scat_mc(ScatParams P) {
         uint32_t k = 1, nev = 0, nzero = 0, nstep = 0;
         for (;;) {
             int kind;
-            const float tw = next_wall(g, p, kind);
+            const float tw = next_wall<1>(g, p, kind);
             float aabs = 0.f, asca = 0.f;
             int c = -1;
             if (p.ir >= 0) {

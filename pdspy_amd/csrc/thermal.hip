@@ -941,7 +941,7 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
             aRc = -1.f;
         }
         int kind;
-        float tw = next_wall(g, p, kind);
+        float tw = next_wall<0>(g, p, kind);
         float aabs = 0.f, asca = 0.f;
         if (c >= 0) {
 #pragma unroll
