@@ -54,6 +54,7 @@
 // those of its plain run bit for bit.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -133,6 +134,13 @@ struct BatchArgs {
     unsigned long long *abort;     // [1] watchdog flag
     unsigned int *runs_done;       // [1] runs whose last snapshot is published
     int *parked;                   // [1] packets parked in the runs' pools (batch)
+};
+
+// the kernel's arguments as they lie in its argument segment
+struct KernelArgs {
+    BatchArgs A;
+    const ThermParams *runs;
+    ThermParams P1;
 };
 
 #define RT_PARK_WORDS 22   // words of a parked packet's state
@@ -224,26 +232,41 @@ __device__ __forceinline__ float xrow_of(const double *lq, int ntemp, double e) 
     return (float)(m + (le - lq[m]) / (lq[m + 1] - lq[m]));
 }
 
-// Adds the packet's pending deposits to the tallies of cell c with atomics
+// Adds the packet's pending deposits to the tallies of cell c in its slot with atomics
 // whose result nobody waits for.  Overflow is ruled out by bounds instead of
 // by the values the atomics find: every add stays below 2^62 (ovf), and the
 // packet's adds into its current slot are summed (ssum, FP64) and added to the
 // slot's total when the packet leaves the slot; a slot whose total of adds
 // stays below 2^61 has no tally near 2^64 (checked after the launch).
-template <int MG>
-__device__ __forceinline__ void flush_tally(const ThermParams &P, unsigned long long *tb, int c,
+// ALL: also adds of 0 (an atomic the compiler can count on).
+template <int MG, bool ALL = false>
+__device__ __forceinline__ void flush_tally(const ThermParams &P, int slot, int c,
                                             unsigned long long (&acc)[MG],
-                                            unsigned long long &ovf, double &ssum) {
+                                            unsigned &ovf, double &ssum) {
+    unsigned long long *const tb = P.tslot + (size_t)slot * P.slot;
 #pragma unroll
     for (int q = 0; q < MG; ++q) {
-        if (q < P.ngroup && acc[q]) {
-            ovf |= acc[q];
+        if ((MG == 1 || q < P.ngroup) && (ALL || acc[q])) {
+            ovf |= (unsigned)(acc[q] >> 32);
             ssum += (double)acc[q];
-            __hip_atomic_fetch_add(&tb[(size_t)c * P.ngroup + q], acc[q], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(&tb[(size_t)c * (MG == 1 ? 1 : P.ngroup) + q], acc[q],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             acc[q] = 0;
         }
     }
+}
+
+// requests cell c's densities and the temperature rows a packet of epoch pe
+// sees there (none before epoch 2: T = 0)
+template <int MS, int MG>
+__device__ __forceinline__ void load_cell(const ThermParams &P, int pe, int c, int S, int G,
+                                          float (&rcache)[MS], float (&xcache)[MG]) {
+    const float *xs = P.xsnap + (size_t)(pe - 2) * P.slot;
+    const float *rc = P.rhoL + (size_t)c * S;
+#pragma unroll
+    for (int s = 0; s < MS; ++s) rcache[s] = s < S ? rc[s] : 0.f;
+#pragma unroll
+    for (int q = 0; q < MG; ++q) xcache[q] = (q < G && pe >= 2) ? xs[(size_t)c * G + q] : -1.f;
 }
 
 // the packet leaves slot `slot`: its adds there join the slot's total
@@ -437,7 +460,7 @@ __device__ __forceinline__ void wave_count(unsigned *row, int k, int lane) {
 
 // adds the wave's counts to run R's counters and clears them (whole wave)
 __device__ __forceinline__ void flush_counts(const ThermParams &R, int lane, unsigned *row,
-                                             unsigned long long &ovf) {
+                                             unsigned &ovf) {
     if (lane == 0) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -447,7 +470,7 @@ __device__ __forceinline__ void flush_counts(const ThermParams &R, int lane, uns
         if (row[8]) atomicMax(&R.cnt[CNT_MAXPKT], (unsigned long long)row[8]);
         row[8] = 0u;
     }
-    if (__any((ovf >> 62) != 0ull) && lane == 0) atomicOr(&R.cnt[CNT_OVERFLOW], 1ull);
+    if (__any((ovf >> 30) != 0u) && lane == 0) atomicOr(&R.cnt[CNT_OVERFLOW], 1ull);
     ovf = 0;
 }
 
@@ -480,6 +503,14 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
     // the run this wave serves (wave-uniform; -1: none yet) and its staged data
     int m = -1;
     const ThermParams *Pp = BATCH ? runs : &P1;
+    // (one run) where the argument block lies; the loop hides the address from
+    // the compiler once per pass, so that the block's words are read again
+    // (scalar cache) instead of being held over the loop in more scalar
+    // registers than there are
+    typedef const __attribute__((address_space(4))) ThermParams *ConstParams;
+    uint64_t p1a = (uint64_t)((const __attribute__((address_space(4))) char *)
+                                  __builtin_amdgcn_kernarg_segment_ptr() +
+                              offsetof(KernelArgs, P1));
 #define P (*Pp)
     int S = 0, NL = 0, G = 0, E = 0;
     DevGrid g = P.g;  // LDS pointers set below, FP64 walls stay in global memory
@@ -515,12 +546,12 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
     uint32_t nev = 0, nstep = 0, nev_cell = 0, nzero = 0;
     uint32_t slice_left = 0;  // interactions until the packet moves to the next slot
     bool alive = false;
-    int pe = 0;                                // epoch of this lane's packet
-    int slot = 0;                              // its current deposit slot
-    const float *xs = nullptr;                 // its temperature snapshot (null: T = 0)
-    unsigned long long *tb = nullptr;          // its deposit slot's tallies
-    int ccell = -1;                            // cell whose data sit in registers
-    float aRc = -1.f;                          // its Rosseland extinction (-1: not yet)
+    int ps = 0;  // epoch of this lane's packet, and above 16 bits its deposit slot
+#define RT_PE (ps & 0xffff)
+#define RT_SLOT (ps >> 16)
+    // Rosseland extinction of the cell whose data sit in registers (-1: not yet;
+    // -2: the packet has just started, no cell's data are there)
+    float aRc = -2.f;
     float rcache[MS];
     float xcache[MG];
 #pragma unroll
@@ -528,7 +559,7 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
 #pragma unroll
     for (int q = 0; q < MG; ++q) xcache[q] = -1.f;
     unsigned long long acc[MG];
-    unsigned long long ovf = 0;  // OR of the adds (overflow check)
+    unsigned ovf = 0;            // OR of the adds' high words (overflow check)
     double ssum = 0.0;           // the packet's adds into its current slot
 #pragma unroll
     for (int q = 0; q < MG; ++q) acc[q] = 0;
@@ -583,7 +614,12 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
         NL = (int)uniform32((unsigned)NL);
         G = (int)uniform32((unsigned)G);
         E = (int)uniform32((unsigned)E);
-        Pp = BATCH ? runs + (m < 0 ? 0 : m) : &P1;
+        if (BATCH) {
+            Pp = runs + (m < 0 ? 0 : m);
+        } else {
+            __asm__ volatile("" : "+s"(p1a));
+            Pp = (const ThermParams *)(ConstParams)p1a;
+        }
         const bool any0 = __any(alive);
 
         // ---- watchdog (wave-uniform check)
@@ -593,8 +629,8 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
             if (stop) {
                 if (lane == 0) atomicOr(A.abort, 1ull);
                 if (alive) {
-                    if (p.ir >= 0) flush_tally(P, tb, cell_index(g, p), acc, ovf, ssum);
-                    flush_ssum(P, slot, ssum);
+                    if (p.ir >= 0) flush_tally(P, RT_SLOT, cell_index(g, p), acc, ovf, ssum);
+                    flush_ssum(P, RT_SLOT, ssum);
                     RT_MAXPKT(nev + nstep);
                     RT_COUNT(4);
                     alive = false;
@@ -730,8 +766,8 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                 ok = lane64(ok, leader);
                 base = lane64(base, leader);
                 if (ok && alive) {
-                    if (p.ir >= 0) flush_tally(P, tb, cell_index(g, p), acc, ovf, ssum);
-                    flush_ssum(P, slot, ssum);
+                    if (p.ir >= 0) flush_tally(P, RT_SLOT, cell_index(g, p), acc, ovf, ssum);
+                    flush_ssum(P, RT_SLOT, ssum);
                     const unsigned long long idx = base + __popcll(live & ((1ull << lane) - 1ull));
                     const size_t s0 = (size_t)(idx % P.park_cap);
                     unsigned *w = P.park + s0 * RT_PARK_WORDS;
@@ -763,8 +799,8 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                     park_put(w, 17, nev_cell);
                     park_put(w, 18, nzero);
                     park_put(w, 19, slice_left);
-                    park_put(w, 20, (unsigned)pe);
-                    park_put(w, 21, (unsigned)slot);
+                    park_put(w, 20, (unsigned)RT_PE);
+                    park_put(w, 21, (unsigned)RT_SLOT);
                     order_release();
                     st_rlx32(&P.park_flag[s0], (unsigned)(idx + 1ull));
                     alive = false;
@@ -778,7 +814,9 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
         }
 
         // ---- refill dead lanes with packets of the current epoch
-        if (cur_e < E && !epoch_ok) {
+        // (a wave with packets to step looks for the snapshot now and then: the
+        // device-coherent read takes as long as a step)
+        if (cur_e < E && !epoch_ok && (!any0 || (iter & 7u) == 0u)) {
             epoch_ok = cur_e < 2 || uniform32(ld_rlx32(&P.snap_ready[cur_e - 2])) != 0u;
             if (epoch_ok) order_acquire();
         }
@@ -842,14 +880,10 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                             nev_cell = park_get(w, 17);
                             nzero = park_get(w, 18);
                             slice_left = park_get(w, 19);
-                            pe = (int)park_get(w, 20);
-                            slot = (int)park_get(w, 21);
+                            ps = (int)park_get(w, 20) | (int)park_get(w, 21) << 16;
                             order_release();  // read before the slot is handed back
                             st_rlx32(&P.park_flag[s0], 0u);
-                            xs = pe >= 2 ? P.xsnap + (size_t)(pe - 2) * P.slot : nullptr;
-                            tb = P.tslot + (size_t)slot * P.slot;
-                            ccell = -1;
-                            aRc = -1.f;
+                            aRc = -2.f;
                             alive = true;
                         } else {
                             atomicOr(A.abort, 1ull);  // a lost packet: the run is invalid
@@ -875,10 +909,7 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                     uint64_t idx = base + __popcll(need & ((1ull << lane) - 1ull));
                     if (idx < size) {
                         pid = e0 + idx;
-                        pe = cur_e;
-                        slot = pe;
-                        xs = pe >= 2 ? P.xsnap + (size_t)(pe - 2) * P.slot : nullptr;
-                        tb = P.tslot + (size_t)pe * P.slot;
+                        ps = cur_e | cur_e << 16;
                         // emission (random event 0): star, frequency, direction, tau
                         float u[8];
                         rng8(P.seed, pid, 0u, u);
@@ -897,10 +928,10 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                         nev_cell = 0;
                         nzero = 0;
                         slice_left = P.slice;
-                        ccell = -1;
+                        aRc = -2.f;
                         if (p.ir >= g.nr) {
                             RT_COUNT(3);
-                            count_up(&P.slot_out[pe]);
+                            count_up(&P.slot_out[RT_PE]);
                         } else {
                             alive = true;
                             if (p.ir >= 0 && P.visits) atomicAdd(&P.visits[cell_index(g, p)], 1u);
@@ -926,19 +957,20 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
         RT_PHASE(0);
         if (!alive) continue;
 
-        // ---- one step: to the next wall or to the next interaction
-        // (a new cell's data are requested first, the wall distances computed
-        // while they arrive)
+        // ---- one step: to the next wall or to the next interaction.  A cell's
+        // data are requested at the crossing that enters it (below) and used one
+        // next_wall later; only a packet that has just started or been adopted
+        // reads them here.  The reads of this branch are waited for inside it,
+        // so that the wait after the branch counts only the crossing's requests
+        // and not the tally atomic issued behind them.
         const int c = p.ir >= 0 ? cell_index(g, p) : -1;
-        if (c >= 0 && c != ccell) {
-            const float *rc = P.rhoL + (size_t)c * S;
-#pragma unroll
-            for (int s = 0; s < MS; ++s) rcache[s] = s < S ? rc[s] : 0.f;
-#pragma unroll
-            for (int q = 0; q < MG; ++q)
-                xcache[q] = (q < G && xs) ? xs[(size_t)c * G + q] : -1.f;
-            ccell = c;
+        if (c >= 0 && aRc == -2.f) {
+            load_cell<MS, MG>(P, RT_PE, c, S, G, rcache, xcache);
             aRc = -1.f;
+#pragma unroll
+            for (int s = 0; s < MS; ++s) __asm__ volatile("" : "+v"(rcache[s]));
+#pragma unroll
+            for (int q = 0; q < MG; ++q) __asm__ volatile("" : "+v"(xcache[q]));
         }
         int kind;
         float tw = next_wall<0>(g, p, kind);
@@ -967,14 +999,13 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
             nev++;
             nev_cell++;
             nzero = 0;
-            if (--slice_left == 0u && slot < E) {
+            if (--slice_left == 0u && RT_SLOT < E) {
                 // next slot: earlier deposits are final for snapshots <= slot
-                flush_tally(P, tb, c, acc, ovf, ssum);
-                flush_ssum(P, slot, ssum);
-                if (slot + 1 < E) count_up(&P.slot_in[slot + 1]);
-                count_up(&P.slot_out[slot]);
-                slot++;
-                tb = P.tslot + (size_t)slot * P.slot;
+                flush_tally(P, RT_SLOT, c, acc, ovf, ssum);
+                flush_ssum(P, RT_SLOT, ssum);
+                if (RT_SLOT + 1 < E) count_up(&P.slot_in[RT_SLOT + 1]);
+                count_up(&P.slot_out[RT_SLOT]);
+                ps += 1 << 16;
             }
             if (slice_left == 0u) slice_left = P.slice;
             // interaction (one random event): u0 scatter or absorb, u1 species,
@@ -1027,12 +1058,12 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
             tau = -__logf(u[6]);
             RT_PHASE(6);
             if (P.max_events && nev >= P.max_events) {
-                flush_tally(P, tb, c, acc, ovf, ssum);
-                flush_ssum(P, slot, ssum);
+                flush_tally(P, RT_SLOT, c, acc, ovf, ssum);
+                flush_ssum(P, RT_SLOT, ssum);
                 RT_MAXPKT(nev + nstep);
                 RT_COUNT(4);
                 alive = false;
-                if (slot < E) count_up(&P.slot_out[slot]);
+                if (RT_SLOT < E) count_up(&P.slot_out[RT_SLOT]);
                 continue;
             }
             if (P.mrw && nev_cell >= (uint32_t)P.mrw_count) {
@@ -1108,7 +1139,6 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                 for (int q = 0; q < MG; ++q)
                     if (q < G)
                         acc[q] += (unsigned long long)rintf(s_gka[q * NL + ifr] * wf);
-                flush_tally(P, tb, c, acc, ovf, ssum);
             }
             tau -= aext * tw;
             RT_COUNT(0);
@@ -1128,12 +1158,22 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                     end = true;
                 }
             }
+            // the new cell's data first, then the tally of the cell left: vmcnt
+            // counts in issue order, and a device-scope atomic takes several
+            // times as long as a read, so a read issued behind it waits for it
+            if (!end && p.ir >= 0) {
+                load_cell<MS, MG>(P, RT_PE, cell_index(g, p), S, G, rcache, xcache);
+                aRc = -1.f;
+            }
+            // (a packet in the inner hole adds 0: the atomic stays unconditional,
+            // which lets the compiler count it)
+            flush_tally<MG, true>(P, RT_SLOT, c >= 0 ? c : 0, acc, ovf, ssum);
             RT_PHASE(5);
             if (end) {
-                flush_ssum(P, slot, ssum);
+                flush_ssum(P, RT_SLOT, ssum);
                 RT_MAXPKT(nev + nstep);
                 alive = false;
-                if (slot < E) count_up(&P.slot_out[slot]);
+                if (RT_SLOT < E) count_up(&P.slot_out[RT_SLOT]);
                 continue;
             }
             if (p.ir >= 0 && P.visits) atomicAdd(&P.visits[cell_index(g, p)], 1u);
@@ -1159,6 +1199,8 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
 #undef RT_PHASE
 #undef RT_COUNT
 #undef RT_MAXPKT
+#undef RT_PE
+#undef RT_SLOT
 #undef P
 }
 
