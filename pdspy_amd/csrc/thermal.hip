@@ -480,6 +480,112 @@ __device__ __forceinline__ void flush_counts(const ThermParams &R, int lane, uns
 #define RT_THERMAL_WAVES 4
 #endif
 
+// ---- random walks inside one cell -------------------------------------------
+// A packet deep in an optically thick cell interacts thousands of times without
+// leaving it, and those walks are what an epoch's snapshot and the end of a run
+// wait for: one lane of a wave, one interaction per pass of the loop below
+// (3.2 us: every pass computes the distances to the cell's walls, two Philox
+// blocks, a direction and a re-emission, all of it one after the other on one
+// lane).  walk_cell() takes up to 64 interactions of one packet at once.  The
+// random numbers of interaction k depend on k alone, so lane i draws those of
+// the packet's i-th next interaction, and with them its direction, its optical
+// depth and -- the cell's temperature being fixed -- the frequency it would be
+// re-emitted at and that frequency's opacities.  What is left in order is short:
+// the flight's length, the tally, the position, scattering or absorption.
+// The distances to the walls are not needed while the flight is shorter than a
+// lower bound of them: the perpendicular distance to the nearest wall
+// (wall_dist, the equatorial mirror plane included), less the lengths flown
+// since, less a margin over the rounding of the positions and of next_wall.  A
+// flight beyond the bound, a modified-random-walk step, the last interaction of
+// a slice and the max_events-th are left to the loop.  Every operation on the
+// packet is the loop's own, in the same order: its history is the same bit for
+// bit.
+#ifndef RT_WALK_LIVE
+#define RT_WALK_LIVE 2    // waves with at most this many live packets look for walks
+#endif
+#define RT_WALK_FROM 4    // interactions in the cell before a packet is looked at
+#define RT_WALK_MIN 3.0f  // optical depth to the bound from which a walk is worth its draws
+
+struct CellWalls {
+    float r0, r1, ct0, st0, ct1, st1, cp0, sp0, cp1, sp1;
+    bool lo, hi, phi, mirror, eq;  // which walls there are; eq: the mirror plane is one
+};
+
+__device__ __forceinline__ CellWalls cell_walls(const DevGrid &g, int ir, int it, int ip) {
+    CellWalls w;
+    w.r0 = g.rw[ir];
+    w.r1 = g.rw[ir + 1];
+    w.lo = it > 0;
+    w.hi = it + 1 < g.nt;
+    w.mirror = g.mirror != 0;
+    w.eq = w.mirror && !w.hi;
+    w.phi = g.np > 1;
+    w.ct0 = g.ct[it];
+    w.st0 = g.st[it];
+    w.ct1 = g.ct[it + 1];
+    w.st1 = g.st[it + 1];
+    w.cp0 = g.cp[ip];
+    w.sp0 = g.sp[ip];
+    w.cp1 = g.cp[ip + 1];
+    w.sp1 = g.sp[ip + 1];
+    return w;
+}
+
+// wall_dist (rt_device.h) with the cell's walls at hand: the same operations
+__device__ __forceinline__ float walls_dist(const CellWalls &w, float x, float y, float z) {
+    const float r = sqrtf(fmaf(z, z, fmaf(x, x, y * y)));
+    float d = fminf(r - w.r0, w.r1 - r);
+    const float rho = sqrtf(fmaf(x, x, y * y));
+    const float zf = w.mirror ? fabsf(z) : z;
+    if (w.lo) {
+        const float sn = fmaf(rho, w.ct0, -(zf * w.st0)), cs = fmaf(zf, w.ct0, rho * w.st0);
+        d = fminf(d, cs >= 0.f ? fabsf(sn) : r);
+    }
+    if (w.hi) {
+        const float sn = fmaf(rho, w.ct1, -(zf * w.st1)), cs = fmaf(zf, w.ct1, rho * w.st1);
+        d = fminf(d, cs >= 0.f ? fabsf(sn) : r);
+    }
+    if (w.phi) {
+        float sn = fmaf(y, w.cp0, -(x * w.sp0)), cs = fmaf(x, w.cp0, y * w.sp0);
+        d = fminf(d, cs >= 0.f ? fabsf(sn) : rho);
+        sn = fmaf(y, w.cp1, -(x * w.sp1));
+        cs = fmaf(x, w.cp1, y * w.sp1);
+        d = fminf(d, cs >= 0.f ? fabsf(sn) : rho);
+    }
+    return d;
+}
+
+// lower bound of the distance to the cell's walls for up to 64 flights, by
+// signed distances (a packet a hair past a wall that its index has not crossed
+// yet has none), less a margin: the positions round to ulps of r (6e-8 r
+// each), next_wall to a few more.  Next to a cone that is a plane but for the
+// rounding of pi/2 -- the equator of a grid over [0, pi] -- there is no bound:
+// next_wall's quadratic has a double root there.
+__device__ __forceinline__ float walk_bound(const CellWalls &w, float x, float y, float z) {
+    const float rho = sqrtf(fmaf(x, x, y * y)), r = sqrtf(fmaf(z, z, rho * rho));
+    const float zf = w.mirror ? fabsf(z) : z;
+    float d = fminf(r - w.r0, w.r1 - r);
+    if (w.lo) {
+        d = fminf(d, fmaf(rho, w.ct0, -(zf * w.st0)));
+        if (fabsf(w.ct0) < 1e-4f) d = -1.f;
+    }
+    if (w.hi) {
+        d = fminf(d, fmaf(zf, w.st1, -(rho * w.ct1)));
+        if (fabsf(w.ct1) < 1e-4f) d = -1.f;
+    }
+    if (w.eq) d = fminf(d, zf);
+    if (w.phi) {
+        const float c0 = fmaf(x, w.cp0, y * w.sp0), c1 = fmaf(x, w.cp1, y * w.sp1);
+        d = fminf(d, c0 >= 0.f ? fmaf(y, w.cp0, -(x * w.sp0)) : rho);
+        d = fminf(d, c1 >= 0.f ? fmaf(x, w.sp1, -(y * w.cp1)) : rho);
+    }
+    return fmaf(-1e-5f, w.r1, d) * 0.999f;
+}
+
+__device__ __forceinline__ float lanef(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+
 // One persistent launch for a batch of runs (one model each).  Each wavefront
 // serves one run at a time: its LDS slice holds that run's opacities and
 // walls; when it has no packet left and the run has none to hand out (all
@@ -730,6 +836,196 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
             }
         }
         RT_PHASE(2);
+
+        // ---- random walks inside one cell (see walk_bound): the wave's sparse
+        // packets one after the other
+        if (MG <= 2 && (MG == 1 || MS <= 2)) {
+            const uint64_t live = __ballot(alive);
+            if (live && __popcll(live) <= RT_WALK_LIVE) {
+                bool el = alive && nev_cell >= RT_WALK_FROM && p.ir >= 0 && slice_left > 8u;
+                if (__any(el)) {
+                    if (el) {
+                        float a = 0.f;
+#pragma unroll
+                        for (int s = 0; s < MS; ++s)
+                            if (s < S) {
+                                a = fmaf(rcache[s], s_ka[s * NL + ifr], a);
+                                a = fmaf(rcache[s], s_ks[s * NL + ifr], a);
+                            }
+                        const CellWalls w = cell_walls(g, p.ir, p.it, p.ip);
+                        el = a * walk_bound(w, p.x, p.y, p.z) > RT_WALK_MIN;
+                    }
+                    for (uint64_t todo = __ballot(el); todo; todo &= todo - 1ull) {
+                        const int L = (int)uniform32(
+                            (unsigned)(__ffsll((unsigned long long)todo) - 1));
+                        // the packet of lane L, the same in every lane
+                        const uint64_t w_pid = lane64(pid, L);
+                        const uint32_t k0 = (uint32_t)__builtin_amdgcn_readlane((int)krng, L);
+                        const uint32_t w_nev = (uint32_t)__builtin_amdgcn_readlane((int)nev, L);
+                        const uint32_t w_nc = (uint32_t)__builtin_amdgcn_readlane((int)nev_cell, L);
+                        const uint32_t w_sl = (uint32_t)__builtin_amdgcn_readlane((int)slice_left, L);
+                        uint32_t nmax = min(64u, w_sl - 1u);
+                        if (P.max_events)
+                            nmax = min(nmax, (uint32_t)std::min<uint64_t>(
+                                                 64u, P.max_events - 1u - std::min<uint64_t>(
+                                                          P.max_events - 1u, w_nev)));
+                        const int w_ir = __builtin_amdgcn_readlane(p.ir, L);
+                        const CellWalls w =
+                            cell_walls(g, w_ir, __builtin_amdgcn_readlane(p.it, L),
+                                       __builtin_amdgcn_readlane(p.ip, L));
+                        const float inv = s_invdr[w_ir];
+                        float rho[MS], xr[MG];
+#pragma unroll
+                        for (int s = 0; s < MS; ++s) rho[s] = lanef(rcache[s], L);
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) xr[q] = lanef(xcache[q], L);
+                        // this lane's interaction of the next 64
+                        float u[8];
+                        rng8(P.seed, w_pid, k0 + (uint32_t)lane, u);
+                        float ex, ey, ez;
+                        iso_dir(u[4], u[5], ex, ey, ez);
+                        const float etau = -__logf(u[6]);
+                        int ec[MG];                         // re-emitted at, per group
+                        float eabs[MG], esca[MG], e0[MG];   // its opacities (e0: first species)
+                        float ek[MG][MG];                   // and tally factors
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) {
+                            ec[q] = 0;
+                            eabs[q] = esca[q] = e0[q] = 0.f;
+                            if (MG == 1 || q < G) {
+                                const float x = fminf(fmaxf(xr[q], 0.f), (float)(P.ntemp - 1));
+                                const int lo = min((int)x, P.ntemp - 2);
+                                const float wt = x - (float)lo;
+                                const int row = lo + (u[2] < wt ? 1 : 0);
+                                const size_t ro = (size_t)q * P.ntemp + row;
+                                ec[q] = sample_guided(P.cdf + ro * NL, P.guide + ro * RT_NGUIDE,
+                                                      u[3]);
+#pragma unroll
+                                for (int s = 0; s < MS; ++s)
+                                    if (s < S) {
+                                        eabs[q] = fmaf(rho[s], s_ka[s * NL + ec[q]], eabs[q]);
+                                        esca[q] = fmaf(rho[s], s_ks[s * NL + ec[q]], esca[q]);
+                                        if (s == 0) e0[q] = eabs[q];
+                                    }
+                            }
+#pragma unroll
+                            for (int t = 0; t < MG; ++t)
+                                ek[q][t] = (MG == 1 || (q < G && t < G)) ? s_gka[t * NL + ec[q]] : 0.f;
+                        }
+                        // the packet's own state
+                        int f = __builtin_amdgcn_readlane(ifr, L);
+                        float x = lanef(p.x, L), y = lanef(p.y, L), z = lanef(p.z, L);
+                        float dx = lanef(p.dx, L), dy = lanef(p.dy, L), dz = lanef(p.dz, L);
+                        float tl = lanef(tau, L), aR = lanef(aRc, L);
+                        float cabs = 0.f, csca = 0.f, c0 = 0.f, ck[MG];
+#pragma unroll
+                        for (int s = 0; s < MS; ++s)
+                            if (s < S) {
+                                cabs = fmaf(rho[s], s_ka[s * NL + f], cabs);
+                                csca = fmaf(rho[s], s_ks[s * NL + f], csca);
+                                if (s == 0) c0 = cabs;
+                            }
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) ck[q] = (MG == 1 || q < G) ? s_gka[q * NL + f] : 0.f;
+                        unsigned long long add[MG];
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) add[q] = 0;
+                        float lowd = walk_bound(w, x, y, z);
+                        uint32_t n = 0, nsc = 0;
+                        for (; n < nmax; ++n) {
+                            const float cext = cabs + csca;
+                            const float sseg = tl / cext;
+                            if (!(sseg < lowd)) break;
+                            const float nx = fmaf(sseg, dx, x), ny = fmaf(sseg, dy, y),
+                                        nz = fmaf(sseg, dz, z);
+                            if (P.mrw && w_nc + n + 1u >= (uint32_t)P.mrw_count) {
+                                if (aR < 0.f) {
+                                    float a = 0.f;
+                                    for (int s = 0; s < S; ++s) {
+                                        const float rs = pickn<MS>(rho, s);
+                                        if (rs > 0.f)
+                                            a = fmaf(rs, trow(P.kross + (size_t)s * P.ntemp, P.ntemp,
+                                                              pickn<MG>(xr, pickn<MS>(grpr, s))), a);
+                                    }
+                                    aR = a;
+                                }
+                                const float dmin = walls_dist(w, nx, ny, nz);
+                                if (aR * dmin >= P.mrw_tau && dmin - P.mrw_gamma / aR > 0.f) break;
+                            }
+                            const float wf = inv * sseg;
+#pragma unroll
+                            for (int q = 0; q < MG; ++q)
+                                if (MG == 1 || q < G) add[q] += (unsigned long long)rintf(ck[q] * wf);
+                            lowd -= sseg;
+                            x = nx;
+                            y = ny;
+                            z = nz;
+                            const float v0 = lanef(u[0], (int)n);
+                            const bool scat = v0 * cext < csca;
+                            dx = scat && P.hg ? dx : lanef(ex, (int)n);
+                            dy = scat && P.hg ? dy : lanef(ey, (int)n);
+                            dz = scat && P.hg ? dz : lanef(ez, (int)n);
+                            if (scat) {
+                                ++nsc;
+                                if (P.hg) {
+                                    const float us = lanef(u[1], (int)n) * csca;
+                                    float a = 0.f;
+                                    int sp = S - 1;
+                                    for (int s = 0; s < S; ++s) {
+                                        a = fmaf(pickn<MS>(rho, s), s_ks[s * NL + f], a);
+                                        if (us <= a) {
+                                            sp = s;
+                                            break;
+                                        }
+                                    }
+                                    hg_dir(lanef(u[4], (int)n), lanef(u[5], (int)n),
+                                           s_g[sp * NL + f], dx, dy, dz);
+                                }
+                            } else {
+                                // the absorbing species' group: with two groups
+                                // there are at most two species here (MS <= 2)
+                                int q = 0;
+                                if (MG > 1) q = (S < 2 || lanef(u[1], (int)n) * cabs <= c0) ? grpr[0]
+                                                                                             : grpr[MS > 1 ? 1 : 0];
+                                q = (int)uniform32((unsigned)q);
+#pragma unroll
+                                for (int t = 0; t < MG; ++t)
+                                    if (q == t) {
+                                        f = __builtin_amdgcn_readlane(ec[t], (int)n);
+                                        cabs = lanef(eabs[t], (int)n);
+                                        csca = lanef(esca[t], (int)n);
+                                        c0 = lanef(e0[t], (int)n);
+#pragma unroll
+                                        for (int h = 0; h < MG; ++h) ck[h] = lanef(ek[t][h], (int)n);
+                                    }
+                            }
+                            tl = lanef(etau, (int)n);
+                        }
+                        if (lane == L) {
+                            p.x = x;
+                            p.y = y;
+                            p.z = z;
+                            p.dx = dx;
+                            p.dy = dy;
+                            p.dz = dz;
+                            tau = tl;
+                            ifr = f;
+                            aRc = aR;
+                            krng += n;
+                            nev += n;
+                            nev_cell += n;
+                            slice_left -= n;
+                            if (n) nzero = 0;
+#pragma unroll
+                            for (int q = 0; q < MG; ++q) acc[q] += add[q];
+                            crow[5] += n;
+                            crow[2] += nsc;
+                            crow[1] += n - nsc;
+                        }
+                    }
+                }
+            }
+        }
 
         // ---- batch: a wave left with a few live packets and nothing to hand out
         // in its run parks them in the run's pool and moves on to another run

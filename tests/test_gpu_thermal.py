@@ -199,3 +199,26 @@ def test_device_density_generator_matches_host_builders():
         assert np.array_equal(got > 0, want > 0), c
         rel = np.abs(got - want) / np.maximum(want, 1e-300)
         assert rel.max() <= 2e-7, (c, rel.max())
+
+
+@pytest.mark.parametrize("max_events,slice_events", [
+    (1, 10000), (4, 10000), (5, 10000), (12, 10000), (68, 10000), (69, 10000), (70, 10000),
+    (133, 10000), (1000, 10000), (1000, 9), (1000, 10), (1000, 64), (1000, 65), (1000, 73)])
+def test_walk_inside_a_thick_cell_counts_every_interaction(max_events, slice_events):
+    """Two packets in a cell of optical depth 1e9: neither can leave, so each
+    interacts exactly max_events times, wherever a walk of up to 64
+    interactions ends (the cap, a slice's last interaction), and every tally
+    add is counted once: the temperature equals that of a batch of the same
+    run, whose slots and waves are laid out differently, bit for bit."""
+    print("case: thick cell, max_events %d, slice %d" % (max_events, slice_events), flush=True)
+    arr = oracle_arrays(configs.disk_c1(nr=4, nt=2))
+    arr["rho"] = np.full(arr["rho"].shape, 1e-4)
+    dm = rt.DeviceModel(arr)
+    st = dm.thermal(2, 5, max_events=max_events, slice_events=slice_events)
+    assert st["n_killed"] == 2 and st["n_escape"] == 0
+    assert st["n_events"] == 2 * max_events == st["n_abs"] + st["n_scat"]
+    T = dm.temperature()
+    other = rt.DeviceModel(arr)
+    b = rt.Batch([other, dm])
+    b.thermal([2, 2], [5, 5], max_events=max_events, slice_events=slice_events)
+    assert np.array_equal(other.temperature(), T) and np.array_equal(dm.temperature(), T)
