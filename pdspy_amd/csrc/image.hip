@@ -11,11 +11,12 @@
 // zoomau produces (Model.py:522-527).
 //
 // Kernels: a per-cell prep pass (alpha and S per cell) so
-// the ray loop reads 8 bytes per crossed cell; one ray per lane; the adjoint
+// the ray loop reads 8 bytes per crossed cell; a ray's crossings split over
+// lanes; the adjoint
 // re-integrates each ray twice (first for I, then for dI/d dtau_k = e^-tau_k
 // e^-dtau_k S_k - (I - I_<=k)) instead of storing tau, and accumulates
-// dL/dalpha, dL/dS per cell with FP64 atomics; a post pass applies the chain
-// rule to log(rho_s) and T.
+// dL/dalpha, dL/dS per cell as 64-bit fixed-point integers; a post pass applies
+// the chain rule to log(rho_s) and T.
 #include <algorithm>
 #include <cmath>
 
@@ -25,12 +26,15 @@ using namespace rt;
 
 struct CamParams {
     DevGrid g;
-    float n[3], ex[3], ey[3];
-    float cpa, spa;
-    float pix;       // au
+    float n[3];               // towards the observer
+    double nd[3], ex[3], ey[3];
+    double cpa, spa;
+    double pix;      // au
+    float pixf;
     int nx, ny, nsub, mode;
-    int tw, th, ntx;  // ray tile of a block: tw x th pixels, ntx tiles per image row
-    unsigned hbits;   // adjoint LDS table: 2^hbits entries (>= 4 per ray of a block)
+    int tw, th, ntx, nty;  // ray tiles: tw x th pixels, ntx per image row, nty rows of them
+    unsigned hbits;   // adjoint LDS table: 2^hbits entries
+    int lanes;        // lanes per ray (a power of two)
     float tau_stop;
     const float *alpha;  // [cell] per au
     const float *src;    // [cell]
@@ -51,121 +55,343 @@ __device__ __forceinline__ void count_crossings(unsigned long long *dst, uint32_
 }
 
 // A camera ray is the line p0 + s d: p0 the point closest to the origin (in
-// the sky plane through it), d = -n.  Marching the FP32 position from the
-// outer sphere accumulates a transverse error of a few ulp of the outer radius
-// (~1e-3 au at 5000 au); on a nearly radial ray (the central pixels) the theta
-// crossings then move along the ray by that error times r/b, a sizeable part
-// of a cell.  At every radial crossing the position is therefore set back on
-// the exact line at s = -+sqrt(r_wall^2 - b^2) (FP64), which leaves only the
-// error gathered since the last radial crossing, a few ulp of the local radius.
-struct CamRay {
-    float x0, y0, z0;  // p0 (au)
-    double b2;         // |p0|^2
+// the sky plane through it), d = -n, s in [-S, S] inside the outer sphere.  All
+// its crossings are known in closed form, so it is not marched from wall to
+// wall:
+//  * spheres: s = -+sqrt(R_i^2 - b^2), inwards down to the innermost one that
+//    the ray meets, then outwards;
+//  * cones: with z reflected so that z0 >= 0, u = z / r = cos(theta) rises
+//    along the ray to u* = sqrt(z0^2 + dz^2 b^2) / b at s* = dz b^2 / z0 and
+//    falls from there, so the walls met are those from the entry's down to u*'s
+//    and back up to the exit's, wall c at s = (dz b^2 c -+ z0 Q) / (z0 c +- dz Q)
+//    with Q = sqrt(z0^2 + b^2 (dz^2 - c^2)) (upper signs before s*, lower ones
+//    after).  An equatorially mirrored grid is unfolded to 2 nt cells from pole
+//    to pole;
+//  * phi half-planes, in the order the ray turns about the axis.
+// Each sequence is sorted and numbered, the k-th sphere or cone crossing costs
+// one square root (and a quotient) whatever came before, in FP64, and the ray's
+// segments are the merged sequence.  No test has to decide whether a wall is hit,
+// so near-tangent rays need no care, and -- what it is done for -- a ray can be
+// entered anywhere: `lanes` lanes take equal shares of the merged sequence (found
+// by a binary search over the two sequences' counters) and combine their
+// (optical depth, intensity) afterwards.  An image of 256 x 256 rays is 1024
+// waves, one per SIMD, and a march of one ray per lane left it waiting on the
+// longest chains (~700 crossings of ~6000 clocks: 1.47 ms); with 8 lanes per ray
+// and ~150 instructions per crossing see k_image.
+struct RayGeo {
+    double b2, z0, dz, S;
+    int nin, w;    // spheres met inwards (as many outwards); the innermost one
+    int js, jt;    // theta cells of the entry and of u* (unfolded, flipped frame)
+    int nA, nT;    // cone crossings before s*, and in all
+    double x0, y0; // p0 in the equatorial plane (phi cells)
+    bool flip;     // z reflected
 };
 
-__device__ __forceinline__ bool ray_start(const CamParams &C, float X, float Y, Pos &p,
-                                          CamRay &cr) {
-    float xp = X * C.cpa + Y * C.spa;
-    float yp = -X * C.spa + Y * C.cpa;
-    cr.x0 = xp * C.ex[0] + yp * C.ey[0];
-    cr.y0 = xp * C.ex[1] + yp * C.ey[1];
-    cr.z0 = xp * C.ex[2] + yp * C.ey[2];
-    cr.b2 = (double)cr.x0 * cr.x0 + (double)cr.y0 * cr.y0 + (double)cr.z0 * cr.z0;
-    const double R = C.g.rwd[C.g.nr];
-    if (cr.b2 >= R * R) return false;
-    p.dx = -C.n[0];
-    p.dy = -C.n[1];
-    p.dz = -C.n[2];
-    const float s = (float)-sqrt(R * R - cr.b2);
-    p.x = fmaf(s, p.dx, cr.x0);
-    p.y = fmaf(s, p.dy, cr.y0);
-    p.z = fmaf(s, p.dz, cr.z0);
-    p.ir = C.g.nr - 1;
-    locate_angles(C.g, p);
+__device__ __forceinline__ double rcp_d(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// cells of the unfolded theta axis, its walls' cosines (descending) and the
+// grid's cell of an unfolded one
+__device__ __forceinline__ int ntheta_u(const DevGrid &g) { return g.mirror ? 2 * g.nt : g.nt; }
+__device__ __forceinline__ double cos_u(const DevGrid &g, bool flip, int j) {
+    if (g.mirror) return j <= g.nt ? g.ctd[j] : -g.ctd[2 * g.nt - j];
+    return flip ? -g.ctd[g.nt - j] : g.ctd[j];
+}
+__device__ __forceinline__ int fold_u(const DevGrid &g, bool flip, int j) {
+    if (g.mirror) return j < g.nt ? j : 2 * g.nt - 1 - j;
+    return flip ? g.nt - 1 - j : j;
+}
+// the unfolded cell j with cos(wall j) > u >= cos(wall j + 1)
+__device__ __forceinline__ int find_u(const DevGrid &g, bool flip, double u) {
+    int lo = 0, hi = ntheta_u(g);
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (cos_u(g, flip, mid) > u)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// the ray through sky position (X, Y) (au); false: it misses the grid
+__device__ __forceinline__ bool ray_setup(const CamParams &C, double X, double Y, RayGeo &q) {
+    const DevGrid &g = C.g;
+    const double R = g.rwd[g.nr];
+    double xp = X * C.cpa + Y * C.spa, yp = -X * C.spa + Y * C.cpa;
+    // a ray through the origin is moved off it by 1e-12 of the grid's radius
+    // (which direction it would turn to there is not defined)
+    if (xp * xp + yp * yp < 1e-24 * R * R) yp = 1e-12 * R;
+    q.x0 = xp * C.ex[0] + yp * C.ey[0];
+    q.y0 = xp * C.ex[1] + yp * C.ey[1];
+    q.z0 = xp * C.ex[2] + yp * C.ey[2];
+    q.dz = -C.nd[2];
+    q.b2 = fma(q.x0, q.x0, fma(q.y0, q.y0, q.z0 * q.z0));
+    if (!(q.b2 < R * R)) return false;
+    q.S = sqrt(R * R - q.b2);
+    q.flip = q.z0 < 0.0;
+    if (q.flip) {
+        q.z0 = -q.z0;
+        q.dz = -q.dz;
+    }
+    // innermost sphere met: the first with R_w > b
+    int lo = -1, hi = g.nr;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        const double r = g.rwd[mid];
+        if (r * r > q.b2)
+            hi = mid;
+        else
+            lo = mid;
+    }
+    q.w = hi;
+    q.nin = g.nr - hi;
+    // theta cells of the entry, the turning point and the exit
+    const double iR = rcp_d(R), b = sqrt(q.b2);
+    const double us = (q.z0 - q.S * q.dz) * iR, ue = (q.z0 + q.S * q.dz) * iR;
+    const double ut = sqrt(fma(q.z0, q.z0, q.dz * q.dz * q.b2)) * rcp_d(b);
+    const double st = q.dz * q.b2;  // s* z0
+    q.js = find_u(g, q.flip, us);
+    const int je = find_u(g, q.flip, ue);
+    // s* outside [-S, S]: u is monotonic there
+    q.jt = st <= -q.S * q.z0 ? q.js : (st >= q.S * q.z0 ? je : find_u(g, q.flip, ut));
+    q.jt = min(q.jt, min(q.js, je));
+    q.nA = q.js - q.jt;
+    q.nT = q.nA + je - q.jt;
     return true;
 }
 
-// cross_wall for a camera ray: radial crossings put the position on the exact
-// line (see CamRay); theta, phi and mirror crossings as cross_wall
-__device__ __forceinline__ bool cross_wall_cam(const DevGrid &g, Pos &p, float t, int kind,
-                                               const CamRay &cr) {
-    if (kind != W_RIN && kind != W_ROUT && kind != W_HOLE) return cross_wall(g, p, t, kind);
-    const bool out = kind != W_RIN;
-    const int ir = kind == W_HOLE ? 0 : p.ir + (out ? 1 : -1);
-    p.ir = ir;
-    if (ir >= g.nr) return true;
-    const double rw = g.rwd[out ? ir : ir + 1];
-    float s = (float)sqrt(fmax(rw * rw - cr.b2, 0.0));
-    if (!out) s = -s;
-    p.x = fmaf(s, p.dx, cr.x0);
-    p.y = fmaf(s, p.dy, cr.y0);
-    p.z = fmaf(s, p.dz, cr.z0);
-    if (kind == W_HOLE) locate_angles(g, p);
-    return false;
+// position of the k-th sphere crossing (k = 2 nin: the outer sphere)
+__device__ __forceinline__ double sph_at(const CamParams &C, const RayGeo &q, int k) {
+    const bool inw = k < q.nin;
+    const double r = C.g.rwd[inw ? C.g.nr - 1 - k : q.w + k - q.nin];
+    const double s = sqrt(fmax(fma(r, r, -q.b2), 0.0));
+    return inw ? -s : s;
 }
 
-// formal solution along the ray from p; with LMIN also the smallest cell size
-// on the part of the ray traced (RT_INF when it crosses no cell)
-template <bool LMIN>
-__device__ __forceinline__ float integrate_ray_l(const CamParams &C, Pos p, const CamRay &cr,
-                                                 float &lmin, uint32_t &nseg) {
-    float I = 0.f, tau = 0.f;
-    uint32_t nzero = 0;
-    for (int guard = 0; guard < (1 << 24); ++guard) {
-        int kind;
-        float tw = next_wall<1>(C.g, p, kind);
-        const float rcell = C.g.rw[p.ir + 1];
-        if (p.ir >= 0) {
-            ++nseg;
-            int c = cell_index(C.g, p);
-            if (LMIN) lmin = fminf(lmin, C.csize[c]);
-            float dtau = C.alpha[c] * tw;
-            if (C.mode == 0) {
-                I = fmaf(__expf(-tau) * (-expm1f(-dtau)), C.src[c], I);
-                tau += dtau;
-                if (tau > C.tau_stop) break;
-            } else {
-                tau += dtau;
+// position of the k-th cone crossing (none left: beyond every sphere)
+__device__ __forceinline__ double cone_at(const CamParams &C, const RayGeo &q, int k) {
+    if (k >= q.nT) return 1e300;
+    const bool A = k < q.nA;
+    const double c = cos_u(C.g, q.flip, A ? q.js - k : q.jt + 1 + k - q.nA);
+    const double Q = sqrt(fmax(fma(q.b2, fma(q.dz, q.dz, -c * c), q.z0 * q.z0), 0.0));
+    const double sQ = A ? -Q : Q;
+    const double s = fma(q.dz * q.b2, c, q.z0 * sQ) * rcp_d(fma(q.z0, c, -q.dz * sQ));
+    return s > -q.S ? (s < q.S ? s : q.S) : -q.S;   // (NaN: -S)
+}
+
+// position where the ray, turning in direction `up` about the axis, leaves phi
+// cell ip; 1e300 if it never does
+__device__ __forceinline__ double phi_at(const CamParams &C, const RayGeo &q, int ip, bool up, double s) {
+    const int k = up ? ip + 1 : ip;
+    const double cp = C.g.cp[k], sp = C.g.sp[k];
+    const double dx = -C.nd[0], dy = -C.nd[1];
+    const double den = dy * cp - dx * sp;
+    if (up ? !(den > 0.0) : !(den < 0.0)) return 1e300;
+    const double t = (q.x0 * sp - q.y0 * cp) * rcp_d(den);
+    // in a cell of more than half a turn the wall ahead may be one that the
+    // line has passed behind the position
+    if (t < s - 1e-12 * fabs(s) && C.g.pw[ip + 1] - C.g.pw[ip] > 3.2f) return 1e300;
+    return fmax(t, s);
+}
+
+// Lane `l` of `L` walks its share of the ray's segments: f(cell, length) for each
+// of them that lies in a cell, until f returns true.
+template <class F>
+__device__ __forceinline__ void walk_ray(const CamParams &C, const RayGeo &q, int l, int L, F f) {
+    const DevGrid &g = C.g;
+    const int NR = 2 * q.nin + 1, M = NR + q.nT;
+    const int m0 = (int)(((long long)M * l) / L), m1 = (int)(((long long)M * (l + 1)) / L);
+    if (m0 >= m1) return;
+    // the first m0 crossings: kr spheres and kt cones (a sphere first on a tie)
+    int lo = max(0, m0 - q.nT), hi = min(m0, NR);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sph_at(C, q, mid) <= cone_at(C, q, m0 - 1 - mid))
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    int kr = lo, kt = m0 - lo;
+    if (kr >= NR) return;  // cones beyond the outer sphere by rounding
+    double s = -q.S;
+    if (kr > 0) s = fmax(s, sph_at(C, q, kr - 1));
+    if (kt > 0) s = fmax(s, cone_at(C, q, kt - 1));
+    double sr = sph_at(C, q, kr), st = cone_at(C, q, kt);
+    int ir = kr <= q.nin ? g.nr - 1 - kr : q.w - 1 + kr - q.nin;
+    int it = fold_u(g, q.flip, kt <= q.nA ? q.js - kt : q.jt + kt - q.nA);
+    int ip = 0;
+    double sp = 1e300;
+    int nphi = g.np;  // a ray turns by less than a whole turn: each wall once at most
+    bool up = true;
+    if (g.np > 1) {
+        up = q.x0 * -C.nd[1] - q.y0 * -C.nd[0] >= 0.0;
+        float ph = atan2f((float)(q.y0 - s * C.nd[1]), (float)(q.x0 - s * C.nd[0]));
+        if (ph < 0.f) ph += 6.28318530718f;
+        ip = search_walls(g.pw, g.np, ph);
+        sp = phi_at(C, q, ip, up, s);
+    }
+    for (int n = m1 - m0; n > 0;) {
+        double sn = fmin(sr, st);
+        const bool phi = sp < sn;
+        sn = fmax(phi ? sp : sn, s);
+        if (ir >= 0)
+            if (f(ir + g.nr * (it + g.nt * ip), (float)(sn - s))) return;
+        s = sn;
+        if (phi) {
+            ip = up ? (ip + 1 < g.np ? ip + 1 : 0) : (ip > 0 ? ip - 1 : g.np - 1);
+            sp = --nphi > 0 ? phi_at(C, q, ip, up, s) : 1e300;
+            continue;
+        }
+        --n;
+        if (sr <= st) {
+            ++kr;
+            if (kr >= NR) return;
+            ir = kr <= q.nin ? g.nr - 1 - kr : q.w - 1 + kr - q.nin;
+            sr = sph_at(C, q, kr);
+        } else {
+            ++kt;
+            it = fold_u(g, q.flip, kt <= q.nA ? q.js - kt : q.jt + kt - q.nA);
+            st = cone_at(C, q, kt);
+        }
+    }
+}
+
+// what a lane's share of a ray adds up to
+template <class A>
+struct RaySum {
+    A I;          // its own emission, attenuated from its own front on
+    float tau;    // its own optical depth
+    float tau0;   // optical depth in front of it
+    A front;      // attenuation in front of it (0: the ray has ended there, tau_stop)
+    float lmin;   // smallest cell size on the part traced (LMIN)
+};
+
+// 1 - e^-dtau and e^-dtau as two numbers that sum to 1
+__device__ __forceinline__ void absorb(float dtau, double &om, double &e) {
+    const bool thin = dtau < 0.5f;
+    const double x = thin ? (double)-expm1f(-dtau) : (double)__expf(-dtau);
+    om = thin ? x : 1.0 - x;
+    e = thin ? 1.0 - x : x;
+}
+
+// The formal solution along the ray by L neighbouring lanes; every lane gets the
+// ray's value (the intensity, or tau).  A ray ends once its optical depth
+// exceeds tau_stop: the share it ends in is walked again with the optical depth
+// in front of it, the shares behind it count for nothing.  A: type the intensity
+// is summed in; in double (the adjoint) the attenuation is the running product
+// of the segments' e^-dtau, so that emission and attenuation of a segment add up
+// to what comes in, whatever their rounding.
+template <bool LMIN, class A>
+__device__ __forceinline__ A trace_ray(const CamParams &C, const RayGeo &q, bool act, int l, int L,
+                                       RaySum<A> &r, uint32_t &nseg) {
+    r.I = 0;
+    r.tau = r.tau0 = 0.f;
+    r.front = 1;
+    r.lmin = RT_INF;
+    uint32_t ns = 0;
+    A att = 1;
+    const bool inten = C.mode == 0;
+    auto share = [&](float tau0) {
+        float tau = 0.f, lm = RT_INF;
+        A I = 0;
+        att = 1;
+        ns = 0;
+        walk_ray(C, q, l, L, [&](int c, float ds) {
+            ++ns;
+            if (LMIN) lm = fminf(lm, C.csize[c]);
+            const float dtau = C.alpha[c] * ds;
+            if (inten) {
+                if (sizeof(A) == 8) {
+                    double om, e;
+                    absorb(dtau, om, e);
+                    I = fma((A)(att * om), (A)C.src[c], I);
+                    att *= (A)e;
+                } else {
+                    I = fma((A)(__expf(-tau) * (-expm1f(-dtau))), (A)C.src[c], I);
+                }
+            }
+            tau += dtau;
+            return inten && tau0 + tau > C.tau_stop;
+        });
+        r.I = I;
+        r.tau = tau;
+        r.lmin = lm;
+    };
+    if (act) share(0.f);
+    if (L > 1) {
+        float t = r.tau;
+        A f = att;
+        for (int o = 1; o < L; o <<= 1) {
+            const float v = __shfl_up(t, o, L);
+            const A w = __shfl_up(f, o, L);
+            if (l >= o) {
+                t += v;
+                f *= w;
             }
         }
-        if (cross_wall_cam(C.g, p, tw, kind, cr)) break;
-        if (unstick(C.g, p, tw, rcell, nzero) && p.ir >= C.g.nr) break;
+        t = __shfl_up(t, 1, L);
+        f = __shfl_up(f, 1, L);
+        r.tau0 = l > 0 ? t : 0.f;
+        if (inten) {
+            const bool past = r.tau0 > C.tau_stop;
+            if (act && !past && l > 0 && r.tau0 + r.tau > C.tau_stop) share(r.tau0);
+            r.front = past ? (A)0 : sizeof(A) == 8 ? (l > 0 ? f : (A)1) : (A)__expf(-r.tau0);
+            if (past) {
+                r.lmin = RT_INF;
+                ns = 0;
+            }
+        }
+        A x = inten ? r.I * r.front : (A)r.tau;
+        for (int o = 1; o < L; o <<= 1) x += __shfl_xor(x, o, L);
+        if (LMIN)
+            for (int o = 1; o < L; o <<= 1) r.lmin = fminf(r.lmin, __shfl_xor(r.lmin, o, L));
+        nseg += ns;
+        return x;
     }
-    return C.mode == 0 ? I : tau;
+    nseg += ns;
+    return inten ? r.I : (A)r.tau;
 }
 
-__device__ __forceinline__ float integrate_ray(const CamParams &C, Pos p, const CamRay &cr,
-                                              uint32_t &nseg) {
-    float unused = RT_INF;
-    return integrate_ray_l<false>(C, p, cr, unused, nseg);
-}
-
-// pixel of this lane: blocks cover tw x th tiles of the image, so the rays of
-// a wavefront stay close together (they cross the same cells)
-__device__ __forceinline__ bool tile_pixel(const CamParams &C, int &j, int &k) {
-    const int tile = blockIdx.x, ty = tile / C.ntx, tx = tile - ty * C.ntx;
-    const int t = threadIdx.x, dy = t / C.tw, dx = t - dy * C.tw;
+// pixel of the n-th ray group: the image's tiles in order, the tile's pixels
+__device__ __forceinline__ bool tile_pixel(const CamParams &C, unsigned n, int &j, int &k) {
+    const unsigned tp = (unsigned)(C.tw * C.th), tile = n / tp, t = n - tile * tp;
+    const int ty = (int)tile / C.ntx, tx = (int)tile - ty * C.ntx;
+    const int dy = (int)t / C.tw, dx = (int)t - dy * C.tw;
     k = tx * C.tw + dx;
     j = ty * C.th + dy;
     return k < C.nx && j < C.ny;
 }
 
-__global__ void __launch_bounds__(256) k_image(CamParams C, float *img) {
+__device__ __forceinline__ double sky_x(const CamParams &C, int k, int b) {
+    return ((double)(k - C.nx / 2) + ((b + 0.5) / C.nsub - 0.5)) * C.pix;
+}
+__device__ __forceinline__ double sky_y(const CamParams &C, int j, int a) {
+    return ((double)(j - C.ny / 2) + ((a + 0.5) / C.nsub - 0.5)) * C.pix;
+}
+
+#define IMG_BS 256
+#define IMG_LANES 524288u  // lanes a launch is spread over, if the rays allow
+#define IMG_MAXL 32         // at most this many of them per ray
+
+__global__ void __launch_bounds__(IMG_BS) k_image(CamParams C, float *img) {
     int j, k;
     uint32_t nseg = 0;
-    if (tile_pixel(C, j, k)) {
-        const int pix = j * C.nx + k;
-        float acc = 0.f;
-        for (int a = 0; a < C.nsub; ++a)
-            for (int b = 0; b < C.nsub; ++b) {
-                float X = ((float)(k - C.nx / 2) + ((b + 0.5f) / C.nsub - 0.5f)) * C.pix;
-                float Y = ((float)(j - C.ny / 2) + ((a + 0.5f) / C.nsub - 0.5f)) * C.pix;
-                Pos p;
-                CamRay cr;
-                if (ray_start(C, X, Y, p, cr)) acc += integrate_ray(C, p, cr, nseg);
-            }
-        img[pix] = acc / (float)(C.nsub * C.nsub);
-    }
+    const int L = C.lanes, l = (int)(threadIdx.x & (unsigned)(L - 1));
+    const unsigned n = (blockIdx.x * IMG_BS + threadIdx.x) / (unsigned)L;
+    const bool in = tile_pixel(C, n, j, k);
+    float acc = 0.f;
+    for (int a = 0; a < C.nsub; ++a)
+        for (int b = 0; b < C.nsub; ++b) {
+            RayGeo q;
+            RaySum<float> r;
+            const bool act = in && ray_setup(C, sky_x(C, k, b), sky_y(C, j, a), q);
+            acc += trace_ray<false>(C, q, act, l, L, r, nseg);
+        }
+    if (in && l == 0) img[j * C.nx + k] = acc / (float)(C.nsub * C.nsub);
     count_crossings(C.icount, nseg);
 }
 
@@ -218,47 +444,53 @@ __device__ __forceinline__ void adj_flush(const int *key, const u64 *ga, const u
 }
 
 // gI times the gradient of the ray through sky (X, Y) w.r.t. the per-cell
-// alpha and S: the ray is integrated for I, then swept again front to back
-// recomputing tau, with R_k = I - I_<=k (nothing is stored per segment)
-__device__ __forceinline__ void adjoint_ray(const CamParams &C, float X, float Y, float gI,
-                                            int *key, u64 *ga, u64 *gs, double *g_alpha,
+// alpha and S, by L neighbouring lanes: the ray is integrated for I, then each
+// lane sweeps its share again front to back recomputing tau (nothing is stored
+// per segment).  What lies behind segment k, R_k = I - I_<=k, is what the same
+// sums leave of the lane's own share (the sweep repeats the integration's
+// operations, in FP64, so no rounding is left over where R_k is small) plus the
+// shares behind it.
+__device__ __forceinline__ void adjoint_ray(const CamParams &C, double X, double Y, float gI, int l,
+                                            int L, int *key, u64 *ga, u64 *gs, double *g_alpha,
                                             double *g_src, uint32_t &nseg) {
-    Pos p0;
-    CamRay cr;
-    if (!ray_start(C, X, Y, p0, cr)) return;
-    const double qa = C.qs[0], qsrc = C.qs[1];
+    RayGeo q;
+    RaySum<double> r;
+    const bool act = gI != 0.f && ray_setup(C, X, Y, q);
     uint32_t nfwd = 0;
-    float I = integrate_ray(C, p0, cr, nfwd);
-    Pos p = p0;
-    float tau = 0.f, cum = 0.f;
-    uint32_t nzero = 0;
-    for (int guard = 0; guard < (1 << 24); ++guard) {
-        int kind;
-        float tw = next_wall<1>(C.g, p, kind);
-        const float rcell = C.g.rw[p.ir + 1];
-        if (p.ir >= 0) {
-            ++nseg;
-            int c = cell_index(C.g, p);
-            float dtau = C.alpha[c] * tw;
-            float att = __expf(-tau);
-            float om = -expm1f(-dtau);
-            float S = C.src[c];
-            cum = fmaf(att * om, S, cum);
-            float Rk = I - cum;
-            float dI_ddtau = att * (1.f - om) * S - Rk;
-            adj_add(c, __double2ll_rn((double)(gI * dI_ddtau * tw) * qa),
-                    __double2ll_rn((double)(gI * att * om) * qsrc), key, ga, gs, C.hbits,
-                    g_alpha, g_src);
-            tau += dtau;
-            if (tau > C.tau_stop) break;
+    (void)trace_ray<false>(C, q, act, l, L, r, nfwd);
+    double behind = r.I * r.front;
+    if (L > 1) {
+        double x = behind;
+        for (int o = 1; o < L; o <<= 1) {
+            const double v = __shfl_down(x, o, L);
+            if (l + o < L) x += v;
         }
-        if (cross_wall_cam(C.g, p, tw, kind, cr)) break;
-        if (unstick(C.g, p, tw, rcell, nzero) && p.ir >= C.g.nr) break;
+        behind = __shfl_down(x, 1, L);
     }
+    if (l == L - 1) behind = 0.0;
+    if (!act || r.front == 0.0) return;
+    const double qa = C.qs[0] * (double)gI, qsrc = C.qs[1] * (double)gI;
+    float tau = 0.f;
+    double cum = 0.0, att = 1.0;
+    walk_ray(C, q, l, L, [&](int c, float ds) {
+        ++nseg;
+        const float dtau = C.alpha[c] * ds;
+        const double S = C.src[c];
+        double om, e;
+        absorb(dtau, om, e);
+        const double em = att * om;
+        cum = fma(em, S, cum);
+        att *= e;
+        const double dI_ddtau = r.front * fma(att, S, cum - r.I) - behind;
+        adj_add(c, __double2ll_rn(dI_ddtau * (double)ds * qa),
+                __double2ll_rn(r.front * em * qsrc), key, ga, gs, C.hbits, g_alpha, g_src);
+        tau += dtau;
+        return r.tau0 + tau > C.tau_stop;
+    });
 }
 
-__global__ void __launch_bounds__(256) k_image_adj(CamParams C, const float *dimg, double *g_alpha,
-                                                   double *g_src) {
+__global__ void __launch_bounds__(IMG_BS) k_image_adj(CamParams C, const float *dimg, double *g_alpha,
+                                                      double *g_src) {
     extern __shared__ u64 adj_lds[];
     const unsigned H = 1u << C.hbits;
     u64 *ga = adj_lds, *gs = adj_lds + H;
@@ -270,19 +502,14 @@ __global__ void __launch_bounds__(256) k_image_adj(CamParams C, const float *dim
     }
     __syncthreads();
     int j, k;
-    bool act = tile_pixel(C, j, k);
-    float gI = 0.f;
-    if (act) {
-        gI = dimg[j * C.nx + k] / (float)(C.nsub * C.nsub);
-        act = gI != 0.f;
-    }
+    const int L = C.lanes, l = (int)(threadIdx.x & (unsigned)(L - 1));
+    const bool in = tile_pixel(C, (blockIdx.x * IMG_BS + threadIdx.x) / (unsigned)L, j, k);
+    const float gI = in ? dimg[j * C.nx + k] / (float)(C.nsub * C.nsub) : 0.f;
     uint32_t nseg = 0;
-    for (int a = 0; act && a < C.nsub; ++a)
-        for (int b = 0; b < C.nsub; ++b) {
-            float X = ((float)(k - C.nx / 2) + ((b + 0.5f) / C.nsub - 0.5f)) * C.pix;
-            float Y = ((float)(j - C.ny / 2) + ((a + 0.5f) / C.nsub - 0.5f)) * C.pix;
-            adjoint_ray(C, X, Y, gI, key, ga, gs, g_alpha, g_src, nseg);
-        }
+    for (int a = 0; a < C.nsub; ++a)
+        for (int b = 0; b < C.nsub; ++b)
+            adjoint_ray(C, in ? sky_x(C, k, b) : 0.0, in ? sky_y(C, j, a) : 0.0, gI, l, L, key, ga,
+                        gs, g_alpha, g_src, nseg);
     __syncthreads();
     adj_flush(key, ga, gs, H, g_alpha, g_src);
     count_crossings(C.icount ? C.icount + 1 : nullptr, nseg);
@@ -350,10 +577,19 @@ __global__ void k_ref_init(CamParams C, RefArgs R) {
     int j, k, a, b;
     float2 xy = make_float2(RT_REF_DEAD, RT_REF_DEAD);  // tile padding: no ray
     if (node0_pixel(C, R.ns2, i, j, k, a, b)) {
-        xy.x = ((float)(k - C.nx / 2) + ((b + 0.5f) / C.nsub - 0.5f)) * C.pix;
-        xy.y = ((float)(j - C.ny / 2) + ((a + 0.5f) / C.nsub - 0.5f)) * C.pix;
+        xy.x = (float)sky_x(C, k, b);
+        xy.y = (float)sky_y(C, j, a);
     }
     R.xy[i] = xy;
+}
+
+// lanes per ray for n rays: about four waves per SIMD, and no more than a ray's
+// crossings are worth (n depends on the image alone, so the sums do not change
+// with the launch)
+__device__ __host__ __forceinline__ int ref_lanes(unsigned n) {
+    int L = 1;
+    while (L < IMG_MAXL && (size_t)n * (size_t)(2 * L) <= IMG_LANES) L *= 2;
+    return L;
 }
 
 // traces level L: value of every node, children for those that split
@@ -364,23 +600,21 @@ __global__ void __launch_bounds__(256) k_ref_trace(CamParams C, RefArgs R, int L
     const int lane = __lane_id();
     unsigned nrays = 0;
     uint32_t nseg = 0;
-    for (unsigned base = start + blockIdx.x * blockDim.x; base < end;
-         base += gridDim.x * blockDim.x) {
-        const unsigned i = base + threadIdx.x;
+    const int LN = ref_lanes(end > start ? end - start : 0u), l = (int)(threadIdx.x & (unsigned)(LN - 1));
+    const unsigned per = blockDim.x / (unsigned)LN;  // nodes of a block
+    for (unsigned base = start + blockIdx.x * per; base < end; base += gridDim.x * per) {
+        const unsigned i = base + threadIdx.x / (unsigned)LN;
         const bool act = i < end;
-        float I = 0.f, lmin = RT_INF;
         float2 xy = make_float2(RT_REF_DEAD, RT_REF_DEAD);
-        if (act) {
-            xy = R.xy[i];
-            Pos p;
-            CamRay cr;
-            if (xy.x < 0.5f * RT_REF_DEAD && ray_start(C, xy.x, xy.y, p, cr)) {
-                I = integrate_ray_l<true>(C, p, cr, lmin, nseg);
-                ++nrays;
-            }
-            R.val[i] = I;
-        }
-        const bool want = act && may_split && d > R.crit * lmin;
+        if (act) xy = R.xy[i];
+        RayGeo q;
+        RaySum<float> r;
+        const bool ray = act && xy.x < 0.5f * RT_REF_DEAD && ray_setup(C, xy.x, xy.y, q);
+        const float I = trace_ray<true>(C, q, ray, l, LN, r, nseg);
+        const bool first = act && l == 0;
+        if (first) R.val[i] = I;
+        if (first && ray) ++nrays;
+        const bool want = first && may_split && d > R.crit * r.lmin;
         const uint64_t mk = __ballot(want);
         int ch = -1;
         if (mk) {
@@ -415,7 +649,7 @@ __global__ void __launch_bounds__(256) k_ref_trace(CamParams C, RefArgs R, int L
                 }
             }
         }
-        if (act) R.child[i] = ch;
+        if (first) R.child[i] = ch;
     }
     for (int off = 32; off > 0; off >>= 1) nrays += __shfl_down(nrays, off);
     if (lane == 0 && nrays) atomicAdd(&R.ctl[RT_REF_RAYS], nrays);
@@ -470,7 +704,7 @@ __global__ void __launch_bounds__(256) k_ref_down(RefArgs R, int L) {
     }
 }
 
-// the leaves' reverse sweeps; each block gathers a chunk of 256 leaves' cell
+// the leaves' reverse sweeps; each block gathers a chunk of leaves' cell
 // gradients in its LDS table before the global atomics, as k_image_adj does
 __global__ void __launch_bounds__(256) k_ref_adj(CamParams C, RefArgs R, double *g_alpha,
                                                  double *g_src) {
@@ -480,20 +714,23 @@ __global__ void __launch_bounds__(256) k_ref_adj(CamParams C, RefArgs R, double 
     int *key = (int *)(adj_lds + 2 * H);
     const unsigned n = R.ctl[0] < R.cap ? R.ctl[0] : R.cap;
     uint32_t nseg = 0;
-    for (unsigned base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+    const int LN = ref_lanes(n), l = (int)(threadIdx.x & (unsigned)(LN - 1));
+    const unsigned per = blockDim.x / (unsigned)LN;
+    for (unsigned base = blockIdx.x * per; base < n; base += gridDim.x * per) {
         for (unsigned t = threadIdx.x; t < H; t += blockDim.x) {
             key[t] = -1;
             ga[t] = 0ull;
             gs[t] = 0ull;
         }
         __syncthreads();
-        const unsigned i = base + threadIdx.x;
+        const unsigned i = base + threadIdx.x / (unsigned)LN;
+        float g = 0.f;
+        float2 xy = make_float2(0.f, 0.f);
         if (i < n && R.child[i] < 0) {
-            const float g = R.gw[i];
-            const float2 xy = R.xy[i];
-            if (g != 0.f && xy.x < 0.5f * RT_REF_DEAD)
-                adjoint_ray(C, xy.x, xy.y, g, key, ga, gs, g_alpha, g_src, nseg);
+            xy = R.xy[i];
+            g = xy.x < 0.5f * RT_REF_DEAD ? R.gw[i] : 0.f;
         }
+        adjoint_ray(C, xy.x, xy.y, g, l, LN, key, ga, gs, g_alpha, g_src, nseg);
         __syncthreads();
         adj_flush(key, ga, gs, H, g_alpha, g_src);
         __syncthreads();
@@ -519,12 +756,15 @@ __global__ void k_stars(CamParams C, int nstar, const float *spos, StarArg sflux
     if (s >= nstar) return;
     const int lane = threadIdx.x;
     float qx = spos[3 * s], qy = spos[3 * s + 1], qz = spos[3 * s + 2];
-    float xp = qx * C.ex[0] + qy * C.ex[1] + qz * C.ex[2];
-    float yp = qx * C.ey[0] + qy * C.ey[1] + qz * C.ey[2];
-    float X = xp * C.cpa - yp * C.spa;
-    float Y = xp * C.spa + yp * C.cpa;
-    int k = (int)floorf(X / C.pix + 0.5f) + C.nx / 2;
-    int j = (int)floorf(Y / C.pix + 0.5f) + C.ny / 2;
+    const float exx = (float)C.ex[0], exy = (float)C.ex[1], exz = (float)C.ex[2];
+    const float eyx = (float)C.ey[0], eyy = (float)C.ey[1], eyz = (float)C.ey[2];
+    const float cpa = (float)C.cpa, spa = (float)C.spa;
+    float xp = qx * exx + qy * exy + qz * exz;
+    float yp = qx * eyx + qy * eyy + qz * eyz;
+    float X = xp * cpa - yp * spa;
+    float Y = xp * spa + yp * cpa;
+    int k = (int)floorf(X / C.pixf + 0.5f) + C.nx / 2;
+    int j = (int)floorf(Y / C.pixf + 0.5f) + C.ny / 2;
     if (k < 0 || k >= C.nx || j < 0 || j >= C.ny) return;
     const DevGrid &g = C.g;
     if (qx == 0.f && qy == 0.f && qz == 0.f) {
@@ -812,26 +1052,29 @@ static int setup_camera(rt_model *m, const rt_camera *cam, CamParams &C, KapArg 
     C.icount = ctx->d_icount;
     for (int a = 0; a < 3; ++a) {
         C.n[a] = (float)n[a];
-        C.ex[a] = (float)ex[a];
-        C.ey[a] = (float)ey[a];
+        C.nd[a] = n[a];
+        C.ex[a] = ex[a];
+        C.ey[a] = ey[a];
     }
-    C.cpa = (float)std::cos(pa);
-    C.spa = (float)std::sin(pa);
-    C.pix = (float)(cam->pix_cm / RT_LEN_UNIT);
+    C.cpa = std::cos(pa);
+    C.spa = std::sin(pa);
+    C.pix = cam->pix_cm / RT_LEN_UNIT;
+    C.pixf = (float)C.pix;
     C.nx = cam->nx;
     C.ny = cam->ny;
     C.nsub = cam->nsub > 0 ? cam->nsub : 1;
     C.mode = cam->mode;
-    // ray tile: tile_w x tile_h pixels per block (default 64 x 1: one row run)
-    C.tw = cam->tile_w > 0 ? cam->tile_w : 64;
+    // ray tile: neighbouring rays run in tile_w x tile_h pixels (default 8 x 8)
+    C.tw = cam->tile_w > 0 ? cam->tile_w : 8;
     C.th = cam->tile_h > 0 ? cam->tile_h : 64 / C.tw;
     if (C.th < 1) C.th = 1;
     if (C.tw * C.th > 256 || (C.tw * C.th) % 64)
         return set_err(ctx, RT_E_ARG, "ray tile %d x %d: need a multiple of 64 pixels, at most 256",
                        C.tw, C.th);
     C.ntx = (C.nx + C.tw - 1) / C.tw;
-    C.hbits = 8;
-    while ((1u << C.hbits) < 4u * (unsigned)(C.tw * C.th)) ++C.hbits;
+    C.nty = (C.ny + C.th - 1) / C.th;
+    C.hbits = 11;
+    C.lanes = ref_lanes((unsigned)std::min<size_t>((size_t)C.nx * C.ny, 1u << 30));
     C.tau_stop = (float)(cam->tau_stop > 0 ? cam->tau_stop : 40.0);
     for (int s = 0; s < RT_MAX_SPEC; ++s) {
         kap.k[s] = s < m->nspec ? (float)kappa_at(m, m->kabs, s, cam->lam_um) : 0.f;
@@ -865,7 +1108,7 @@ static int refine_run(rt_model *m, const rt_camera *cam, CamParams C, float *d_i
     hipStream_t sm = ctx->stream;
     const int nref = std::min(cam->nrefine, RT_MAX_REFINE);
     const int ns2 = C.nsub * C.nsub;
-    const unsigned ntiles = (unsigned)(C.ntx * ((C.ny + C.th - 1) / C.th));
+    const unsigned ntiles = (unsigned)(C.ntx * C.nty);
     const size_t n0 = (size_t)ntiles * (size_t)(C.tw * C.th) * (size_t)ns2;
     const bool capturing = stream_capturing(sm);
     // a fresh pool starts at 2^21 nodes (40 MB); a reserved one is used as
@@ -884,7 +1127,7 @@ static int refine_run(rt_model *m, const rt_camera *cam, CamParams C, float *d_i
         if (rc) return rc;
         RefinePool &P = ctx->ref;
         RefArgs R{P.xy, P.val, P.child, P.gw, P.ctl, (unsigned)P.cap,
-                  (float)(cam->refine_crit > 0 ? cam->refine_crit : 1.0), nref, C.pix / C.nsub,
+                  (float)(cam->refine_crit > 0 ? cam->refine_crit : 1.0), nref, C.pixf / C.nsub,
                   (unsigned)n0, ns2};
         hipLaunchKernelGGL(k_ref_init, dim3(nblk(n0, 256)), dim3(256), 0, sm, C, R);
         for (int L = 0; L <= nref; ++L) {
@@ -912,8 +1155,7 @@ static int refine_run(rt_model *m, const rt_camera *cam, CamParams C, float *d_i
             hipLaunchKernelGGL(k_ref_gw0, dim3(nblk(n0, 256)), dim3(256), 0, sm, C, R, d_dimg);
             for (int L = 0; L < nref; ++L)
                 hipLaunchKernelGGL(k_ref_down, dim3(gblk), dim3(256), 0, sm, R, L);
-            CamParams Ca = C;
-            Ca.hbits = 10;  // >= 4 entries per ray of a 256-ray chunk
+            const CamParams &Ca = C;
             const size_t lds = (size_t)(1u << Ca.hbits) * (2 * sizeof(u64) + sizeof(int));
             hipLaunchKernelGGL(k_ref_adj, dim3(gblk), dim3(256), lds, sm, Ca, R, m->d_galpha,
                                m->d_gsrc);
@@ -921,6 +1163,11 @@ static int refine_run(rt_model *m, const rt_camera *cam, CamParams C, float *d_i
         HIPCHK(ctx, hipGetLastError());
         return RT_OK;
     }
+}
+
+// blocks of k_image / k_image_adj: every pixel of every tile, C.lanes lanes each
+static unsigned image_blocks(const CamParams &C) {
+    return nblk((size_t)C.ntx * C.nty * (size_t)(C.tw * C.th) * (size_t)C.lanes, IMG_BS);
 }
 
 static void star_fluxes(const rt_model *m, const rt_camera *cam, StarArg &fl) {
@@ -947,12 +1194,11 @@ int image_run(rt_model *m, const rt_camera *cam, const float *d_T, const float *
     hipLaunchKernelGGL(k_cam_prep, dim3(nblk(m->ncell, 256)), dim3(256), 0, sm, rho, m->nspec,
                        m->ncell, kap, (float)RT_LEN_UNIT, d_T, pre, hnu_k, cam->mode,
                        cam->d_jscat, m->d_alpha, m->d_src);
-    const unsigned ntiles = (unsigned)(C.ntx * ((C.ny + C.th - 1) / C.th));
     if (cam->nrefine > 0) {
         rc = refine_run(m, cam, C, d_img, nullptr);
         if (rc) return rc;
     } else {
-        hipLaunchKernelGGL(k_image, dim3(ntiles), dim3(C.tw * C.th), 0, sm, C, d_img);
+        hipLaunchKernelGGL(k_image, dim3(image_blocks(C)), dim3(IMG_BS), 0, sm, C, d_img);
     }
     if (cam->incl_star && cam->mode == 0 && m->nstar > 0) {
         StarArg fl;
@@ -991,13 +1237,12 @@ int image_adjoint_run(rt_model *m, const rt_camera *cam, const float *d_T, const
                        m->ncell, fmax_star, stars ? m->nstar : 0,
                        (float)(m->rw[m->nr] / RT_LEN_UNIT), m->d_qscale);
     C.qs = m->d_qscale;
-    const unsigned ntiles = (unsigned)(C.ntx * ((C.ny + C.th - 1) / C.th));
     if (cam->nrefine > 0) {
         rc = refine_run(m, cam, C, nullptr, d_dimg);
         if (rc) return rc;
     } else {
         const size_t adj_lds = (size_t)(1u << C.hbits) * (2 * sizeof(u64) + sizeof(int));
-        hipLaunchKernelGGL(k_image_adj, dim3(ntiles), dim3(C.tw * C.th), adj_lds, sm, C, d_dimg,
+        hipLaunchKernelGGL(k_image_adj, dim3(image_blocks(C)), dim3(IMG_BS), adj_lds, sm, C, d_dimg,
                            m->d_galpha, m->d_gsrc);
     }
     if (stars)
