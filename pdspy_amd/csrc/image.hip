@@ -93,16 +93,44 @@ __device__ __forceinline__ double rcp_d(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 
+// square root to a few ulp (positive arguments far from the ends of the range;
+// anything below counts as 1e-280), without the library's scaling
+__device__ __forceinline__ double sqrt_d(double x) {
+    x = fmax(x, 1e-280);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    return fma(fma(-g, g, x), h, g);
+}
+
+// 1 - e^-x for x >= 0: its series up to x^8 / 8! below 0.5 (the rest is below
+// 1e-8 of it), the difference above
+__device__ __forceinline__ float one_minus_exp(float x) {
+    float p = -1.f / 40320.f;
+    p = fmaf(p, x, 1.f / 5040.f);
+    p = fmaf(p, x, -1.f / 720.f);
+    p = fmaf(p, x, 1.f / 120.f);
+    p = fmaf(p, x, -1.f / 24.f);
+    p = fmaf(p, x, 1.f / 6.f);
+    p = fmaf(p, x, -0.5f);
+    p = fmaf(p, x, 1.f);
+    return x < 0.5f ? p * x : 1.f - __expf(-x);
+}
+
 // cells of the unfolded theta axis, its walls' cosines (descending) and the
 // grid's cell of an unfolded one
 __device__ __forceinline__ int ntheta_u(const DevGrid &g) { return g.mirror ? 2 * g.nt : g.nt; }
 __device__ __forceinline__ double cos_u(const DevGrid &g, bool flip, int j) {
-    if (g.mirror) return j <= g.nt ? g.ctd[j] : -g.ctd[2 * g.nt - j];
-    return flip ? -g.ctd[g.nt - j] : g.ctd[j];
+    const int n = ntheta_u(g);
+    const bool neg = g.mirror ? j > g.nt : flip;  // (one load, whichever side)
+    const double c = g.ctd[neg ? n - j : j];
+    return neg ? -c : c;
 }
 __device__ __forceinline__ int fold_u(const DevGrid &g, bool flip, int j) {
-    if (g.mirror) return j < g.nt ? j : 2 * g.nt - 1 - j;
-    return flip ? g.nt - 1 - j : j;
+    const bool neg = g.mirror ? j >= g.nt : flip;
+    return neg ? ntheta_u(g) - 1 - j : j;
 }
 // the unfolded cell j with cos(wall j) > u >= cos(wall j + 1)
 __device__ __forceinline__ int find_u(const DevGrid &g, bool flip, double u) {
@@ -117,19 +145,13 @@ __device__ __forceinline__ int find_u(const DevGrid &g, bool flip, double u) {
     return lo;
 }
 
-// the ray through sky position (X, Y) (au); false: it misses the grid
-__device__ __forceinline__ bool ray_setup(const CamParams &C, double X, double Y, RayGeo &q) {
+// the crossing sequences of the ray with p0 at (q.x0, q.y0, q.z0) and q.b2; false:
+// it misses the grid.  clear > 0: spheres of R^2 <= b^2 (1 + clear), which a march
+// in FP32 may take for missed, are left out.
+__device__ __forceinline__ bool ray_geometry(const CamParams &C, RayGeo &q, double clear) {
     const DevGrid &g = C.g;
     const double R = g.rwd[g.nr];
-    double xp = X * C.cpa + Y * C.spa, yp = -X * C.spa + Y * C.cpa;
-    // a ray through the origin is moved off it by 1e-12 of the grid's radius
-    // (which direction it would turn to there is not defined)
-    if (xp * xp + yp * yp < 1e-24 * R * R) yp = 1e-12 * R;
-    q.x0 = xp * C.ex[0] + yp * C.ey[0];
-    q.y0 = xp * C.ex[1] + yp * C.ey[1];
-    q.z0 = xp * C.ex[2] + yp * C.ey[2];
     q.dz = -C.nd[2];
-    q.b2 = fma(q.x0, q.x0, fma(q.y0, q.y0, q.z0 * q.z0));
     if (!(q.b2 < R * R)) return false;
     q.S = sqrt(R * R - q.b2);
     q.flip = q.z0 < 0.0;
@@ -142,7 +164,7 @@ __device__ __forceinline__ bool ray_setup(const CamParams &C, double X, double Y
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         const double r = g.rwd[mid];
-        if (r * r > q.b2)
+        if (r * r > q.b2 * (1.0 + clear))
             hi = mid;
         else
             lo = mid;
@@ -164,11 +186,30 @@ __device__ __forceinline__ bool ray_setup(const CamParams &C, double X, double Y
     return true;
 }
 
+// p0 and b^2 of the ray through sky position (X, Y) (au)
+__device__ __forceinline__ void ray_line(const CamParams &C, double X, double Y, RayGeo &q) {
+    const double R = C.g.rwd[C.g.nr];
+    double xp = X * C.cpa + Y * C.spa, yp = -X * C.spa + Y * C.cpa;
+    // a ray through the origin is moved off it by 1e-12 of the grid's radius
+    // (which direction it would turn to there is not defined)
+    if (xp * xp + yp * yp < 1e-24 * R * R) yp = 1e-12 * R;
+    q.x0 = xp * C.ex[0] + yp * C.ey[0];
+    q.y0 = xp * C.ex[1] + yp * C.ey[1];
+    q.z0 = xp * C.ex[2] + yp * C.ey[2];
+    q.b2 = fma(q.x0, q.x0, fma(q.y0, q.y0, q.z0 * q.z0));
+}
+
+// the ray through sky position (X, Y) (au); false: it misses the grid
+__device__ __forceinline__ bool ray_setup(const CamParams &C, double X, double Y, RayGeo &q) {
+    ray_line(C, X, Y, q);
+    return ray_geometry(C, q, 0.0);
+}
+
 // position of the k-th sphere crossing (k = 2 nin: the outer sphere)
 __device__ __forceinline__ double sph_at(const CamParams &C, const RayGeo &q, int k) {
     const bool inw = k < q.nin;
     const double r = C.g.rwd[inw ? C.g.nr - 1 - k : q.w + k - q.nin];
-    const double s = sqrt(fmax(fma(r, r, -q.b2), 0.0));
+    const double s = sqrt_d(fma(r, r, -q.b2));
     return inw ? -s : s;
 }
 
@@ -177,7 +218,7 @@ __device__ __forceinline__ double cone_at(const CamParams &C, const RayGeo &q, i
     if (k >= q.nT) return 1e300;
     const bool A = k < q.nA;
     const double c = cos_u(C.g, q.flip, A ? q.js - k : q.jt + 1 + k - q.nA);
-    const double Q = sqrt(fmax(fma(q.b2, fma(q.dz, q.dz, -c * c), q.z0 * q.z0), 0.0));
+    const double Q = sqrt_d(fma(q.b2, fma(q.dz, q.dz, -c * c), q.z0 * q.z0));
     const double sQ = A ? -Q : Q;
     const double s = fma(q.dz * q.b2, c, q.z0 * sQ) * rcp_d(fma(q.z0, c, -q.dz * sQ));
     return s > -q.S ? (s < q.S ? s : q.S) : -q.S;   // (NaN: -S)
@@ -260,6 +301,99 @@ __device__ __forceinline__ void walk_ray(const CamParams &C, const RayGeo &q, in
     }
 }
 
+// ---- the march of the adjoint.  A gradient's value hangs on which cell a piece
+// of a ray is charged to: where a ray grazes a cone for long, a shift of the wall
+// by an ulp of the radius (1e-5 au at 200 au) moves up to 1e-3 of a cell's
+// gradient to its neighbour, and either is as good.  The adjoint keeps the FP32
+// march from wall to wall (next_wall) that defines those gradients, and takes
+// from the sequences above only where a lane's share begins: at a radial
+// crossing, where the march sets its position on the line again (cross_cam) and
+// so depends on nothing before it.
+struct CamRay {
+    float x0, y0, z0;  // p0 (au)
+    double b2;         // |p0|^2
+};
+
+// the ray's line in FP32; false: it misses the grid
+__device__ __forceinline__ bool cam_line(const CamParams &C, float X, float Y, CamRay &cr) {
+    const float cpa = (float)C.cpa, spa = (float)C.spa;
+    const float xp = fmaf(cpa, X, spa * Y), yp = fmaf(-spa, X, cpa * Y);
+    cr.x0 = fmaf((float)C.ex[0], xp, (float)C.ey[0] * yp);
+    cr.y0 = fmaf((float)C.ex[1], xp, (float)C.ey[1] * yp);
+    cr.z0 = fmaf((float)C.ex[2], xp, (float)C.ey[2] * yp);
+    const double x = cr.x0, y = cr.y0, z = cr.z0, R = C.g.rwd[C.g.nr];
+    cr.b2 = fma(z, z, fma(x, x, y * y));
+    return cr.b2 < R * R;
+}
+
+// puts p on the line at the sphere of wall iw, inbound or outbound
+__device__ __forceinline__ void put_on_sphere(const DevGrid &g, const CamRay &cr, int iw, bool inw,
+                                              Pos &p) {
+    const double rw = g.rwd[iw];
+    float s = (float)sqrt(fmax(fma(rw, rw, -cr.b2), 0.0));
+    if (inw) s = -s;
+    p.x = fmaf(s, p.dx, cr.x0);
+    p.y = fmaf(s, p.dy, cr.y0);
+    p.z = fmaf(s, p.dz, cr.z0);
+}
+
+// Lane l of L marches its share: from the sphere its equal part of the merged
+// crossings begins at (the ray's entry for lane 0) to the one where the next
+// lane's does.  `at` counts the spheres passed as RayGeo does.  imin: the innermost
+// shell of the exact line (a sphere it is tangent to is met or missed as there).
+template <class F>
+__device__ __forceinline__ void march_ray(const CamParams &C, const CamRay &cr, const RayGeo &q,
+                                          int imin, int l, int L, F f) {
+    const DevGrid &g = C.g;
+    const int NR = 2 * q.nin + 1, M = NR + q.nT;
+    int at[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int m0 = (int)(((long long)M * (l + e)) / L);
+        int lo = max(0, m0 - q.nT), hi = min(m0, NR);
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (sph_at(C, q, mid) <= cone_at(C, q, m0 - 1 - mid))
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        at[e] = l + e == L ? NR : lo;
+    }
+    if (at[0] >= at[1]) return;
+    Pos p;
+    p.dx = -C.n[0];
+    p.dy = -C.n[1];
+    p.dz = -C.n[2];
+    const int k = at[0];
+    p.ir = k <= q.nin ? g.nr - 1 - k : q.w - 1 + k - q.nin;
+    if (k <= q.nin)
+        put_on_sphere(g, cr, g.nr - k, true, p);
+    else
+        put_on_sphere(g, cr, p.ir, false, p);
+    p.it = p.ip = 0;
+    p.hemi = 1;
+    locate_angles<1>(g, p);
+    uint32_t nzero = 0;
+    for (int guard = 0; guard < (1 << 24); ++guard) {
+        int kind;
+        const float tw = next_wall<1, true>(g, p, kind, p.ir <= imin);
+        const float rcell = g.rw[p.ir + 1];
+        if (p.ir >= 0 && f(cell_index(g, p), tw)) return;
+        if (kind == W_RIN || kind == W_ROUT || kind == W_HOLE) {
+            const bool inw = kind == W_RIN;
+            const int ir = kind == W_HOLE ? 0 : p.ir + (inw ? -1 : 1);
+            p.ir = ir;
+            if ((inw ? min(g.nr - 1 - ir, q.nin) : q.nin + ir - q.w + 1) >= at[1]) return;
+            put_on_sphere(g, cr, inw ? ir + 1 : ir, inw, p);
+            if (kind == W_HOLE) locate_angles<1>(g, p);
+        } else {
+            cross_wall(g, p, tw, kind);
+        }
+        if (unstick(g, p, tw, rcell, nzero) && p.ir >= g.nr) return;
+    }
+}
+
 // what a lane's share of a ray adds up to
 template <class A>
 struct RaySum {
@@ -273,7 +407,7 @@ struct RaySum {
 // 1 - e^-dtau and e^-dtau as two numbers that sum to 1
 __device__ __forceinline__ void absorb(float dtau, double &om, double &e) {
     const bool thin = dtau < 0.5f;
-    const double x = thin ? (double)-expm1f(-dtau) : (double)__expf(-dtau);
+    const double x = thin ? (double)one_minus_exp(dtau) : (double)__expf(-dtau);
     om = thin ? x : 1.0 - x;
     e = thin ? 1.0 - x : x;
 }
@@ -285,8 +419,8 @@ __device__ __forceinline__ void absorb(float dtau, double &om, double &e) {
 // is summed in; in double (the adjoint) the attenuation is the running product
 // of the segments' e^-dtau, so that emission and attenuation of a segment add up
 // to what comes in, whatever their rounding.
-template <bool LMIN, class A>
-__device__ __forceinline__ A trace_ray(const CamParams &C, const RayGeo &q, bool act, int l, int L,
+template <bool LMIN, class A, class W>
+__device__ __forceinline__ A trace_ray(const CamParams &C, const W &walk, bool act, int l, int L,
                                        RaySum<A> &r, uint32_t &nseg) {
     r.I = 0;
     r.tau = r.tau0 = 0.f;
@@ -300,7 +434,7 @@ __device__ __forceinline__ A trace_ray(const CamParams &C, const RayGeo &q, bool
         A I = 0;
         att = 1;
         ns = 0;
-        walk_ray(C, q, l, L, [&](int c, float ds) {
+        walk([&](int c, float ds) {
             ++ns;
             if (LMIN) lm = fminf(lm, C.csize[c]);
             const float dtau = C.alpha[c] * ds;
@@ -311,7 +445,7 @@ __device__ __forceinline__ A trace_ray(const CamParams &C, const RayGeo &q, bool
                     I = fma((A)(att * om), (A)C.src[c], I);
                     att *= (A)e;
                 } else {
-                    I = fma((A)(__expf(-tau) * (-expm1f(-dtau))), (A)C.src[c], I);
+                    I = fma((A)(__expf(-tau) * one_minus_exp(dtau)), (A)C.src[c], I);
                 }
             }
             tau += dtau;
@@ -373,6 +507,11 @@ __device__ __forceinline__ double sky_y(const CamParams &C, int j, int a) {
     return ((double)(j - C.ny / 2) + ((a + 0.5) / C.nsub - 0.5)) * C.pix;
 }
 
+// (in FP32, as the adjoint's march takes them)
+__device__ __forceinline__ float sky_f(const CamParams &C, int k, int n, int b) {
+    return ((float)(k - n / 2) + ((b + 0.5f) / C.nsub - 0.5f)) * C.pixf;
+}
+
 #define IMG_BS 256
 #define IMG_LANES 524288u  // lanes a launch is spread over, if the rays allow
 #define IMG_MAXL 32         // at most this many of them per ray
@@ -389,7 +528,8 @@ __global__ void __launch_bounds__(IMG_BS) k_image(CamParams C, float *img) {
             RayGeo q;
             RaySum<float> r;
             const bool act = in && ray_setup(C, sky_x(C, k, b), sky_y(C, j, a), q);
-            acc += trace_ray<false>(C, q, act, l, L, r, nseg);
+            auto walk = [&](auto f) { walk_ray(C, q, l, L, f); };
+            acc += trace_ray<false>(C, walk, act, l, L, r, nseg);
         }
     if (in && l == 0) img[j * C.nx + k] = acc / (float)(C.nsub * C.nsub);
     count_crossings(C.icount, nseg);
@@ -443,21 +583,41 @@ __device__ __forceinline__ void adj_flush(const int *key, const u64 *ga, const u
     }
 }
 
-// gI times the gradient of the ray through sky (X, Y) w.r.t. the per-cell
+// gI times the gradient of the ray through sky (X, Y) ((Xf, Yf) in FP32) w.r.t. the per-cell
 // alpha and S, by L neighbouring lanes: the ray is integrated for I, then each
 // lane sweeps its share again front to back recomputing tau (nothing is stored
 // per segment).  What lies behind segment k, R_k = I - I_<=k, is what the same
 // sums leave of the lane's own share (the sweep repeats the integration's
 // operations, in FP64, so no rounding is left over where R_k is small) plus the
 // shares behind it.
-__device__ __forceinline__ void adjoint_ray(const CamParams &C, double X, double Y, float gI, int l,
-                                            int L, int *key, u64 *ga, u64 *gs, double *g_alpha,
+__device__ __forceinline__ void adjoint_ray(const CamParams &C, double X, double Y, float Xf,
+                                            float Yf, float gI, int l, int L, int *key, u64 *ga, u64 *gs, double *g_alpha,
                                             double *g_src, uint32_t &nseg) {
     RayGeo q;
+    CamRay cr;
     RaySum<double> r;
-    const bool act = gI != 0.f && ray_setup(C, X, Y, q);
+    int imin = 0;
+    bool act = gI != 0.f && cam_line(C, Xf, Yf, cr);
+    if (act) {
+        ray_line(C, X, Y, q);
+        const double b2 = q.b2;
+        q.x0 = cr.x0;
+        q.y0 = cr.y0;
+        q.z0 = cr.z0;
+        q.b2 = cr.b2;
+        if (cr.b2 == 0.0) ray_line(C, X, Y, q);  // (for the shares only)
+        act = ray_geometry(C, q, 1e-4);
+        if (act) {
+            imin = q.w - 1;
+            for (; imin >= 0; --imin) {
+                const double w = C.g.rwd[imin];
+                if (!(w * w > b2)) break;
+            }
+        }
+    }
     uint32_t nfwd = 0;
-    (void)trace_ray<false>(C, q, act, l, L, r, nfwd);
+    auto walk = [&](auto f) { march_ray(C, cr, q, imin, l, L, f); };
+    (void)trace_ray<false>(C, walk, act, l, L, r, nfwd);
     double behind = r.I * r.front;
     if (L > 1) {
         double x = behind;
@@ -472,7 +632,7 @@ __device__ __forceinline__ void adjoint_ray(const CamParams &C, double X, double
     const double qa = C.qs[0] * (double)gI, qsrc = C.qs[1] * (double)gI;
     float tau = 0.f;
     double cum = 0.0, att = 1.0;
-    walk_ray(C, q, l, L, [&](int c, float ds) {
+    walk([&](int c, float ds) {
         ++nseg;
         const float dtau = C.alpha[c] * ds;
         const double S = C.src[c];
@@ -508,8 +668,8 @@ __global__ void __launch_bounds__(IMG_BS) k_image_adj(CamParams C, const float *
     uint32_t nseg = 0;
     for (int a = 0; a < C.nsub; ++a)
         for (int b = 0; b < C.nsub; ++b)
-            adjoint_ray(C, in ? sky_x(C, k, b) : 0.0, in ? sky_y(C, j, a) : 0.0, gI, l, L, key, ga,
-                        gs, g_alpha, g_src, nseg);
+            adjoint_ray(C, sky_x(C, k, b), sky_y(C, j, a), sky_f(C, k, C.nx, b),
+                        sky_f(C, j, C.ny, a), gI, l, L, key, ga, gs, g_alpha, g_src, nseg);
     __syncthreads();
     adj_flush(key, ga, gs, H, g_alpha, g_src);
     count_crossings(C.icount ? C.icount + 1 : nullptr, nseg);
@@ -577,8 +737,8 @@ __global__ void k_ref_init(CamParams C, RefArgs R) {
     int j, k, a, b;
     float2 xy = make_float2(RT_REF_DEAD, RT_REF_DEAD);  // tile padding: no ray
     if (node0_pixel(C, R.ns2, i, j, k, a, b)) {
-        xy.x = (float)sky_x(C, k, b);
-        xy.y = (float)sky_y(C, j, a);
+        xy.x = sky_f(C, k, C.nx, b);
+        xy.y = sky_f(C, j, C.ny, a);
     }
     R.xy[i] = xy;
 }
@@ -610,7 +770,8 @@ __global__ void __launch_bounds__(256) k_ref_trace(CamParams C, RefArgs R, int L
         RayGeo q;
         RaySum<float> r;
         const bool ray = act && xy.x < 0.5f * RT_REF_DEAD && ray_setup(C, xy.x, xy.y, q);
-        const float I = trace_ray<true>(C, q, ray, l, LN, r, nseg);
+        auto walk = [&](auto f) { walk_ray(C, q, l, LN, f); };
+        const float I = trace_ray<true>(C, walk, ray, l, LN, r, nseg);
         const bool first = act && l == 0;
         if (first) R.val[i] = I;
         if (first && ray) ++nrays;
@@ -730,7 +891,7 @@ __global__ void __launch_bounds__(256) k_ref_adj(CamParams C, RefArgs R, double 
             xy = R.xy[i];
             g = xy.x < 0.5f * RT_REF_DEAD ? R.gw[i] : 0.f;
         }
-        adjoint_ray(C, xy.x, xy.y, g, l, LN, key, ga, gs, g_alpha, g_src, nseg);
+        adjoint_ray(C, xy.x, xy.y, xy.x, xy.y, g, l, LN, key, ga, gs, g_alpha, g_src, nseg);
         __syncthreads();
         adj_flush(key, ga, gs, H, g_alpha, g_src);
         __syncthreads();

@@ -283,9 +283,13 @@ __device__ __forceinline__ float phi_hit(float x, float y, float dx, float dy, f
     return hit ? t : RT_INF;
 }
 
-// distance to the next wall of the current cell and which wall it is
-template <int XF>
-__device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &kind) {
+// distance to the next wall of the current cell and which wall it is.  noin: the
+// inner sphere is not met.  EQ: a cone that is a plane but for the rounding of
+// pi/2 -- the equator of a grid over [0, pi] -- is taken as the plane (its
+// quadratic has a double root).
+template <int XF, bool EQ = false>
+__device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &kind,
+                                           bool noin = false) {
     const bool in = p.ir >= 0;
     const int i = in ? p.ir : 0, j = p.it;
     // the walls' words first: one wait for all of them
@@ -311,7 +315,7 @@ __device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &
     {
         const float c = rr - R2i;
         const float D = fmaf(b, b, -c);
-        const bool cand = in && b < 0.f && !(D < -1e-5f * (rr + R2i));
+        const bool cand = in && !noin && b < 0.f && !(D < -1e-5f * (rr + R2i));
         float t = fmaxf(c / (sqrtf(D) - b), 0.f);
         if (cand && D < 1e-4f * b * b) t = sph_in_d<XF>(p, g.rwd[i]);
         const bool hit = cand && t < tb;
@@ -321,7 +325,7 @@ __device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &
     // lower cone; the equatorial plane of a full-sphere grid is left upwards
     // (a crossing behind the position is taken at once)
     {
-        const bool plane = !g.mirror && ctl == 0.f;
+        const bool plane = !g.mirror && (EQ ? fabsf(ctl) < 1e-6f : ctl == 0.f);
         float t = cone_hit<XF>(p, q, ctl, stl, g.ctd + j, g.std_ + j, -1, in && j > 0 && !plane);
         if (!g.mirror && plane && in && j > 0 && p.dz > 0.f) t = fmaxf(-p.z / p.dz, 0.f);
         const bool hit = t < tb;
@@ -331,7 +335,7 @@ __device__ __forceinline__ float next_wall(const DevGrid &g, const Pos &p, int &
     // upper cone, or the mirror plane under the last row of cells
     {
         const bool last = j + 1 == g.nt;
-        const bool plane = !g.mirror && cth == 0.f;
+        const bool plane = !g.mirror && (EQ ? fabsf(cth) < 1e-6f : cth == 0.f);
         float t = cone_hit<XF>(p, q, cth, sth, g.ctd + j + 1, g.std_ + j + 1, +1,
                                in && !last && !plane);
         const bool fold = g.mirror ? last && q.dz < 0.f : plane && !last && p.dz < 0.f;
