@@ -8,105 +8,145 @@
 // gridded sampler further down samples it as galario does.
 // chi^2 = sum w ((Re_d - Re_m)^2 + (Im_d - Im_m)^2) (libinterferometry.pyx:619-633).
 //
-// Forward: one (u,v) point per lane in each of four row groups of a
-// workgroup; the image is staged through LDS in column strips and read as
-// wave-wide broadcasts; the strip's column phasors sit in registers and the row
-// phasor is one sincospi every 16 rows and a rotation by one row step in
-// between, so the inner loop is two FMAs per pixel.  Adjoint: 16x16 tiles, four groups of lanes per tile taking alternate
-// chunks of 64 points; per chunk the tile's column phasors (times the point's
-// complex cotangent) and row phasors are built once in LDS, and the tile's
-// update G += B^T Ha (16 x 16, 4 points deep) runs on v_mfma_f32_16x16x4f32.
+// Both directions of the exact DFT run on the matrix cores over the image folded
+// about its centre (c_x, c_y) = the middle of its pixel positions: with
+// x_k - c_x = +-X_m and y_j - c_y = +-Y_l the four pixels of a (l, m) pair enter as
+// their sums and differences, with cosines and sines of X_m and Y_l alone --
+// half the multiplications of the plain sum, and real ones.
 #include <cmath>
 #include <mutex>
 
 #include "rt_internal.h"
 
 #define VIS_BS 256
-#define VIS_STRIP 32
 #define VIS_MAXROWS 1024
-#define VIS_G 4  // row groups per workgroup of the forward DFT
+#define VIS_TK 32  // columns (of the folded image) per staged tile
+#define VIS_REF 8  // matrix-core steps between exact phasors
 
-// NG groups of VIS_BS lanes per workgroup share the points and take a
-// contiguous range of rows each; their sums are added in group order
-template <int NG>
-__global__ void __launch_bounds__(VIS_BS * NG) k_vis(const float *img, int nx, int ny,
-                                                     const double *u, const double *v, int K,
-                                                     double dxy, double dra, double ddec,
-                                                     float *re, float *im) {
-    constexpr int ng = NG;
-    __shared__ float strip[VIS_MAXROWS * VIS_STRIP / 4];  // rows x 8 columns per pass (32 KB)
-    const int g = NG == 1 ? 0 : (int)threadIdx.x / VIS_BS;
-    const int lt = (int)threadIdx.x - g * VIS_BS;
-    const int q = blockIdx.x * VIS_BS + lt;
-    const bool act = q < K;
-    const int rpg = NG == 1 ? ny : (ny + ng - 1) / ng;
-    const int jb = NG == 1 ? 0 : min(ny, g * rpg), je = NG == 1 ? ny : min(ny, jb + rpg);
-    float ud = 0.f, vd = 0.f;
-    if (act) {
-        ud = (float)(u[q] * dxy);
-        vd = (float)(v[q] * dxy);
-    }
+typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef float vf16 __attribute__((ext_vector_type(16)));
+
+// cos and sin of 2 pi a, a reduced in FP64
+__device__ __forceinline__ void phasor(double a, float &c, float &s) {
+    sincospif(2.f * (float)(a - rint(a)), &s, &c);
+}
+
+// entries of a folded axis of n pixels and the first one's distance from the
+// centre (pixels): pixel n/2 + l lies at l + off, its partner at -(l + off)
+__device__ __host__ __forceinline__ int fold_n(int n) { return (n + 1) / 2; }
+__device__ __forceinline__ double fold_off(int n) { return (n & 1) ? 0.0 : 0.5; }
+__device__ __forceinline__ int fold_lo(int n, int l) { return (n & 1) ? n / 2 - l : n / 2 - 1 - l; }
+
+// V(u,v): with the folded planes EE, EO, OE, OO (E: sum, O: difference; first
+// letter rows), a = 2 pi u X_m, b = 2 pi v Y_l,
+//   Re V = sum_l cos b (sum_m EE cos a) - sin b (sum_m OO sin a)
+//   Im V = -sum_l cos b (sum_m EO sin a) + sin b (sum_m OE cos a)
+// times the shift of the centre.  The inner sums are four products
+// [32 rows x m] x [m x 32 points] with v_mfma_f32_32x32x2f32: a lane holds its
+// point's cos a or sin a of one column (rotated by two pixels a step, exact
+// every VIS_REF steps, so no table is needed), the folded rows come from LDS, one
+// 16-byte read per step for all four.  2 nx ny flops per point: 6.5 GFLOP
+// at 256 x 256 and 5e4 points, 42 us at the FP32 matrix peak.  4 / NRS groups of 32
+// points per workgroup share the staged rows; with NRS = 4 the four waves take
+// every fourth 32 rows of one group of points instead (few points: the GPU would
+// be short of waves), added in order.
+template <int NRS>
+__global__ void __launch_bounds__(VIS_BS) k_vis(const float *img, int nx, int ny, const double *u,
+                                                const double *v, int K, double dxy, double dra,
+                                                double ddec, float *re, float *im) {
+    constexpr int NP = 4 / NRS;
+    __shared__ vf4 pl[NRS][32][VIS_TK + 1];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, rs = w % NRS, pg = w / NRS;
+    const int i32 = lane & 31, kh = lane >> 5;
+    const int q = (blockIdx.x * NP + pg) * 32 + i32;
+    const int hx = fold_n(nx), hy = fold_n(ny);
+    const double ox = fold_off(nx), oy = fold_off(ny);
+    const double uq = q < K ? u[q] : 0.0, vq = q < K ? v[q] : 0.0;
+    const double ud = uq * dxy, vd = vq * dxy;
+    float c2, s2, c1, s1;  // two columns, one row
+    phasor(2.0 * ud, c2, s2);
+    phasor(vd, c1, s1);
     float sr = 0.f, si = 0.f;
-    float ds, dc;  // one row step of the row phasor
-    sincospif(-2.f * vd, &ds, &dc);
-    // process columns in strips of 8 so that a strip of up to 1024 rows fits LDS
-    const int W = 8;
-    for (int k0 = 0; k0 < nx; k0 += W) {
-        int wk = min(W, nx - k0);
-        __syncthreads();
-        for (int i = threadIdx.x; i < ny * W; i += VIS_BS * ng) {
-            int j = i / W, kk = i - j * W;
-            strip[i] = (kk < wk) ? img[(size_t)j * nx + k0 + kk] : 0.f;
-        }
-        __syncthreads();
-        float ar[W], ai[W];
-#pragma unroll
-        for (int kk = 0; kk < W; ++kk) {
-            float s, c;
-            sincospif(-2.f * ud * (float)(k0 + kk - nx / 2), &s, &c);
-            ar[kk] = c;
-            ai[kk] = s;
-        }
-        // row phasors: exact every 16 rows from the group's first row, rotated
-        // by one row step in between (FP32 drift below 2e-6 over 15 rotations)
-        float bs = 0.f, bc = 1.f;
-        for (int j = jb; j < je; ++j) {
-            const float *row = strip + j * W;
-            float rr = 0.f, ri = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < W; ++kk) {
-                rr = fmaf(row[kk], ar[kk], rr);
-                ri = fmaf(row[kk], ai[kk], ri);
+    const int nt = (hy + 32 * NRS - 1) / (32 * NRS);
+    for (int t = 0; t < nt; ++t) {
+        const int l0 = (t * NRS + rs) * 32;
+        vf16 pee = {}, poo = {}, peo = {}, poe = {};
+        for (int m0 = 0; m0 < hx; m0 += VIS_TK) {
+            __syncthreads();
+            for (int e = pg * 64 + lane; e < 32 * VIS_TK; e += NP * 64) {
+                const int l = l0 + e / VIS_TK, m = m0 + e % VIS_TK;
+                float a = 0.f, b = 0.f, c = 0.f, d = 0.f;
+                if (l < hy && m < hx) {
+                    const int jp = ny / 2 + l, jm = fold_lo(ny, l), kp = nx / 2 + m,
+                              km = fold_lo(nx, m);
+                    const bool two_r = jm != jp, two_c = km != kp;
+                    a = img[(size_t)jp * nx + kp];
+                    if (two_c) b = img[(size_t)jp * nx + km];
+                    if (two_r) c = img[(size_t)jm * nx + kp];
+                    if (two_r && two_c) d = img[(size_t)jm * nx + km];
+                }
+                const float ab = a + b, cd = c + d, am = a - b, cm = c - d;
+                vf4 o = {ab + cd, am - cm, am + cm, ab - cd};  // EE, OO, EO, OE
+                pl[rs][e / VIS_TK][e % VIS_TK] = o;
             }
-            if (((j - jb) & 15) == 0) {
-                sincospif(-2.f * vd * (float)(j - ny / 2), &bs, &bc);
-            } else {
-                const float nc = bc * dc - bs * ds;
-                bs = fmaf(bc, ds, bs * dc);
-                bc = nc;
+            __syncthreads();
+            const int ns = min(VIS_TK, (hx - m0 + 1) & ~1) / 2;
+            float ca = 1.f, sa = 0.f;
+            for (int st = 0; st < ns; ++st) {
+                const int m = 2 * st + kh;
+                if (st % VIS_REF == 0) {
+                    phasor(ud * ((double)(m0 + m) + ox), ca, sa);
+                } else {
+                    const float nc = ca * c2 - sa * s2;
+                    sa = fmaf(ca, s2, sa * c2);
+                    ca = nc;
+                }
+                const vf4 f = pl[rs][i32][m];
+                pee = __builtin_amdgcn_mfma_f32_32x32x2f32(f[0], ca, pee, 0, 0, 0);
+                poo = __builtin_amdgcn_mfma_f32_32x32x2f32(f[1], sa, poo, 0, 0, 0);
+                peo = __builtin_amdgcn_mfma_f32_32x32x2f32(f[2], sa, peo, 0, 0, 0);
+                poe = __builtin_amdgcn_mfma_f32_32x32x2f32(f[3], ca, poe, 0, 0, 0);
             }
-            sr += rr * bc - ri * bs;
-            si += rr * bs + ri * bc;
+        }
+        // lane: point i32, rows l0 + 8 g + 4 kh .. + 3 in elements 4 g .. 4 g + 3
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float cb, sb;
+            phasor(vd * ((double)(l0 + 8 * g + 4 * kh) + oy), cb, sb);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 4 * g + e;
+                sr += cb * pee[r] - sb * poo[r];
+                si -= cb * peo[r] + sb * poe[r];
+                const float nc = cb * c1 - sb * s1;
+                sb = fmaf(cb, s1, sb * c1);
+                cb = nc;
+            }
         }
     }
-    // the groups' sums through the strip buffer (free after the last strip)
-    if (ng > 1) __syncthreads();
-    float *red = strip;  // [2][VIS_G - 1][VIS_BS]
-    if (g > 0) {
-        red[(g - 1) * VIS_BS + lt] = sr;
-        red[((VIS_G - 1) + g - 1) * VIS_BS + lt] = si;
-    }
-    if (ng > 1) __syncthreads();
-    if (g == 0 && act) {
-        for (int h = 0; h < ng - 1; ++h) {
-            sr += red[h * VIS_BS + lt];
-            si += red[((VIS_G - 1) + h) * VIS_BS + lt];
+    sr += __shfl_xor(sr, 32);
+    si += __shfl_xor(si, 32);
+    if (NRS > 1) {
+        __syncthreads();
+        float *red = (float *)&pl[0][0][0];  // [NRS][2][32]
+        if (kh == 0) {
+            red[rs * 64 + i32] = sr;
+            red[rs * 64 + 32 + i32] = si;
         }
-        double ph = -2.0 * (u[q] * dra + v[q] * ddec);
-        double s, c;
-        sincospi(ph, &s, &c);
-        re[q] = (float)(sr * c - si * s);
-        im[q] = (float)(sr * s + si * c);
+        __syncthreads();
+        sr = si = 0.f;
+#pragma unroll
+        for (int r = 0; r < NRS; ++r) {
+            sr += red[r * 64 + i32];
+            si += red[r * 64 + 32 + i32];
+        }
+    }
+    if (rs == 0 && kh == 0 && q < K) {
+        // the image's phase centre lies ox, oy pixels past the folding centre
+        double sn, cs;
+        sincospi(-2.0 * (uq * dra + vq * ddec - ox * ud - oy * vd), &sn, &cs);
+        re[q] = (float)(sr * cs - si * sn);
+        im[q] = (float)(sr * sn + si * cs);
     }
 }
 
@@ -114,8 +154,6 @@ __global__ void __launch_bounds__(VIS_BS * NG) k_vis(const float *img, int nx, i
 #define ADJ_CH 64
 #define ADJ_G 4   // point groups per tile: each takes every ADJ_G-th chunk of points
 #define ADJ_BS (ADJ_T * ADJ_T * ADJ_G)
-
-typedef float vf4 __attribute__((ext_vector_type(4)));
 
 // g[j][k] = Re sum_q H_q a_qk b_qj,  H_q = (gre_q - i gim_q) shift_q,
 // a_qk = exp(-2 pi i u_q x_k), b_qj = exp(-2 pi i v_q y_j)
@@ -513,10 +551,10 @@ int vis_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const d
     if (K == 0) return RT_OK;
     if (!d_img || !d_u || !d_v || !d_re || !d_im)
         return set_err(ctx, RT_E_ARG, "vis: NULL image, (u,v) or output");
-    // row groups only where the points alone leave the GPU short of waves
-    const int nb = (K + VIS_BS - 1) / VIS_BS;
-    if (nb < 2 * ctx->n_cu)
-        hipLaunchKernelGGL(k_vis<VIS_G>, dim3(nb), dim3(VIS_BS * VIS_G), 0, ctx->stream, d_img, nx,
+    // rows split over the waves where the points alone leave the GPU short of them
+    const int nb = (K + 127) / 128;
+    if (nb < 2 * ctx->n_cu && ny > 64)
+        hipLaunchKernelGGL(k_vis<4>, dim3((K + 31) / 32), dim3(VIS_BS), 0, ctx->stream, d_img, nx,
                            ny, d_u, d_v, K, dxy, dra, ddec, d_re, d_im);
     else
         hipLaunchKernelGGL(k_vis<1>, dim3(nb), dim3(VIS_BS), 0, ctx->stream, d_img, nx, ny, d_u,
