@@ -325,9 +325,10 @@ int rt_create(int device, rt_ctx **out) {
 }
 
 rt_ctx::~rt_ctx() {
-    void *p[] = {ref.xy, ref.val, ref.child, ref.gw, ref.ctl, d_icount};
+    void *p[] = {ref.xy, ref.val, ref.child, ref.gw, ref.ctl, d_icount, vis_ws};
     for (void *q : p)
         if (q) (void)hipFree(q);
+    if (vis_ws_ev) (void)hipEventDestroy(vis_ws_ev);
 }
 
 int rt_destroy(rt_ctx *ctx) {
@@ -648,7 +649,7 @@ int rt_vis_dft_adjoint(rt_ctx *ctx, const float *d_gre, const float *d_gim, int 
                        double dxy, const double *d_u, const double *d_v, int K, double dra,
                        double ddec, float *d_g_img) {
     if (!ctx) return RT_E_ARG;
-    return vis_adjoint_run(ctx, d_gre, d_gim, nx, ny, dxy, d_u, d_v, K, dra, ddec, d_g_img);
+    return vis_adjoint_run(ctx, d_gre, d_gim, nx, ny, dxy, d_u, d_v, K, dra, ddec, d_g_img, nullptr);
 }
 
 int rt_vis_grid(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const double *d_u,

@@ -46,6 +46,13 @@ struct rt_ctx {
     int n_cu = 0;
     int wallclock_khz = 0;
     RefinePool ref;
+    // scratch of the transposed DFT's partial sums: at most 64 KiB for
+    // each of 4 x CUs workgroups, kept between calls; its last user's stream and an event behind that use
+    void *vis_ws = nullptr;
+    size_t vis_ws_cap = 0;
+    hipEvent_t vis_ws_ev = nullptr;
+    hipStream_t vis_ws_stream = nullptr;
+    bool vis_ws_used = false;
     // cells crossed by camera rays since the last read: [0] image rays
     // (sub-pixels included), [1] adjoint sweeps
     unsigned long long *d_icount = nullptr;
@@ -243,9 +250,13 @@ int image_adjoint_run(rt_model *m, const rt_camera *cam, const float *d_T, const
                       const float *d_dimg, float *d_g_logrho, float *d_g_T);
 int vis_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const double *d_u,
             const double *d_v, int K, double dra, double ddec, float *d_re, float *d_im);
+// ws: vis_adjoint_workspace bytes, or NULL (the context's; in a capture none, and
+// the kernel that needs none runs)
 int vis_adjoint_run(rt_ctx *ctx, const float *d_gre, const float *d_gim, int nx, int ny,
                     double dxy, const double *d_u, const double *d_v, int K, double dra,
-                    double ddec, float *d_g_img);
+                    double ddec, float *d_g_img, void *ws);
+// bytes of scratch the transposed DFT wants (0: none)
+size_t vis_adjoint_workspace(const rt_ctx *ctx, int nx, int ny, int K);
 // ws: nullable workspace of chisq_workspace(K) doubles (else allocated stream-ordered)
 int chisq_run(rt_ctx *ctx, const float *dre, const float *dim, const float *w, const float *mre,
               const float *mim, int K, double *out, float *gre, float *gim, double *ws);

@@ -13,6 +13,7 @@
 // x_k - c_x = +-X_m and y_j - c_y = +-Y_l the four pixels of a (l, m) pair enter as
 // their sums and differences, with cosines and sines of X_m and Y_l alone --
 // half the multiplications of the plain sum, and real ones.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -150,6 +151,164 @@ __global__ void __launch_bounds__(VIS_BS) k_vis(const float *img, int nx, int ny
     }
 }
 
+// ---- the transpose: g[j][k] = Re sum_q H_q exp(-i (+-a_qm +- b_ql)) about the
+// folding centre, H_q = (gre_q - i gim_q) times the shift, a = 2 pi u X_m, b = 2 pi v
+// Y_l.  With
+//   P1 = sum Hr cos a cos b, P2 = sum Hr sin a sin b,
+//   P3 = sum Hi sin a cos b, P4 = sum Hi cos a sin b
+// the pixel at signs (s, t) of (X, Y) is P1 - s t P2 + s P3 + t P4: four products
+// [l x q] x [q x m] on v_mfma_f32_32x32x2f32, half the multiplications of the
+// plain sum.  A workgroup takes 64 x 64 entries (l, m) -- four waves of 32 x 32 --
+// and a share of the points, 32 at a time: their cosines and sines go through
+// LDS once (16 entries per lane, exact every 8, rotated in between) and serve
+// 64 x 64 x 4 products, so the matrix cores set the pace.  The folded image has
+// few such tiles, so the points are split over two workgroups per CU;
+// their partial planes are added in order by k_vis_adj_sum.
+// 256 x 256 pixels, 5e4 points: 467 us with k_vis_adj, 111 now; 1024 x 1024: 7446
+// and 1241.
+#define VA_CH 32  // points per chunk
+// below this many pixel x point products k_vis_adj, which needs no scratch and one
+// launch, is the faster one: 22 against 27 us at 256 x 256 and 2e3 points, 51
+// against 31 at 5e3 (smaller images count as 256 x 256: they take as long)
+#define VIS_ADJ_MIN (65536.0 * 3072.0)
+
+struct AdjSplit {
+    int tx, ty, splits, per;  // tiles, shares of the points, chunks per share
+};
+
+static AdjSplit adj_split(const rt_ctx *ctx, int nx, int ny, int K) {
+    AdjSplit a;
+    a.tx = (fold_n(nx) + 63) / 64;
+    a.ty = (fold_n(ny) + 63) / 64;
+    const long tiles = (long)a.tx * a.ty, chunks = ((long)K + VA_CH - 1) / VA_CH;
+    long s = (2l * ctx->n_cu + tiles - 1) / tiles;
+    s = std::max(1l, std::min(s, (chunks + 3) / 4));
+    a.per = (int)((chunks + s - 1) / s);
+    a.splits = (int)((chunks + a.per - 1) / a.per);
+    return a;
+}
+
+static bool adj_tiled(int nx, int ny, int K) {
+    return std::max(65536.0, (double)nx * ny) * K >= VIS_ADJ_MIN;
+}
+
+// at most (2 n_cu + tiles) planes' worth: 64 MiB on 256 CUs
+size_t vis_adjoint_workspace(const rt_ctx *ctx, int nx, int ny, int K) {
+    if (nx < 1 || ny < 1 || !adj_tiled(nx, ny, K)) return 0;
+    const AdjSplit a = adj_split(ctx, nx, ny, K);
+    return a.splits > 1 ? (size_t)a.tx * a.ty * a.splits * 4 * 64 * 64 * sizeof(float) : 0;
+}
+
+// the four pixels of the folded entry (l, m)
+__device__ __forceinline__ void unfold_pixels(int l, int m, int nx, int ny, float p1, float p2,
+                                              float p3, float p4, float *gimg) {
+    if (l >= fold_n(ny) || m >= fold_n(nx)) return;
+    const int jp = ny / 2 + l, jm = fold_lo(ny, l), kp = nx / 2 + m, km = fold_lo(nx, m);
+    gimg[(size_t)jp * nx + kp] = (p1 - p2) + (p3 + p4);
+    if (km != kp) gimg[(size_t)jp * nx + km] = (p1 + p2) + (p4 - p3);
+    if (jm != jp) gimg[(size_t)jm * nx + kp] = (p1 + p2) + (p3 - p4);
+    if (jm != jp && km != kp) gimg[(size_t)jm * nx + km] = (p1 - p2) - (p3 + p4);
+}
+
+__global__ void __launch_bounds__(256) k_vis_adj_part(const float *gre, const float *gim, int nx,
+                                                      int ny, const double *u, const double *v,
+                                                      int K, double dxy, double dra, double ddec,
+                                                      int per, float *part, float *gimg) {
+    __shared__ float2 ra[VA_CH][64 + 1], ca[VA_CH][64 + 1];  // rows: cos b, sin b; columns: cos a, sin a
+    __shared__ float2 H[VA_CH];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i32 = lane & 31, kh = lane >> 5, wr = (w >> 1) * 32, wc = (w & 1) * 32;
+    const int l0 = blockIdx.y * 64, m0 = blockIdx.x * 64;
+    const double ox = fold_off(nx), oy = fold_off(ny);
+    vf16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
+    // table: lane of point tp, 16 rows (tg < 4) or columns
+    const int tp = threadIdx.x >> 3, tg = threadIdx.x & 7;
+    const int c0 = blockIdx.z * per, c1 = min(c0 + per, (K + VA_CH - 1) / VA_CH);
+    for (int c = c0; c < c1; ++c) {
+        const int q = c * VA_CH + tp;
+        const double uq = q < K ? u[q] : 0.0, vq = q < K ? v[q] : 0.0;
+        __syncthreads();
+        {
+            const bool row = tg < 4;
+            const int e0 = (tg & 3) * 16;
+            const double f = (row ? vq : uq) * dxy;
+            const double base = (row ? (double)l0 + oy : (double)m0 + ox) + e0;
+            float2(*tab)[64 + 1] = row ? ra : ca;
+            float cs, sn, c1s, s1s;
+            phasor(f, c1s, s1s);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                if (e % 8 == 0) {
+                    phasor(f * (base + e), cs, sn);
+                } else {
+                    const float nc = cs * c1s - sn * s1s;
+                    sn = fmaf(cs, s1s, sn * c1s);
+                    cs = nc;
+                }
+                tab[tp][e0 + e] = make_float2(cs, sn);
+            }
+            if (tg == 0) {
+                float hr = 0.f, hi = 0.f;
+                if (q < K) {
+                    double s, cc;
+                    sincospi(-2.0 * (uq * dra + vq * ddec - (ox * uq + oy * vq) * dxy), &s, &cc);
+                    const float gr = gre[q], gi = gim[q];
+                    hr = (float)(gr * cc + gi * s);
+                    hi = (float)(gr * s - gi * cc);
+                }
+                H[tp] = make_float2(hr, hi);
+            }
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int st = 0; st < VA_CH / 2; ++st) {
+            const int k = 2 * st + kh;
+            const float2 r = ra[k][wr + i32], a = ca[k][wc + i32], h = H[k];
+            p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.x, h.x * a.x, p1, 0, 0, 0);
+            p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.y, h.x * a.y, p2, 0, 0, 0);
+            p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.x, h.y * a.y, p3, 0, 0, 0);
+            p4 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.y, h.y * a.x, p4, 0, 0, 0);
+        }
+    }
+    if (!part) {  // one share: no planes
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            unfold_pixels(l0 + wr + 8 * (r >> 2) + 4 * kh + (r & 3), m0 + wc + i32, nx, ny, p1[r],
+                          p2[r], p3[r], p4[r], gimg);
+        return;
+    }
+    // [share][tile][plane][64][64]
+    float *o = part + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) *
+                          (4 * 64 * 64);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int at = (wr + 8 * (r >> 2) + 4 * kh + (r & 3)) * 64 + wc + i32;
+        o[at] = p1[r];
+        o[at + 4096] = p2[r];
+        o[at + 2 * 4096] = p3[r];
+        o[at + 3 * 4096] = p4[r];
+    }
+}
+
+// one folded entry (l, m) per lane: the shares' planes added in order, four pixels
+__global__ void __launch_bounds__(256) k_vis_adj_sum(const float *part, int splits, int nx, int ny,
+                                                     float *gimg) {
+    const int tx = gridDim.x, ty = gridDim.y;
+    const int e = blockIdx.z * 256 + threadIdx.x;  // of the tile's 64 x 64
+    const int l = blockIdx.y * 64 + e / 64, m = blockIdx.x * 64 + e % 64;
+    const float *p = part + ((size_t)blockIdx.y * tx + blockIdx.x) * (4 * 4096) + e;
+    float p1 = 0.f, p2 = 0.f, p3 = 0.f, p4 = 0.f;
+    const size_t step = (size_t)tx * ty * (4 * 4096);
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s, p += step) {
+        p1 += p[0];
+        p2 += p[4096];
+        p3 += p[2 * 4096];
+        p4 += p[3 * 4096];
+    }
+    unfold_pixels(l, m, nx, ny, p1, p2, p3, p4, gimg);
+}
+
 #define ADJ_T 16
 #define ADJ_CH 64
 #define ADJ_G 4   // point groups per tile: each takes every ADJ_G-th chunk of points
@@ -171,7 +330,7 @@ __global__ void __launch_bounds__(ADJ_BS) k_vis_adj(const float *gre, const floa
     __shared__ float H_r[ADJ_G][ADJ_CH], H_i[ADJ_G][ADJ_CH];
     __shared__ float sa_c[ADJ_G][ADJ_CH], sa_s[ADJ_G][ADJ_CH], sb_c[ADJ_G][ADJ_CH],
         sb_s[ADJ_G][ADJ_CH];
-    __shared__ float s_u[ADJ_G][ADJ_CH], s_v[ADJ_G][ADJ_CH];  // u dxy, v dxy
+    __shared__ double s_u[ADJ_G][ADJ_CH], s_v[ADJ_G][ADJ_CH];  // u dxy, v dxy
     const int g = threadIdx.x / (ADJ_T * ADJ_T), lt = threadIdx.x - g * (ADJ_T * ADJ_T);
     const int tx = lt % ADJ_T, ty = lt / ADJ_T;
     const int k0 = blockIdx.x * ADJ_T, j0 = blockIdx.y * ADJ_T;
@@ -209,17 +368,18 @@ __global__ void __launch_bounds__(ADJ_BS) k_vis_adj(const float *gre, const floa
         // one-pixel steps of its column and row phasors
         if (lt < ADJ_CH) {
             const int q = q0 + lt;
-            float hr = 0.f, hi = 0.f, s1 = 0.f, c1 = 1.f, s2 = 0.f, c2 = 1.f, su = 0.f, sv = 0.f;
+            float hr = 0.f, hi = 0.f, s1 = 0.f, c1 = 1.f, s2 = 0.f, c2 = 1.f;
+            double su = 0.0, sv = 0.0;
             if (q < K) {
                 double s, c;
                 sincospi(-2.0 * (cu * dra + cv * ddec), &s, &c);
                 // H = (gre - i gim) * (c + i s)
                 hr = (float)(gr * c + gi * s);
                 hi = (float)(gr * s - gi * c);
-                su = (float)(cu * dxy);
-                sv = (float)(cv * dxy);
-                sincospif(-2.f * su, &s1, &c1);
-                sincospif(-2.f * sv, &s2, &c2);
+                su = cu * dxy;
+                sv = cv * dxy;
+                phasor(-su, c1, s1);
+                phasor(-sv, c2, s2);
             }
             H_r[g][lt] = hr;
             H_i[g][lt] = hi;
@@ -238,8 +398,8 @@ __global__ void __launch_bounds__(ADJ_BS) k_vis_adj(const float *gre, const floa
             if (q < K) {
                 hr = H_r[g][lq];
                 hi = H_i[g][lq];
-                sincospif(-2.f * s_u[g][lq] * (float)(k0 + ll - nx / 2), &ai, &ar);
-                sincospif(-2.f * s_v[g][lq] * (float)(j0 + ll - ny / 2), &bi, &br);
+                phasor(-s_u[g][lq] * (double)(k0 + ll - nx / 2), ar, ai);
+                phasor(-s_v[g][lq] * (double)(j0 + ll - ny / 2), br, bi);
                 dac = sa_c[g][lq];
                 das = sa_s[g][lq];
                 dbc = sb_c[g][lq];
@@ -563,13 +723,60 @@ int vis_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const d
     return RT_OK;
 }
 
+// the context's scratch for a call on its stream: grown if need be, the call
+// ordered behind the last one that used it.  NULL in a capture (which can
+// neither allocate nor wait on an event from outside) and without memory.
+static void *adj_scratch(rt_ctx *ctx, size_t bytes) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
+        return nullptr;
+    if (!ctx->vis_ws_ev &&
+        hipEventCreateWithFlags(&ctx->vis_ws_ev, hipEventDisableTiming) != hipSuccess)
+        return nullptr;
+    if (ctx->vis_ws_cap < bytes) {
+        if (ctx->vis_ws_used && hipEventSynchronize(ctx->vis_ws_ev) != hipSuccess) return nullptr;
+        if (ctx->vis_ws) (void)hipFree(ctx->vis_ws);
+        ctx->vis_ws = nullptr;
+        ctx->vis_ws_cap = 0;
+        ctx->vis_ws_used = false;
+        if (hipMalloc(&ctx->vis_ws, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->vis_ws = nullptr;
+            return nullptr;
+        }
+        ctx->vis_ws_cap = bytes;
+    }
+    if (ctx->vis_ws_used && ctx->vis_ws_stream != ctx->stream &&
+        hipStreamWaitEvent(ctx->stream, ctx->vis_ws_ev, 0) != hipSuccess)
+        return nullptr;
+    return ctx->vis_ws;
+}
+
 int vis_adjoint_run(rt_ctx *ctx, const float *d_gre, const float *d_gim, int nx, int ny, double dxy,
                     const double *d_u, const double *d_v, int K, double dra, double ddec,
-                    float *d_g_img) {
+                    float *d_g_img, void *ws) {
     if (nx < 1 || ny < 1 || K < 0 || !(dxy > 0)) return set_err(ctx, RT_E_ARG, "vis adjoint: invalid sizes");
-    dim3 grid((nx + ADJ_T - 1) / ADJ_T, (ny + ADJ_T - 1) / ADJ_T);
-    hipLaunchKernelGGL(k_vis_adj, grid, dim3(ADJ_BS), 0, ctx->stream, d_gre, d_gim, nx, ny,
-                       d_u, d_v, K, dxy, dra, ddec, d_g_img);
+    const size_t need = vis_adjoint_workspace(ctx, nx, ny, K);
+    const bool own = need > 0 && !ws;
+    if (own) ws = adj_scratch(ctx, need);
+    if (need > 0 ? ws != nullptr : adj_tiled(nx, ny, K)) {
+        const AdjSplit a = adj_split(ctx, nx, ny, K);
+        hipLaunchKernelGGL(k_vis_adj_part, dim3(a.tx, a.ty, a.splits), dim3(256), 0, ctx->stream,
+                           d_gre, d_gim, nx, ny, d_u, d_v, K, dxy, dra, ddec, a.per,
+                           need > 0 ? (float *)ws : nullptr, d_g_img);
+        if (need > 0)
+            hipLaunchKernelGGL(k_vis_adj_sum, dim3(a.tx, a.ty, 16), dim3(256), 0, ctx->stream,
+                               (const float *)ws, a.splits, nx, ny, d_g_img);
+        if (own) {
+            HIPCHK(ctx, hipEventRecord(ctx->vis_ws_ev, ctx->stream));
+            ctx->vis_ws_stream = ctx->stream;
+            ctx->vis_ws_used = true;
+        }
+    } else {
+        dim3 grid((nx + ADJ_T - 1) / ADJ_T, (ny + ADJ_T - 1) / ADJ_T);
+        hipLaunchKernelGGL(k_vis_adj, grid, dim3(ADJ_BS), 0, ctx->stream, d_gre, d_gim, nx, ny,
+                           d_u, d_v, K, dxy, dra, ddec, d_g_img);
+    }
     HIPCHK(ctx, hipGetLastError());
     return RT_OK;
 }

@@ -743,3 +743,68 @@ def test_rays_split_over_lanes_match_oracle(nr, nt, pw, full, npix, tau_stop):
     # gradients within 5e-5 of the largest, as the adjoint tests above
     assert np.abs(glr.double().cpu().numpy() - rlr).max() <= 5e-5 * np.abs(rlr).max()
     assert np.abs(gT.double().cpu().numpy() - rT).max() <= 5e-5 * np.abs(rT).max()
+
+
+@pytest.mark.parametrize("ny,nx,K", [
+    (1, 1, 1), (1, 2, 5), (2, 1, 33), (3, 5, 31), (32, 64, 32), (33, 65, 127), (63, 64, 129),
+    (64, 63, 128), (65, 66, 1000), (130, 129, 3000), (66, 97, 66000), (200, 40, 20001),
+    (1024, 70, 300)])
+def test_vis_dft_and_adjoint_at_tile_edges(ny, nx, K):
+    """The folded matrix-core DFT and its transpose against the plain sums in FP64
+    at sizes around their tiles (32 rows, 32 columns, 32 and 128 points).  A
+    phasor is rotated at most 16 times between exact ones (6e-8 each), a product
+    and its sum round once each: within 2e-6 of sum |I| (sum |H|)."""
+    print("case: vis %dx%d, K=%d" % (ny, nx, K), flush=True)
+    rng = np.random.default_rng(ny * 1000 + nx)
+    img = torch.tensor(rng.standard_normal((ny, nx)), dtype=torch.float32, device="cuda")
+    dxy = 4e-8
+    u = torch.tensor(rng.uniform(-0.7, 0.7, K) / dxy, device="cuda")
+    v = torch.tensor(rng.uniform(-0.7, 0.7, K) / dxy, device="cuda")
+    dra, ddec = 3e-7, -5e-7
+    re, im = rt.vis_dft(img, dxy, u, v, dra, ddec)
+    g = torch.tensor(rng.standard_normal((2, K)), dtype=torch.float32, device="cuda")
+    adj = rt.vis_dft_adjoint(g[0], g[1], nx, ny, dxy, u, v, dra, ddec).double()
+    x = (torch.arange(nx, device="cuda", dtype=torch.float64) - nx // 2) * dxy
+    y = (torch.arange(ny, device="cuda", dtype=torch.float64) - ny // 2) * dxy
+    I = img.double()
+    ref = torch.zeros((ny, nx), device="cuda", dtype=torch.float64)
+    worst = 0.0
+    for i in range(0, K, 8192):
+        s = slice(i, i + 8192)
+        ax, ay = (-2 * np.pi * (u[s, None] * x), -2 * np.pi * (v[s, None] * y + u[s, None] * dra +
+                                                               v[s, None] * ddec))
+        ar, ai, br, bi = torch.cos(ax), torch.sin(ax), torch.cos(ay), torch.sin(ay)
+        rr, ri = ar @ I.T.contiguous(), ai @ I.T.contiguous()
+        vr, vi = (rr * br - ri * bi).sum(1), (rr * bi + ri * br).sum(1)
+        worst = max(worst, float((vr - re[s].double()).abs().max()),
+                    float((vi - im[s].double()).abs().max()))
+        hr, hi = g[0, s, None].double(), g[1, s, None].double()
+        ref += (br * hr + bi * hi).T.contiguous() @ ar + (br * hi - bi * hr).T.contiguous() @ ai
+    assert worst <= 2e-6 * float(I.abs().sum())
+    assert float((adj - ref).abs().max()) <= 2e-6 * float(g.double().abs().sum())
+
+
+@pytest.mark.parametrize("ny,nx,K", [(192, 201, 7000), (1300, 1601, 100)])
+def test_vis_adjoint_on_two_streams(ny, nx, K):
+    """The transposed DFT's scratch is the context's: calls on two streams (one or
+    several shares of the points) give what each gives alone, bit for bit."""
+    print("case: adjoint %dx%d, K=%d" % (ny, nx, K), flush=True)
+    rng = np.random.default_rng(K)
+    dxy = 4e-8
+    uv = torch.tensor(rng.uniform(-0.5, 0.5, (2, K)) / dxy, device="cuda")
+    gs = [torch.tensor(rng.standard_normal((2, K)), dtype=torch.float32, device="cuda")
+          for _ in range(6)]
+    alone = [rt.vis_dft_adjoint(g[0], g[1], nx, ny, dxy, uv[0], uv[1]) for g in gs]
+    x = (torch.arange(nx, device="cuda", dtype=torch.float64) - nx // 2) * dxy * 2 * np.pi
+    y = (torch.arange(ny, device="cuda", dtype=torch.float64) - ny // 2) * dxy * 2 * np.pi
+    ph = torch.exp(-1j * uv[1, :, None] * y).T.contiguous()
+    ref = ((ph * (gs[0][0] - 1j * gs[0][1])) @ torch.exp(-1j * uv[0, :, None] * x)).real
+    assert float((alone[0] - ref).abs().max()) <= 2e-6 * float(gs[0].double().abs().sum())
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    out = []
+    for i, g in enumerate(gs):
+        with torch.cuda.stream(streams[i % 2]):
+            out.append(rt.vis_dft_adjoint(g[0], g[1], nx, ny, dxy, uv[0], uv[1]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(alone, out))
