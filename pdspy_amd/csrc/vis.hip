@@ -454,9 +454,10 @@ __global__ void __launch_bounds__(ADJ_BS) k_vis_adj(const float *gre, const floa
 // F[b][a] = sum_jk I[j][k] w_nx((a - nx/2)(k - nx/2)) w_ny((b - ny/2)(j - ny/2)),
 // w_n(r) = exp(-2 pi i r / n), is the exact DFT at u_a = (a - nx/2) / (nx dxy),
 // v_b = (b - ny/2) / (ny dxy); it is computed as two passes of 1D transforms
-// (rows, then columns) with integer phase indices into one twiddle table per
-// axis, so every twiddle is exact to FP32 rounding.  Work:
-// [A: ny x nx float2][F: ny x nx float2][twiddles: nx + ny float2].
+// with integer phase indices into one twiddle table per axis, so every twiddle
+// is exact to FP32 rounding.  Work:
+// [A: ny x nx float2][F: ny x nx float2][twiddles: nx + ny float2] (of A one half
+// is used).
 #define GRID_BS 256
 #define GRID_MAXN 4096
 
@@ -469,78 +470,121 @@ __global__ void __launch_bounds__(GRID_BS) k_grid_twiddles(int nx, int ny, float
     tw[i] = make_float2((float)c, (float)s);
 }
 
-// n-periodic phase index of k * x0 and of the step k, both in [0, n)
-__device__ __forceinline__ void phase_index(int k, int x0, int n, int &r, int &dr) {
-    long long a = ((long long)k * (long long)x0) % n;
-    r = (int)(a < 0 ? a + n : a);
-    const int d = k % n;
-    dr = d < 0 ? d + n : d;
-}
+// The transform on the grid, folded in both image and grid axes about their node 0
+// (index n/2): with the planes EE, OE, EO, OO over k = 0..nx/2, l = 0..ny/2 (E: sum,
+// O: difference of the pixels at +-; first letter rows), angles a k of 2 pi / nx and
+// b l of 2 pi / ny,
+//   rows:    X0 = sum_l EE cos bl, X1 = sum_l OE sin bl, X2 = sum_l EO cos bl,
+//            X3 = sum_l OO sin bl                                 (FIRST)
+//   columns: F1 = sum_k X0 cos ak, F2 = sum_k X3 sin ak, F3 = sum_k X2 sin ak,
+//            F4 = sum_k X1 cos ak
+// and the node (sgn_a a, sgn_b b) is (F1 - sgn_a sgn_b F2) - i (sgn_a F3 + sgn_b F4):
+// a quarter of the plain sums' multiplications, on v_mfma_f32_16x16x4f32.  A
+// workgroup makes 16 x (16 * GRID_NB) entries of the four planes, its four waves
+// taking every fourth group of four terms; a lane's value operand is read from
+// L2 where the sum is (64-byte runs), its cosines and sines from the twiddle
+// table in LDS.  1024 x 1024: 32 + 29 us (572 with the
+// plain sums), 7 us each at the FP32 matrix peak; the operands' address and
+// fold instructions pace it.  Measured without effect: rotated instead of looked-up
+// phases, the loads of 4 or 8 groups ahead, 16 x 64 entries; 16 x 16 entries: 34 us.
+#define GRID_NB 2
 
-// rows: A[j][a] = sum_k I[j'][k] w_nx((a - nx/2)(k - nx/2)); block = 256 a's of
-// row j, which reads image row j' = j, or j' = ny - 1 - j when flip is set (the
-// transform of image[::-1])
-__global__ void __launch_bounds__(GRID_BS) k_grid_rows(const float *img, const float2 *twx,
-                                                       int nx, int ny, int flip, float2 *A) {
-    __shared__ float row[GRID_MAXN];
-    __shared__ float2 tw[GRID_MAXN];
-    const int j = blockIdx.y;
-    const int js = flip ? ny - 1 - j : j;
-    for (int i = threadIdx.x; i < nx; i += GRID_BS) {
-        row[i] = img[(size_t)js * nx + i];
-        tw[i] = twx[i];
-    }
+template <bool FIRST>
+__global__ void __launch_bounds__(GRID_BS) k_grid_dft(const float *src, const float2 *twg, int nx,
+                                                      int ny, int flip, float *X, float2 *F) {
+    __shared__ __align__(16) float sm[4 * 16 * GRID_NB * 64];  // twiddles, then the waves' sums
+    static_assert(sizeof(sm) >= GRID_MAXN * sizeof(float2), "the table fits");
+    float2 *tw = (float2 *)sm;
+    const int n = FIRST ? ny : nx;  // the transformed axis
+    for (int i = threadIdx.x; i < n; i += GRID_BS) tw[i] = twg[i];
     __syncthreads();
-    const int a = blockIdx.x * GRID_BS + threadIdx.x;
-    if (a >= nx) return;
-    int r, dr;
-    phase_index(a - nx / 2, -(nx / 2), nx, r, dr);
-    float sr = 0.f, si = 0.f;
-    for (int k = 0; k < nx; ++k) {
-        const float p = row[k];
-        const float2 w = tw[r];
-        sr = fmaf(p, w.x, sr);
-        si = fmaf(p, w.y, si);
-        r += dr;
-        if (r >= nx) r -= nx;
-    }
-    A[(size_t)j * nx + a] = make_float2(sr, si);
-}
-
-// columns: F[b][a] = sum_j A[j][a] w_ny((b - ny/2)(j - ny/2)); block = 256 a's x
-// KB rows b, so each A element read serves KB outputs (KB = 1 for small grids,
-// where the launch would otherwise hold fewer blocks than the GPU has CUs)
-template <int GRID_KB>
-__global__ void __launch_bounds__(GRID_BS) k_grid_cols(const float2 *A, const float2 *twy, int nx,
-                                                       int ny, float2 *F) {
-    __shared__ float2 tw[GRID_MAXN];
-    for (int i = threadIdx.x; i < ny; i += GRID_BS) tw[i] = twy[i];
-    __syncthreads();
-    const int a = blockIdx.x * GRID_BS + threadIdx.x;
-    const int b0 = blockIdx.y * GRID_KB;
-    if (a >= nx) return;
-    int r[GRID_KB], dr[GRID_KB];
-    float fr[GRID_KB], fi[GRID_KB];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, kh = lane >> 4;
+    const int cx = nx / 2, cy = ny / 2, hx = cx + 1, hy = cy + 1;  // E entries
+    const int ox = (nx - 1) / 2, oy = (ny - 1) / 2;                // O entries (1, 2, ..)
+    // X0 [hx][hy], X1 [hx][oy], X2 [ox][hy], X3 [ox][oy]: nx ny floats
+    float *X1 = X + (size_t)hx * hy, *X2 = X1 + (size_t)hx * oy, *X3 = X2 + (size_t)ox * hy;
+    const int v0 = blockIdx.x * 16, f0 = blockIdx.y * (16 * GRID_NB);
+    const int vi = v0 + i16, h = FIRST ? hy : hx;
+    int r[GRID_NB], dr[GRID_NB];
+    vf4 acc[GRID_NB][4];
 #pragma unroll
-    for (int t = 0; t < GRID_KB; ++t) {
-        phase_index(b0 + t - ny / 2, -(ny / 2), ny, r[t], dr[t]);
-        fr[t] = 0.f;
-        fi[t] = 0.f;
-    }
-    for (int j = 0; j < ny; ++j) {
-        const float2 x = A[(size_t)j * nx + a];
+    for (int b = 0; b < GRID_NB; ++b) {
+        const int f = f0 + 16 * b + i16;
+        r[b] = (f * (4 * w + kh)) % n;
+        dr[b] = (16 * f) % n;
 #pragma unroll
-        for (int t = 0; t < GRID_KB; ++t) {
-            const float2 w = tw[r[t]];
-            fr[t] = fmaf(x.x, w.x, fmaf(-x.y, w.y, fr[t]));
-            fi[t] = fmaf(x.x, w.y, fmaf(x.y, w.x, fi[t]));
-            r[t] += dr[t];
-            if (r[t] >= ny) r[t] -= ny;
+        for (int p = 0; p < 4; ++p) acc[b][p] = vf4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll 4
+    for (int t0 = 4 * w; t0 < h; t0 += 16) {
+        const int t = t0 + kh;
+        float x[4] = {0.f, 0.f, 0.f, 0.f};
+        if (FIRST) {
+            const int jp = cy + t, jm = cy - t, kp = cx + vi, km = cx - vi;
+            const bool rp = jp < ny, rm = t > 0 && jm >= 0, cp = kp < nx, cm = vi > 0 && km >= 0;
+            const float *ip = src + (size_t)(flip ? ny - 1 - jp : jp) * nx;
+            const float *im = src + (size_t)(flip ? ny - 1 - jm : jm) * nx;
+            const float pp = rp && cp ? ip[kp] : 0.f, pm = rp && cm ? ip[km] : 0.f;
+            const float mp = rm && cp ? im[kp] : 0.f, mm = rm && cm ? im[km] : 0.f;
+            const float e = pp + pm, d = pp - pm, em = mp + mm, dm = mp - mm;
+            x[0] = e + em;
+            x[1] = e - em;
+            x[2] = d + dm;
+            x[3] = d - dm;
+        } else {
+            const bool ek = t < hx, ok = t > 0 && t <= ox, eb = vi < hy, ob = vi > 0 && vi <= oy;
+            if (ek && eb) x[0] = X[(size_t)t * hy + vi];
+            if (ek && ob) x[1] = X1[(size_t)t * oy + vi - 1];
+            if (ok && eb) x[2] = X2[(size_t)(t - 1) * hy + vi];
+            if (ok && ob) x[3] = X3[(size_t)(t - 1) * oy + vi - 1];
+        }
+#pragma unroll
+        for (int b = 0; b < GRID_NB; ++b) {
+            const float c = tw[r[b]].x, s = -tw[r[b]].y;
+            acc[b][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[0], c, acc[b][0], 0, 0, 0);
+            acc[b][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[1], FIRST ? s : c, acc[b][1], 0, 0, 0);
+            acc[b][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[2], FIRST ? c : s, acc[b][2], 0, 0, 0);
+            acc[b][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[3], s, acc[b][3], 0, 0, 0);
+            r[b] += dr[b];
+            if (r[b] >= n) r[b] -= n;
         }
     }
+    // the four waves' sums, in order; wave w finishes elements e = 2w, 2w + 1, .. of a lane
+    __syncthreads();
 #pragma unroll
-    for (int t = 0; t < GRID_KB; ++t)
-        if (b0 + t < ny) F[(size_t)(b0 + t) * nx + a] = make_float2(fr[t], fi[t]);
+    for (int b = 0; b < GRID_NB; ++b)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sm[((w * GRID_NB + b) * 16 + p * 4 + e) * 64 + lane] = acc[b][p][e];
+    __syncthreads();
+    for (int z = w; z < 4 * GRID_NB; z += 4) {
+        const int b = z >> 2, e = z & 3;
+        const int v = v0 + 4 * kh + e, f = f0 + 16 * b + i16;  // row, column of the products
+        float o[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const float *q = sm + (b * 16 + p * 4 + e) * 64 + lane;
+            constexpr int W = GRID_NB * 16 * 64;
+            o[p] = (q[0] + q[W]) + (q[2 * W] + q[3 * W]);
+        }
+        if (FIRST) {
+            const bool ek = v < hx, ok = v > 0 && v <= ox, eb = f < hy, ob = f > 0 && f <= oy;
+            if (ek && eb) X[(size_t)v * hy + f] = o[0];
+            if (ek && ob) X1[(size_t)v * oy + f - 1] = o[1];
+            if (ok && eb) X2[(size_t)(v - 1) * hy + f] = o[2];
+            if (ok && ob) X3[(size_t)(v - 1) * oy + f - 1] = o[3];
+        } else if (v < hy && f < hx) {
+            // o: F1, F4, F3, F2
+            const float pr = o[0] - o[3], mr = o[0] + o[3], ps = o[1] + o[2], ds = o[2] - o[1];
+            const int bp = cy + v, bm = cy - v, ap = cx + f, am = cx - f;
+            if (bp < ny && ap < nx) F[(size_t)bp * nx + ap] = make_float2(pr, -ps);
+            if (bp < ny && f > 0) F[(size_t)bp * nx + am] = make_float2(mr, ds);
+            if (v > 0 && ap < nx) F[(size_t)bm * nx + ap] = make_float2(mr, -ds);
+            if (v > 0 && f > 0) F[(size_t)bm * nx + am] = make_float2(pr, ps);
+        }
+    }
 }
 
 // one (u,v) point per lane: bilinear interpolation between the four grid nodes
@@ -642,21 +686,15 @@ int vis_grid_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, co
         return set_err(ctx, RT_E_ARG, "vis grid: NULL image, (u,v) or output");
     float2 *ws = (float2 *)d_work;
     if (!ws) HIPCHK(ctx, hipMallocAsync((void **)&ws, vis_grid_workspace(nx, ny), ctx->stream));
-    float2 *A = ws, *F = ws + (size_t)nx * ny, *tw = ws + 2 * (size_t)nx * ny;
+    float *A = (float *)ws;  // the folded rows' transforms
+    float2 *F = ws + (size_t)nx * ny, *tw = ws + 2 * (size_t)nx * ny;
     hipLaunchKernelGGL(k_grid_twiddles, dim3((nx + ny + GRID_BS - 1) / GRID_BS), dim3(GRID_BS), 0,
                        ctx->stream, nx, ny, tw);
-    hipLaunchKernelGGL(k_grid_rows, dim3((nx + GRID_BS - 1) / GRID_BS, ny), dim3(GRID_BS), 0,
-                       ctx->stream, d_img, tw, nx, ny, conv == 1 ? 1 : 0, A);
-    const int bx = (nx + GRID_BS - 1) / GRID_BS;
-    if (bx * ((ny + 7) / 8) >= 512)
-        hipLaunchKernelGGL(k_grid_cols<8>, dim3(bx, (ny + 7) / 8), dim3(GRID_BS), 0, ctx->stream, A,
-                           tw + nx, nx, ny, F);
-    else if (bx * ((ny + 3) / 4) >= 512)
-        hipLaunchKernelGGL(k_grid_cols<4>, dim3(bx, (ny + 3) / 4), dim3(GRID_BS), 0, ctx->stream, A,
-                           tw + nx, nx, ny, F);
-    else
-        hipLaunchKernelGGL(k_grid_cols<1>, dim3(bx, ny), dim3(GRID_BS), 0, ctx->stream, A, tw + nx,
-                           nx, ny, F);
+    const int hx = nx / 2 + 1, hy = ny / 2 + 1, FW = 16 * GRID_NB;
+    hipLaunchKernelGGL(k_grid_dft<true>, dim3((hx + 15) / 16, (hy + FW - 1) / FW), dim3(GRID_BS), 0,
+                       ctx->stream, d_img, tw + nx, nx, ny, conv == 1 ? 1 : 0, A, F);
+    hipLaunchKernelGGL(k_grid_dft<false>, dim3((hy + 15) / 16, (hx + FW - 1) / FW), dim3(GRID_BS), 0,
+                       ctx->stream, d_img, tw, nx, ny, 0, A, F);
     hipLaunchKernelGGL(k_grid_sample, dim3((K + GRID_BS - 1) / GRID_BS), dim3(GRID_BS), 0,
                        ctx->stream, F, nx, ny, dxy, d_u, d_v, K, conv == 1 ? -1.0 : 1.0, dra, ddec,
                        d_re, d_im);

@@ -808,3 +808,27 @@ def test_vis_adjoint_on_two_streams(ny, nx, K):
             out.append(rt.vis_dft_adjoint(g[0], g[1], nx, ny, dxy, uv[0], uv[1]))
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(alone, out))
+
+
+@pytest.mark.parametrize("ny,nx", [(2, 2), (2, 3), (3, 2), (5, 4), (7, 64), (31, 16), (30, 33),
+                                   (66, 63), (129, 128), (512, 27), (3, 4096), (300, 1025)])
+@pytest.mark.parametrize("conv", ["imtovis", "galario"])
+def test_grid_transform_at_tile_edges(ny, nx, conv):
+    """The folded matrix-core transform against numpy's FFT at the grid's nodes
+    (every node but the last of each axis), at the smallest grids, odd and even ones
+    and around its tiles of 16 x 32 nodes and 16 terms.  The foldings, a twiddle, a
+    product and their sums round about ten times: within 1e-6 of sum |I|."""
+    print("case: grid %dx%d %s" % (ny, nx, conv), flush=True)
+    rng = np.random.default_rng(ny * 5000 + nx)
+    img = rng.standard_normal((ny, nx)).astype(np.float32)
+    d = 4e-8
+    sg = -1.0 if conv == "galario" else 1.0
+    b, a = np.meshgrid(np.arange(ny - 1), np.arange(nx - 1), indexing="ij")
+    # half a 1e-9 step inside the node's cell
+    u = sg * (a.ravel() - nx // 2 + 5e-10) / (nx * d)
+    v = sg * (b.ravel() - ny // 2 + 5e-10) / (ny * d)
+    re, im = rt.vis_grid(torch.tensor(img, device="cuda"), d, u, v, conv=conv)
+    src = img[::-1] if conv == "galario" else img
+    F = np.fft.fftshift(np.fft.fft2(np.fft.ifftshift(src.astype(float))))[:-1, :-1].ravel()
+    got = re.double().cpu().numpy() + 1j * im.double().cpu().numpy()
+    assert np.abs(got - F).max() <= 1e-6 * np.abs(img).sum()
