@@ -326,6 +326,11 @@ int rt_vis_grid(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy,
                 const double *d_u, const double *d_v, int K, double dra, double ddec,
                 float *d_re, float *d_im, void *d_work);
 size_t rt_vis_grid_workspace(int nx, int ny);
+/* Whether a point lacks one of its four grid nodes: sets *d_outside (device, zeroed
+ * by the caller) to 1 if any does.  conv: 0 the points of rt_vis_grid, 1 those
+ * of rt_interpolate_galario (at (-u, -v)). */
+int rt_vis_grid_outside(rt_ctx *ctx, int nx, int ny, double dxy, const double *d_u,
+                        const double *d_v, int K, int conv, int *d_outside);
 /* rt_vis_grid without any allocation (no counterpart in the reference): for
  * callers that cannot allocate device memory -- code under stream capture,
  * tight sampler loops, harnesses that forbid hipMalloc.  Its workspace is a

@@ -652,6 +652,12 @@ int rt_vis_dft_adjoint(rt_ctx *ctx, const float *d_gre, const float *d_gim, int 
     return vis_adjoint_run(ctx, d_gre, d_gim, nx, ny, dxy, d_u, d_v, K, dra, ddec, d_g_img, nullptr);
 }
 
+int rt_vis_grid_outside(rt_ctx *ctx, int nx, int ny, double dxy, const double *d_u,
+                        const double *d_v, int K, int conv, int *d_outside) {
+    if (!ctx) return RT_E_ARG;
+    return vis_grid_outside_run(ctx, nx, ny, dxy, d_u, d_v, K, conv, d_outside);
+}
+
 int rt_vis_grid(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const double *d_u,
                 const double *d_v, int K, double dra, double ddec, float *d_re, float *d_im,
                 void *d_work) {

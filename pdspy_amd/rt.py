@@ -502,11 +502,17 @@ def vis_grid(img, dxy, u, v, dra=0.0, ddec=0.0, device=0, work=None, conv="imtov
         # the four nodes around each point must lie on the grid (galario's
         # sampleImage checks the uv coverage against the image the same way);
         # the galario convention interpolates at (-u, -v)
-        sg = -1.0 if conv == "galario" else 1.0
-        fa = sg * u * (nx * dxy) + nx // 2
-        fb = sg * v * (ny * dxy) + ny // 2
-        ok = ((fa >= 0) & (fa < nx - 1) & (fb >= 0) & (fb < ny - 1)).all()
-        if not bool(ok):
+        cu, cv = u, v
+        if u.shape != v.shape:
+            cu, cv = (t.contiguous() for t in torch.broadcast_tensors(u, v))
+            if v.numel() < K:
+                raise ValueError("vis_grid: u and v differ in size (%d, %d)" % (K, v.numel()))
+        outside = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ctx.check(ctx.L.rt_vis_grid_outside(ctx.h, nx, ny, float(dxy), C.c_void_p(cu.data_ptr()),
+                                            C.c_void_p(cv.data_ptr()), cu.numel(),
+                                            1 if conv == "galario" else 0,
+                                            C.c_void_p(outside.data_ptr())))
+        if int(outside):
             raise ValueError("vis_grid: (u,v) beyond the image's uv grid (|u| < (nx/2 - 1) / "
                              "(nx dxy)); use a finer pixel size or vis_dft")
     re = torch.empty(K, dtype=torch.float32, device="cuda")

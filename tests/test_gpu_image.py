@@ -832,3 +832,36 @@ def test_grid_transform_at_tile_edges(ny, nx, conv):
     F = np.fft.fftshift(np.fft.fft2(np.fft.ifftshift(src.astype(float))))[:-1, :-1].ravel()
     got = re.double().cpu().numpy() + 1j * im.double().cpu().numpy()
     assert np.abs(got - F).max() <= 1e-6 * np.abs(img).sum()
+
+
+@pytest.mark.parametrize("conv", ["imtovis", "galario"])
+@pytest.mark.parametrize("K", [1, 64, 257, 300001])
+def test_grid_range_check_is_the_torch_expression(conv, K):
+    """The one-pass range check refuses what the elementwise expression in FP64
+    refuses: one point on or next to an edge of the grid, NaN, at the first, a middle
+    and the last place; a size mismatch is refused."""
+    print("case: range %s K=%d" % (conv, K), flush=True)
+    rng = np.random.default_rng(K)
+    nx, ny, d = 10, 7, 3.3e-8
+    sg = -1.0 if conv == "galario" else 1.0
+    img = torch.rand((ny, nx), device="cuda")
+    base = rng.uniform(-0.2, 0.2, (2, K)) / d
+    for n, axis in ((nx, 0), (ny, 1)):
+        for edge in (-(n // 2) / (n * d), (n - 1 - n // 2) / (n * d), np.nan):
+            for x in (np.nextafter(edge, -np.inf), edge, np.nextafter(edge, np.inf)):
+                for at in {0, K // 2, K - 1}:
+                    uv = base.copy()
+                    uv[axis, at] = sg * x
+                    f = [sg * uv[i] * (m * d) + m // 2 for i, m in ((0, nx), (1, ny))]
+                    ok = all(bool(((g >= 0) & (g < m - 1)).all()) for g, m in zip(f, (nx, ny)))
+                    if ok:
+                        re, im = rt.vis_grid(img, d, uv[0], uv[1], conv=conv)
+                        assert bool(torch.isfinite(re).all() and torch.isfinite(im).all())
+                    else:
+                        with pytest.raises(ValueError):
+                            rt.vis_grid(img, d, uv[0], uv[1], conv=conv)
+    if K > 1:
+        with pytest.raises(RuntimeError):
+            rt.vis_grid(img, d, base[0], np.zeros(K + 1), conv=conv)
+        with pytest.raises(ValueError):
+            rt.vis_grid(img, d, base[0], base[1, :1], conv=conv)
