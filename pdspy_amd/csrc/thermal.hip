@@ -930,44 +930,176 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                         unsigned long long add[MG];
 #pragma unroll
                         for (int q = 0; q < MG; ++q) add[q] = 0;
-                        float lowd = walk_bound(w, x, y, z);
                         uint32_t n = 0, nsc = 0;
-                        for (; n < nmax; ++n) {
-                            const float cext = cabs + csca;
-                            const float sseg = tl / cext;
-                            if (!(sseg < lowd)) break;
-                            const float nx = fmaf(sseg, dx, x), ny = fmaf(sseg, dy, y),
-                                        nz = fmaf(sseg, dz, z);
-                            if (P.mrw && w_nc + n + 1u >= (uint32_t)P.mrw_count) {
-                                if (aR < 0.f) {
-                                    float a = 0.f;
-                                    for (int s = 0; s < S; ++s) {
-                                        const float rs = pickn<MS>(rho, s);
-                                        if (rs > 0.f)
-                                            a = fmaf(rs, trow(P.kross + (size_t)s * P.ntemp, P.ntemp,
-                                                              pickn<MG>(xr, pickn<MS>(grpr, s))), a);
+                        if (!P.hg) {
+                            // isotropic scattering: an interaction needs of those before
+                            // it only the last absorption (its opacities) and the position.
+                            // The absorptions one after the other: which lane's is the
+                            // next after lane m's, all lanes at once
+                            float eext[MG];
+#pragma unroll
+                            for (int q = 0; q < MG; ++q) eext[q] = eabs[q] + esca[q];
+                            int src = -1;  // the last absorption before this lane's (and its group)
+                            uint64_t absm = 0, grpm = 0, left = ~0ull;
+                            {
+                                float cx = cabs + csca, cs = csca, ca = cabs, z0 = c0;
+                                for (;;) {
+                                    const uint64_t ab = __ballot(!(u[0] * cx < cs)) & left;
+                                    if (!ab) break;
+                                    const int b = (int)uniform32(
+                                        (unsigned)(__ffsll((unsigned long long)ab) - 1));
+                                    int q = 0;
+                                    if (MG > 1) {
+                                        q = (S < 2 || lanef(u[1], b) * ca <= z0) ? grpr[0]
+                                                                                : grpr[MS > 1 ? 1 : 0];
+                                        q = (int)uniform32((unsigned)q);
                                     }
-                                    aR = a;
+#pragma unroll
+                                    for (int t = 0; t < MG; ++t)
+                                        if (q == t) {
+                                            cx = lanef(eext[t], b);
+                                            cs = lanef(esca[t], b);
+                                            ca = lanef(eabs[t], b);
+                                            z0 = lanef(e0[t], b);
+                                        }
+                                    absm |= 1ull << b;
+                                    if (MG > 1 && q) grpm |= 1ull << b;
+                                    left = (~0ull << b) << 1;
+                                    src = lane > b ? b * MG + q : src;
                                 }
-                                const float dmin = walls_dist(w, nx, ny, nz);
-                                if (aR * dmin >= P.mrw_tau && dmin - P.mrw_gamma / aR > 0.f) break;
                             }
-                            const float wf = inv * sseg;
+                            // this lane's segment: opacities, optical depth, direction
+                            float lx = cabs + csca, lk[MG];
+#pragma unroll
+                            for (int q = 0; q < MG; ++q) lk[q] = ck[q];
+#pragma unroll
+                            for (int t = 0; t < MG; ++t) {
+                                const int sl = max(src, 0) / MG;
+                                const bool mine = src >= 0 && (MG == 1 || src % MG == t);
+                                const float a = __shfl(eext[t], sl);
+                                lx = mine ? a : lx;
+#pragma unroll
+                                for (int q = 0; q < MG; ++q) {
+                                    const float kq = __shfl(ek[t][q], sl);
+                                    lk[q] = mine ? kq : lk[q];
+                                }
+                            }
+                            float lt = __shfl_up(etau, 1), ldx = __shfl_up(ex, 1),
+                                  ldy = __shfl_up(ey, 1), ldz = __shfl_up(ez, 1);
+                            lt = lane ? lt : tl;
+                            ldx = lane ? ldx : dx;
+                            ldy = lane ? ldy : dy;
+                            ldz = lane ? ldz : dz;
+                            const float seg = lt / lx;
+                            if (P.mrw && aR < 0.f && w_nc + nmax >= (uint32_t)P.mrw_count) {
+                                float a = 0.f;
+                                for (int s = 0; s < S; ++s) {
+                                    const float rs = pickn<MS>(rho, s);
+                                    if (rs > 0.f)
+                                        a = fmaf(rs, trow(P.kross + (size_t)s * P.ntemp, P.ntemp,
+                                                          pickn<MG>(xr, pickn<MS>(grpr, s))), a);
+                                }
+                                aR = a;
+                            }
+                            // positions, sixteen segments at a time, then their bounds on
+                            // all lanes at once: the walk ends at the first segment that
+                            // may reach a wall (or where a larger step begins)
+                            float px = x, py = y, pz = z;  // where this lane's segment starts
+                            uint64_t stop = 0;
+                            for (int j0 = 0; j0 < 64 && !stop; j0 += 16) {
+#pragma unroll
+                                for (int i = 0; i < 16; ++i) {
+                                    const float s = lanef(seg, j0 + i);
+                                    x = fmaf(s, lanef(ldx, j0 + i), x);
+                                    y = fmaf(s, lanef(ldy, j0 + i), y);
+                                    z = fmaf(s, lanef(ldz, j0 + i), z);
+                                    const bool later = lane > j0 + i;
+                                    px = later ? x : px;
+                                    py = later ? y : py;
+                                    pz = later ? z : pz;
+                                }
+                                bool bad = (uint32_t)lane >= nmax || !(seg < walk_bound(w, px, py, pz));
+                                if (P.mrw && w_nc + (uint32_t)lane + 1u >= (uint32_t)P.mrw_count) {
+                                    const float dmin =
+                                        walls_dist(w, fmaf(seg, ldx, px), fmaf(seg, ldy, py),
+                                                   fmaf(seg, ldz, pz));
+                                    bad |= aR * dmin >= P.mrw_tau && dmin - P.mrw_gamma / aR > 0.f;
+                                }
+                                stop = __ballot(bad && lane < j0 + 16);
+                            }
+                            n = stop ? uniform32((unsigned)(__ffsll((unsigned long long)stop) - 1)) : 64u;
 #pragma unroll
                             for (int q = 0; q < MG; ++q)
-                                if (MG == 1 || q < G) add[q] += (unsigned long long)rintf(ck[q] * wf);
-                            lowd -= sseg;
-                            x = nx;
-                            y = ny;
-                            z = nz;
-                            const float v0 = lanef(u[0], (int)n);
-                            const bool scat = v0 * cext < csca;
-                            dx = scat && P.hg ? dx : lanef(ex, (int)n);
-                            dy = scat && P.hg ? dy : lanef(ey, (int)n);
-                            dz = scat && P.hg ? dz : lanef(ez, (int)n);
-                            if (scat) {
-                                ++nsc;
-                                if (P.hg) {
+                                if (MG == 1 || q < G) {
+                                    const float wf = inv * seg;
+                                    unsigned long long a =
+                                        (uint32_t)lane < n ? (unsigned long long)rintf(lk[q] * wf) : 0ull;
+#pragma unroll
+                                    for (int h = 1; h < 64; h <<= 1) a += __shfl_xor(a, h);
+                                    add[q] = a;
+                                }
+                            if (n < 64u) {
+                                x = lanef(px, (int)n);
+                                y = lanef(py, (int)n);
+                                z = lanef(pz, (int)n);
+                                absm &= (1ull << n) - 1ull;
+                            }
+                            nsc = n - (uint32_t)__popcll(absm);
+                            if (n) {
+                                dx = lanef(ex, (int)n - 1);
+                                dy = lanef(ey, (int)n - 1);
+                                dz = lanef(ez, (int)n - 1);
+                                tl = lanef(etau, (int)n - 1);
+                            }
+                            if (absm) {
+                                const int b = (int)uniform32(63u - (unsigned)__clzll((long long)absm));
+                                const int q = MG > 1 ? (int)(grpm >> b & 1ull) : 0;
+#pragma unroll
+                                for (int t = 0; t < MG; ++t)
+                                    if (q == t) f = __builtin_amdgcn_readlane(ec[t], b);
+                            }
+                        } else {
+                            // forward scattering turns the direction: one at a time
+                            float lowd = walk_bound(w, x, y, z);
+                            for (; n < nmax; ++n) {
+                                const float cext = cabs + csca;
+                                const float sseg = tl / cext;
+                                // the bound shrinks by the path walked, the packet by far less
+                                if (!(sseg < lowd)) {
+                                    lowd = walk_bound(w, x, y, z);
+                                    if (!(sseg < lowd)) break;
+                                }
+                                const float nx = fmaf(sseg, dx, x), ny = fmaf(sseg, dy, y),
+                                            nz = fmaf(sseg, dz, z);
+                                if (P.mrw && w_nc + n + 1u >= (uint32_t)P.mrw_count) {
+                                    if (aR < 0.f) {
+                                        float a = 0.f;
+                                        for (int s = 0; s < S; ++s) {
+                                            const float rs = pickn<MS>(rho, s);
+                                            if (rs > 0.f)
+                                                a = fmaf(rs, trow(P.kross + (size_t)s * P.ntemp, P.ntemp,
+                                                                  pickn<MG>(xr, pickn<MS>(grpr, s))), a);
+                                        }
+                                        aR = a;
+                                    }
+                                    const float dmin = walls_dist(w, nx, ny, nz);
+                                    if (aR * dmin >= P.mrw_tau && dmin - P.mrw_gamma / aR > 0.f) break;
+                                }
+                                const float wf = inv * sseg;
+    #pragma unroll
+                                for (int q = 0; q < MG; ++q)
+                                    if (MG == 1 || q < G) add[q] += (unsigned long long)rintf(ck[q] * wf);
+                                lowd -= sseg;
+                                x = nx;
+                                y = ny;
+                                z = nz;
+                                const float v0 = lanef(u[0], (int)n);
+                                const bool scat = v0 * cext < csca;
+                                dx = scat ? dx : lanef(ex, (int)n);
+                                dy = scat ? dy : lanef(ey, (int)n);
+                                dz = scat ? dz : lanef(ez, (int)n);
+                                if (scat) {
+                                    ++nsc;
                                     const float us = lanef(u[1], (int)n) * csca;
                                     float a = 0.f;
                                     int sp = S - 1;
@@ -980,26 +1112,26 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                                     }
                                     hg_dir(lanef(u[4], (int)n), lanef(u[5], (int)n),
                                            s_g[sp * NL + f], dx, dy, dz);
+                                } else {
+                                    // the absorbing species' group: with two groups
+                                    // there are at most two species here (MS <= 2)
+                                    int q = 0;
+                                    if (MG > 1) q = (S < 2 || lanef(u[1], (int)n) * cabs <= c0) ? grpr[0]
+                                                                                                 : grpr[MS > 1 ? 1 : 0];
+                                    q = (int)uniform32((unsigned)q);
+    #pragma unroll
+                                    for (int t = 0; t < MG; ++t)
+                                        if (q == t) {
+                                            f = __builtin_amdgcn_readlane(ec[t], (int)n);
+                                            cabs = lanef(eabs[t], (int)n);
+                                            csca = lanef(esca[t], (int)n);
+                                            c0 = lanef(e0[t], (int)n);
+    #pragma unroll
+                                            for (int h = 0; h < MG; ++h) ck[h] = lanef(ek[t][h], (int)n);
+                                        }
                                 }
-                            } else {
-                                // the absorbing species' group: with two groups
-                                // there are at most two species here (MS <= 2)
-                                int q = 0;
-                                if (MG > 1) q = (S < 2 || lanef(u[1], (int)n) * cabs <= c0) ? grpr[0]
-                                                                                             : grpr[MS > 1 ? 1 : 0];
-                                q = (int)uniform32((unsigned)q);
-#pragma unroll
-                                for (int t = 0; t < MG; ++t)
-                                    if (q == t) {
-                                        f = __builtin_amdgcn_readlane(ec[t], (int)n);
-                                        cabs = lanef(eabs[t], (int)n);
-                                        csca = lanef(esca[t], (int)n);
-                                        c0 = lanef(e0[t], (int)n);
-#pragma unroll
-                                        for (int h = 0; h < MG; ++h) ck[h] = lanef(ek[t][h], (int)n);
-                                    }
+                                tl = lanef(etau, (int)n);
                             }
-                            tl = lanef(etau, (int)n);
                         }
                         if (lane == L) {
                             p.x = x;
