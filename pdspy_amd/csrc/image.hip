@@ -76,8 +76,8 @@ __device__ __forceinline__ void count_crossings(unsigned long long *dst, uint32_
 // by a binary search over the two sequences' counters) and combine their
 // (optical depth, intensity) afterwards.  An image of 256 x 256 rays is 1024
 // waves, one per SIMD, and a march of one ray per lane left it waiting on the
-// longest chains (~700 crossings of ~6000 clocks: 1.47 ms); with 8 lanes per ray
-// and ~150 instructions per crossing see k_image.
+// longest chains (~700 crossings of ~6000 clocks: 1.47 ms); with 8 lanes per ray:
+// 0.164 ms, paced by the FP64 instructions of the merge.
 struct RayGeo {
     double b2, z0, dz, S;
     int nin, w;    // spheres met inwards (as many outwards); the innermost one

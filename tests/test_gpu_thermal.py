@@ -222,3 +222,30 @@ def test_walk_inside_a_thick_cell_counts_every_interaction(max_events, slice_eve
     b = rt.Batch([other, dm])
     b.thermal([2, 2], [5, 5], max_events=max_events, slice_events=slice_events)
     assert np.array_equal(other.temperature(), T) and np.array_equal(dm.temperature(), T)
+
+
+@pytest.mark.parametrize("model", ["one group", "two groups", "modified walk", "forward"])
+def test_walks_leave_a_run_as_it_is(model):
+    """16000 packets in waves of 62 (64-lane blocks, one per CU: a wave looks for walks
+    only near the end) and of four and fewer (the default): the interactions
+    replayed in walks are the loop's own, so the temperatures and the counts are
+    equal bit for bit -- isotropic with one and two absorption groups, with the
+    modified random walk, and with forward scattering."""
+    print("case: walks, %s" % model, flush=True)
+    if model == "forward":
+        arr = oracle_arrays(configs.spiral_3d(nr=12, nt=8, nphi=6))
+    else:
+        arr = oracle_arrays(configs.disk_envelope(nr=24, nt=16))
+    if model == "two groups":
+        lam = arr["lam_um"]
+        arr["kabs"] = np.array(arr["kabs"], dtype=float)
+        arr["kabs"][0] = np.where(lam > 1.0, 1e3 * lam ** -0.6, 1e3)
+    dm = rt.DeviceModel(arr)
+    out = []
+    for bs, bpc in [(64, 1), (256, 0)]:
+        st = dm.thermal(16000, 3, max_events=20000, block_size=bs, blocks_per_cu=bpc,
+                        mrw=1 if model == "modified walk" else 0)
+        out.append((dm.temperature(), [st[k] for k in ("n_cross", "n_abs", "n_scat", "n_events",
+                                                       "n_escape", "n_killed", "n_mrw")]))
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(out[0][0], out[1][0])
