@@ -47,7 +47,9 @@ __device__ __forceinline__ int fold_lo(int n, int l) { return (n & 1) ? n / 2 - 
 // point's cos a or sin a of one column (rotated by two pixels a step, exact
 // every VIS_REF steps, so no table is needed), the folded rows come from LDS, one
 // 16-byte read per step for all four.  2 nx ny flops per point: 6.5 GFLOP
-// at 256 x 256 and 5e4 points, 42 us at the FP32 matrix peak.  4 / NRS groups of 32
+// at 256 x 256 and 5e4 points, 42 us at the FP32 matrix peak; 411 us with plain sums
+// on the vector units, 101 now (1e6 points: 5005 and 1445), the phasors' rotation and
+// the staging between barriers taking the rest.  4 / NRS groups of 32
 // points per workgroup share the staged rows; with NRS = 4 the four waves take
 // every fourth 32 rows of one group of points instead (few points: the GPU would
 // be short of waves), added in order.
@@ -784,9 +786,11 @@ int vis_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const d
     if (K == 0) return RT_OK;
     if (!d_img || !d_u || !d_v || !d_re || !d_im)
         return set_err(ctx, RT_E_ARG, "vis: NULL image, (u,v) or output");
-    // rows split over the waves where the points alone leave the GPU short of them
+    // rows split over the waves while that takes no more than one workgroup per CU (256 x
+    // 256: 31 against 67 us at 5e3 points, 70 against 69 at 2e4, 142 against 101 at 5e4;
+    // 128 x 128: 17 against 20, 35 against 21); up to 64 rows there is one tile of them
     const int nb = (K + 127) / 128;
-    if (nb < 2 * ctx->n_cu && ny > 64)
+    if ((K + 31) / 32 <= ctx->n_cu && ny > 64)
         hipLaunchKernelGGL(k_vis<4>, dim3((K + 31) / 32), dim3(VIS_BS), 0, ctx->stream, d_img, nx,
                            ny, d_u, d_v, K, dxy, dra, ddec, d_re, d_im);
     else
