@@ -55,8 +55,7 @@ struct rt_batch {
     // the per-model image chains run on RT_CHAIN_STREAMS streams forked from
     // the step's stream after the thermal launch and joined before its end
     hipStream_t chain_stream[RT_CHAIN_STREAMS] = {};
-    void *d_vws[RT_CHAIN_STREAMS] = {};   // scratch of the transposed DFT
-    size_t vws_cap[RT_CHAIN_STREAMS] = {};
+    GrowBuffer<HipMem> vws[RT_CHAIN_STREAMS];  // scratch of the transposed DFT
     hipEvent_t e_fork = nullptr, e_join[RT_CHAIN_STREAMS] = {};
     hipStream_t stream = nullptr;
 };
@@ -185,7 +184,7 @@ int batch_destroy(rt_batch *b) {
     if (b->e_fork) (void)hipEventDestroy(b->e_fork);
     for (int k = 0; k < RT_CHAIN_STREAMS; ++k) {
         if (b->chain_stream[k]) (void)hipStreamDestroy(b->chain_stream[k]);
-        (void)hipFree(b->d_vws[k]);
+        b->vws[k].release();
         if (b->e_join[k]) (void)hipEventDestroy(b->e_join[k]);
     }
     delete b;
@@ -335,18 +334,8 @@ static int batch_step_buffers(rt_batch *b, int i, const rt_step_item &it) {
     }
     // one scratch per chain stream: the chains of a stream run one after another
     const size_t vws = it.d_g_T ? vis_adjoint_workspace(ctx, it.cam.nx, it.cam.ny, it.K) : 0;
-    const int k = i % RT_CHAIN_STREAMS;
-    if (b->vws_cap[k] < vws) {
-        (void)hipFree(b->d_vws[k]);
-        b->d_vws[k] = nullptr;
-        b->vws_cap[k] = 0;
-        if (hipMalloc(&b->d_vws[k], vws) == hipSuccess) {
-            b->vws_cap[k] = vws;
-        } else {  // the transpose does without
-            b->d_vws[k] = nullptr;
-            (void)hipGetLastError();
-        }
-    }
+    // (an item for which there is no memory does without, see the chain)
+    b->vws[i % RT_CHAIN_STREAMS].grow(vws);
     return RT_OK;
 }
 
@@ -377,7 +366,8 @@ static int batch_enqueue_image_chain(rt_batch *b, int i, const rt_step_item &it,
     if (!it.d_g_logrho || !it.d_g_T) return RT_OK;
     rc = vis_adjoint_run(ctx, b->d_gre[i], b->d_gim[i], it.cam.nx, it.cam.ny, it.dxy, it.d_u,
                          it.d_v, it.K, it.dra, it.ddec, b->d_gimg[i],
-                         b->d_vws[i % RT_CHAIN_STREAMS]);
+                         b->vws[i % RT_CHAIN_STREAMS].get(
+                             vis_adjoint_workspace(ctx, it.cam.nx, it.cam.ny, it.K)));
     if (rc) return rc;
     hipLaunchKernelGGL(k_scale_copy, dim3(nblk(npix, 256)), dim3(256), 0, sm, b->d_gimg[i],
                        (float)it.scale, (size_t)npix, b->d_gimg[i]);
@@ -402,7 +392,7 @@ static std::vector<const void *> model_buffers(const rt_batch *b) {
     const RefinePool &P = b->ctx->ref;
     const void *q[] = {P.xy, P.val, P.child, P.gw, P.ctl};
     v.insert(v.end(), q, q + 5);
-    v.insert(v.end(), b->d_vws, b->d_vws + RT_CHAIN_STREAMS);
+    for (const GrowBuffer<HipMem> &w : b->vws) v.push_back(w.p);
     return v;
 }
 

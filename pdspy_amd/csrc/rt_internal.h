@@ -8,6 +8,7 @@
 
 #include "../../include/pdspy_amd.h"
 #include "rt_device.h"
+#include "scratch.h"
 #include "tables.h"
 
 #define RT_MAX_SPEC 8    // species per model
@@ -36,6 +37,17 @@ struct RefinePool {
     int *child = nullptr;
     float *gw = nullptr;
     unsigned *ctl = nullptr;
+};
+
+// device memory for GrowBuffer
+struct HipMem {
+    static void *alloc(size_t n) {
+        void *p = nullptr;
+        if (hipMalloc(&p, n) == hipSuccess) return p;
+        (void)hipGetLastError();  // the caller does without
+        return nullptr;
+    }
+    static void free(void *p) { (void)hipFree(p); }
 };
 
 struct rt_ctx {

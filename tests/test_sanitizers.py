@@ -39,6 +39,13 @@ def test_table_builder_under_asan_ubsan(built):
     assert r.returncode == 0 and "tables_check ok" in r.stdout
 
 
+def test_device_scratch_rules_under_asan_ubsan(built):
+    r = subprocess.run([os.path.join(built, "scratch_check")], capture_output=True, text=True,
+                       timeout=120, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1"))
+    print(r.stdout[-2000:], r.stderr[-4000:])
+    assert r.returncode == 0 and "scratch_check ok" in r.stdout
+
+
 def test_oracle_suite_under_asan_ubsan(built):
     """test_oracle.py against the instrumented oracle (the heavier Monte Carlo
     cases are deselected to keep the sanitized run to about a minute)."""
