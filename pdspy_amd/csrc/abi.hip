@@ -325,10 +325,10 @@ int rt_create(int device, rt_ctx **out) {
 }
 
 rt_ctx::~rt_ctx() {
-    void *p[] = {ref.xy, ref.val, ref.child, ref.gw, ref.ctl, d_icount, vis_ws};
+    void *p[] = {ref.xy, ref.val, ref.child, ref.gw, ref.ctl, d_icount};
     for (void *q : p)
         if (q) (void)hipFree(q);
-    if (vis_ws_ev) (void)hipEventDestroy(vis_ws_ev);
+    vis_ws.release();
 }
 
 int rt_destroy(rt_ctx *ctx) {

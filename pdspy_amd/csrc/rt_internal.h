@@ -39,15 +39,42 @@ struct RefinePool {
     unsigned *ctl = nullptr;
 };
 
-// device memory for GrowBuffer
+// the device of GrowBuffer and SharedScratch; a call that fails is one its caller
+// does without, so it leaves no error
 struct HipMem {
-    static void *alloc(size_t n) {
-        void *p = nullptr;
-        if (hipMalloc(&p, n) == hipSuccess) return p;
-        (void)hipGetLastError();  // the caller does without
-        return nullptr;
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    static bool ok(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
     }
-    static void free(void *p) { (void)hipFree(p); }
+    // (a thread may be capturing a stream of its own meanwhile: an allocation, or a
+    // wait for an event, is none of that capture's and must not end it)
+    struct Relaxed {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        bool on = ok(hipThreadExchangeStreamCaptureMode(&mode));
+        ~Relaxed() {
+            if (on) ok(hipThreadExchangeStreamCaptureMode(&mode));
+        }
+    };
+    static void *alloc(size_t n) {
+        Relaxed r;
+        void *p = nullptr;
+        return ok(hipMalloc(&p, n)) ? p : nullptr;
+    }
+    static void free(void *p) {
+        Relaxed r;
+        ok(hipFree(p));
+    }
+    static bool make(Event &e) { return ok(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+    static void drop(Event e) { ok(hipEventDestroy(e)); }
+    static bool wait_host(Event e) {
+        Relaxed r;
+        return ok(hipEventSynchronize(e));
+    }
+    static bool wait(Stream s, Event e) { return ok(hipStreamWaitEvent(s, e, 0)); }
+    static bool record(Event e, Stream s) { return ok(hipEventRecord(e, s)); }
+    static void drain(Stream s) { ok(hipStreamSynchronize(s)); }
 };
 
 struct rt_ctx {
@@ -58,13 +85,9 @@ struct rt_ctx {
     int n_cu = 0;
     int wallclock_khz = 0;
     RefinePool ref;
-    // scratch of the transposed DFT's partial sums: at most 64 KiB for
-    // each of 4 x CUs workgroups, kept between calls; its last user's stream and an event behind that use
-    void *vis_ws = nullptr;
-    size_t vis_ws_cap = 0;
-    hipEvent_t vis_ws_ev = nullptr;
-    hipStream_t vis_ws_stream = nullptr;
-    bool vis_ws_used = false;
+    // scratch of the transposed DFT's partial sums: at most 64 KiB for each of 4 x CUs
+    // workgroups, kept between calls
+    SharedScratch<HipMem> vis_ws;
     // cells crossed by camera rays since the last read: [0] image rays
     // (sub-pixels included), [1] adjoint sweeps
     unsigned long long *d_icount = nullptr;

@@ -800,59 +800,40 @@ int vis_run(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy, const d
     return RT_OK;
 }
 
-// the context's scratch for a call on its stream: grown if need be, the call
-// ordered behind the last one that used it.  NULL in a capture (which can
-// neither allocate nor wait on an event from outside) and without memory.
-static void *adj_scratch(rt_ctx *ctx, size_t bytes) {
+// whether calls on this stream are being recorded (or it cannot be told: a capture
+// elsewhere that the null stream would join)
+static bool capturing(hipStream_t sm) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
-        return nullptr;
-    if (!ctx->vis_ws_ev &&
-        hipEventCreateWithFlags(&ctx->vis_ws_ev, hipEventDisableTiming) != hipSuccess)
-        return nullptr;
-    if (ctx->vis_ws_cap < bytes) {
-        if (ctx->vis_ws_used && hipEventSynchronize(ctx->vis_ws_ev) != hipSuccess) return nullptr;
-        if (ctx->vis_ws) (void)hipFree(ctx->vis_ws);
-        ctx->vis_ws = nullptr;
-        ctx->vis_ws_cap = 0;
-        ctx->vis_ws_used = false;
-        if (hipMalloc(&ctx->vis_ws, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            ctx->vis_ws = nullptr;
-            return nullptr;
-        }
-        ctx->vis_ws_cap = bytes;
-    }
-    if (ctx->vis_ws_used && ctx->vis_ws_stream != ctx->stream &&
-        hipStreamWaitEvent(ctx->stream, ctx->vis_ws_ev, 0) != hipSuccess)
-        return nullptr;
-    return ctx->vis_ws;
+    return !HipMem::ok(hipStreamIsCapturing(sm, &st)) || st != hipStreamCaptureStatusNone;
 }
 
 int vis_adjoint_run(rt_ctx *ctx, const float *d_gre, const float *d_gim, int nx, int ny, double dxy,
                     const double *d_u, const double *d_v, int K, double dra, double ddec,
                     float *d_g_img, void *ws) {
     if (nx < 1 || ny < 1 || K < 0 || !(dxy > 0)) return set_err(ctx, RT_E_ARG, "vis adjoint: invalid sizes");
+    const hipStream_t sm = ctx->stream;
     const size_t need = vis_adjoint_workspace(ctx, nx, ny, K);
-    const bool own = need > 0 && !ws;
-    if (own) ws = adj_scratch(ctx, need);
-    if (need > 0 ? ws != nullptr : adj_tiled(nx, ny, K)) {
+    auto tiled = [&](void *part) {
         const AdjSplit a = adj_split(ctx, nx, ny, K);
-        hipLaunchKernelGGL(k_vis_adj_part, dim3(a.tx, a.ty, a.splits), dim3(256), 0, ctx->stream,
-                           d_gre, d_gim, nx, ny, d_u, d_v, K, dxy, dra, ddec, a.per,
-                           need > 0 ? (float *)ws : nullptr, d_g_img);
-        if (need > 0)
-            hipLaunchKernelGGL(k_vis_adj_sum, dim3(a.tx, a.ty, 16), dim3(256), 0, ctx->stream,
-                               (const float *)ws, a.splits, nx, ny, d_g_img);
-        if (own) {
-            HIPCHK(ctx, hipEventRecord(ctx->vis_ws_ev, ctx->stream));
-            ctx->vis_ws_stream = ctx->stream;
-            ctx->vis_ws_used = true;
-        }
-    } else {
+        hipLaunchKernelGGL(k_vis_adj_part, dim3(a.tx, a.ty, a.splits), dim3(256), 0, sm, d_gre,
+                           d_gim, nx, ny, d_u, d_v, K, dxy, dra, ddec, a.per, (float *)part,
+                           d_g_img);
+        if (part)
+            hipLaunchKernelGGL(k_vis_adj_sum, dim3(a.tx, a.ty, 16), dim3(256), 0, sm,
+                               (const float *)part, a.splits, nx, ny, d_g_img);
+    };
+    bool done = false;
+    if (need == 0 ? adj_tiled(nx, ny, K) : ws != nullptr) {
+        tiled(need ? ws : nullptr);
+        done = true;
+    } else if (need > 0 && !capturing(sm)) {
+        // (a capture can neither allocate nor wait on an event from outside)
+        done = ctx->vis_ws.with(sm, need, tiled);
+    }
+    if (!done) {
         dim3 grid((nx + ADJ_T - 1) / ADJ_T, (ny + ADJ_T - 1) / ADJ_T);
-        hipLaunchKernelGGL(k_vis_adj, grid, dim3(ADJ_BS), 0, ctx->stream, d_gre, d_gim, nx, ny,
-                           d_u, d_v, K, dxy, dra, ddec, d_g_img);
+        hipLaunchKernelGGL(k_vis_adj, grid, dim3(ADJ_BS), 0, sm, d_gre, d_gim, nx, ny, d_u, d_v, K,
+                           dxy, dra, ddec, d_g_img);
     }
     HIPCHK(ctx, hipGetLastError());
     return RT_OK;
