@@ -470,11 +470,18 @@ __device__ __forceinline__ A trace_ray(const CamParams &C, const W &walk, bool a
         t = __shfl_up(t, 1, L);
         f = __shfl_up(f, 1, L);
         r.tau0 = l > 0 ? t : 0.f;
+        // The ray ends in the first share that takes it over tau_stop.  What lies
+        // behind must not count, whatever it is: that share, walked with the optical
+        // depth in front of it unknown, may have gone on into cells whose opacity or
+        // source is not finite, and so have those after it (hence NaN is "over" too).
+        const bool over = inten && !(r.tau0 + r.tau <= C.tau_stop);
+        const uint64_t ends = __ballot(over) >> (__lane_id() - l);
         if (inten) {
-            const bool past = r.tau0 > C.tau_stop;
-            if (act && !past && l > 0 && r.tau0 + r.tau > C.tau_stop) share(r.tau0);
+            const bool past = (ends & ((1ull << l) - 1ull)) != 0ull;
+            if (act && over && !past && l > 0) share(r.tau0);
             r.front = past ? (A)0 : sizeof(A) == 8 ? (l > 0 ? f : (A)1) : (A)__expf(-r.tau0);
             if (past) {
+                r.I = 0;
                 r.lmin = RT_INF;
                 ns = 0;
             }

@@ -865,3 +865,60 @@ def test_grid_range_check_is_the_torch_expression(conv, K):
             rt.vis_grid(img, d, base[0], np.zeros(K + 1), conv=conv)
         with pytest.raises(ValueError):
             rt.vis_grid(img, d, base[0], base[1, :1], conv=conv)
+
+
+def _hidden_shells():
+    """A full sphere of shells of optical depth 6.5: its shells 0 .. 3 lie behind 52,
+    where every ray has ended (tau_stop 40), but not every share of one on its own."""
+    nr, nt = 12, 6
+    lam = np.logspace(-1, 4, 20)
+    k = 1e3 * lam ** -0.5
+    rw = np.logspace(np.log10(0.5), 2.0, nr + 1) * AU
+    ext = 1.3 * np.exp(np.interp(np.log(500.0), np.log(lam), np.log(k)))
+    rho = np.broadcast_to(6.5 / (ext * np.diff(rw)), (1, 1, nt, nr)).copy()
+    arr = dict(rw=rw, tw=np.linspace(0, np.pi, nt + 1), pw=np.array([0, 2 * np.pi]), rho=rho,
+               lam_um=lam, kabs=np.array([k]), ksca=np.array([0.3 * k]), gsca=None,
+               stars=np.array([[7e10, 4000.0, 0.0, 0.0, 0.0]]))
+    hidden = np.zeros((1, nt, nr), bool)
+    hidden[..., :4] = True
+    return arr, hidden.ravel()
+
+
+@pytest.mark.parametrize("npix", [8, 64, 300, 513, 740])
+@pytest.mark.parametrize("nrefine", [0, 2])
+def test_nothing_behind_tau_stop_counts(npix, nrefine):
+    """What lies behind the point where every ray has ended may be anything: a
+    source or density there that is not finite changes neither the image nor the
+    gradient of the other cells (32 lanes per ray to one)."""
+    print("case: behind tau_stop, npix %d nrefine %d" % (npix, nrefine), flush=True)
+    arr, hidden = _hidden_shells()
+    dm = _dev(arr)
+    rng = np.random.default_rng(npix)
+    T = torch.tensor(rng.uniform(50, 200, hidden.size), dtype=torch.float32, device="cuda")
+    J = torch.tensor(rng.uniform(1e-14, 2e-14, hidden.size), dtype=torch.float32, device="cuda")
+    rho = dm.rho_device().clone()
+    h = torch.tensor(hidden, device="cuda")
+    T[h], J[h] = 10.0, 1e-17  # (the gradient's unit is set by the largest source)
+    dimg = torch.tensor(rng.standard_normal((npix, npix)), dtype=torch.float32, device="cuda")
+    pix = 120.0 / npix * AU
+
+    def run(T, J, rho, grad=True):
+        cam = dm.camera(npix, pix, 500.0, incl=40.0, phi=10.0, incl_star=False, jscat=J,
+                        nrefine=nrefine)
+        img = dm.image(cam, T, rho)
+        g = dm.image_adjoint(cam, T, rho, dimg) if grad else ()
+        return (img,) + tuple(x[..., ~h] for x in g)
+
+    def put(t, x):
+        t = t.clone()
+        t[..., h] = x
+        return t
+
+    want = run(T, J, rho)
+    assert bool(torch.isfinite(want[0]).all()) and float(want[1].abs().max()) > 0
+    inf, nan = float("inf"), float("nan")
+    assert torch.equal(run(put(T, inf), J, rho, False)[0], want[0])
+    for Jx, rx in ((put(J, nan), rho), (J, put(rho, nan)), (J, put(rho, inf))):
+        got = run(T, Jx, rx)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
