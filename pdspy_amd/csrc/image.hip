@@ -706,6 +706,7 @@ struct RefArgs {
     int nref;         // levels that may split
     float d0;         // side of a level-0 node (au): pixel / nsub
     unsigned n0;      // level-0 nodes: every tile's pixels x nsub^2
+    unsigned nray0;   // those of them that lie in the image
     int ns2;          // nsub^2
 };
 
@@ -751,8 +752,9 @@ __global__ void k_ref_init(CamParams C, RefArgs R) {
 }
 
 // lanes per ray for n rays: about four waves per SIMD, and no more than a ray's
-// crossings are worth (n depends on the image alone, so the sums do not change
-// with the launch)
+// crossings are worth.  A ray's sums are rounded by its shares, so n is a number
+// that the image alone decides: the nodes that tiles add beyond its edges are
+// not counted
 __device__ __host__ __forceinline__ int ref_lanes(unsigned n) {
     int L = 1;
     while (L < IMG_MAXL && (size_t)n * (size_t)(2 * L) <= IMG_LANES) L *= 2;
@@ -767,7 +769,8 @@ __global__ void __launch_bounds__(256) k_ref_trace(CamParams C, RefArgs R, int L
     const int lane = __lane_id();
     unsigned nrays = 0;
     uint32_t nseg = 0;
-    const int LN = ref_lanes(end > start ? end - start : 0u), l = (int)(threadIdx.x & (unsigned)(LN - 1));
+    const int LN = ref_lanes(L == 0 ? R.nray0 : end > start ? end - start : 0u),
+              l = (int)(threadIdx.x & (unsigned)(LN - 1));
     const unsigned per = blockDim.x / (unsigned)LN;  // nodes of a block
     for (unsigned base = start + blockIdx.x * per; base < end; base += gridDim.x * per) {
         const unsigned i = base + threadIdx.x / (unsigned)LN;
@@ -882,7 +885,7 @@ __global__ void __launch_bounds__(256) k_ref_adj(CamParams C, RefArgs R, double 
     int *key = (int *)(adj_lds + 2 * H);
     const unsigned n = R.ctl[0] < R.cap ? R.ctl[0] : R.cap;
     uint32_t nseg = 0;
-    const int LN = ref_lanes(n), l = (int)(threadIdx.x & (unsigned)(LN - 1));
+    const int LN = ref_lanes(n - R.n0 + R.nray0), l = (int)(threadIdx.x & (unsigned)(LN - 1));
     const unsigned per = blockDim.x / (unsigned)LN;
     for (unsigned base = blockIdx.x * per; base < n; base += gridDim.x * per) {
         for (unsigned t = threadIdx.x; t < H; t += blockDim.x) {
@@ -1312,7 +1315,7 @@ static int refine_run(rt_model *m, const rt_camera *cam, CamParams C, float *d_i
         RefinePool &P = ctx->ref;
         RefArgs R{P.xy, P.val, P.child, P.gw, P.ctl, (unsigned)P.cap,
                   (float)(cam->refine_crit > 0 ? cam->refine_crit : 1.0), nref, C.pixf / C.nsub,
-                  (unsigned)n0, ns2};
+                  (unsigned)n0, (unsigned)((size_t)C.nx * C.ny * ns2), ns2};
         hipLaunchKernelGGL(k_ref_init, dim3(nblk(n0, 256)), dim3(256), 0, sm, C, R);
         for (int L = 0; L <= nref; ++L) {
             hipLaunchKernelGGL(k_ref_trace, dim3(gblk), dim3(256), 0, sm, C, R, L);

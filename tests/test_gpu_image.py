@@ -922,3 +922,24 @@ def test_nothing_behind_tau_stop_counts(npix, nrefine):
         got = run(T, Jx, rx)
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("npix", [72, 360])
+def test_ray_tiles_do_not_change_a_sub_pixelled_image(npix):
+    """360 x 360: with 64 x 1 tiles the padding takes the number of nodes over a
+    power of two, at which a launch would give each ray fewer lanes.  tau_stop
+    ends rays inside their shares."""
+    print("case: tiles with sub-pixels, npix %d" % npix, flush=True)
+    arr, T = _disk_setup(nr=32, nt=16)
+    dm = _dev(arr)
+    Td = torch.tensor(T, dtype=torch.float32, device="cuda")
+    dimg = torch.rand((npix, npix), dtype=torch.float32, device="cuda")
+    ref = None
+    for tile in [(0, 0), (64, 1), (8, 8), (16, 16)]:
+        cam = dm.camera(npix, 288.0 / npix * AU, 1300.0, incl=50.0, pa=10.0, tile=tile, nrefine=3,
+                        tau_stop=0.05)
+        out = [dm.image(cam, Td)] + list(dm.image_adjoint(cam, Td, None, dimg))
+        if ref is None:
+            ref = out
+        for a, b in zip(out, ref):
+            assert torch.equal(a, b), tile
