@@ -233,9 +233,19 @@ __device__ __forceinline__ double phi_at(const CamParams &C, const RayGeo &q, in
     const double den = dy * cp - dx * sp;
     if (up ? !(den > 0.0) : !(den < 0.0)) return 1e300;
     const double t = (q.x0 * sp - q.y0 * cp) * rcp_d(den);
-    // in a cell of more than half a turn the wall ahead may be one that the
-    // line has passed behind the position
-    if (t < s - 1e-12 * fabs(s) && C.g.pw[ip + 1] - C.g.pw[ip] > 3.2f) return 1e300;
+    // In a cell of more than half a turn, a wall ahead of the cell may be one that the
+    // line has passed behind the position (to come round into the cell by its other
+    // end): it is not met again.  Such a position lies past the wall by what the other
+    // cells turn at least.  One just past it is there because a share's first cell is
+    // found in FP32, with angles good to 1e-6, and has yet to cross.
+    if (t < s) {
+        const double w = (double)C.g.pw[ip + 1] - (double)C.g.pw[ip];
+        if (w > 3.1416) {
+            const double x = fma(s, dx, q.x0), y = fma(s, dy, q.y0);
+            const double sn = fabs(fma(y, cp, -(x * sp))), cs = fma(x, cp, y * sp);
+            if (!(sn <= fmin(4e-6, 0.5 * (6.283185307179586 - w)) * cs)) return 1e300;
+        }
+    }
     return fmax(t, s);
 }
 

@@ -943,3 +943,48 @@ def test_ray_tiles_do_not_change_a_sub_pixelled_image(npix):
             ref = out
         for a, b in zip(out, ref):
             assert torch.equal(a, b), tile
+
+
+@pytest.mark.parametrize("thick", [0, 1])
+@pytest.mark.parametrize("wide", [0, 1])
+@pytest.mark.parametrize("incl", [53.0, 127.0])  # rays that turn one way and the other
+def test_share_that_begins_at_the_wall_of_a_wide_phi_cell(incl, wide, thick):
+    """Two phi cells, one of more than half a turn, whose common wall passes within
+    three FP32 ulps of where a share of a ray may begin (at a sphere): the cell
+    found there in FP32 may be the one just left.  The optical depth of 8 x 8 rays
+    (32 lanes each) against the FP64 oracle, to 2e-5 of the largest as above."""
+    print("case: wide phi cell %d, thick cell %d, incl %g" % (wide, thick, incl), flush=True)
+    npix, pix, nr = 8, 20.0, 24
+    rw = np.linspace(4.0, 100.0, nr + 1)
+    lam = np.logspace(-1, 4, 20)
+    i, ph = np.radians(incl), np.radians(23.0)
+    n = np.array([np.sin(i) * np.sin(ph), -np.sin(i) * np.cos(ph), np.cos(i)])
+    ex = np.array([np.cos(ph), np.sin(ph), 0.0])
+    ey = np.cross(n, ex)
+    kw = dict(incl=incl, phi=23.0, lam_um=500.0, mode=1, incl_star=False)
+    walls = set()
+    for j, k in ((2, 3), (5, 6), (6, 2), (3, 6)):
+        p0 = (k - npix // 2) * pix * ex + (j - npix // 2) * pix * ey
+        for r in rw[rw > np.linalg.norm(p0)][:-1]:
+            s = np.sqrt(r * r - p0 @ p0)
+            for x in (p0 - s * n, p0 + s * n):
+                a = np.arctan2(x[1], x[0]) % (2 * np.pi)
+                # the other cell at least 1.6 (a quarter turn, for the oracle)
+                if (3.3 < a < 4.6) if wide == 0 else (1.65 < a < 2.95):
+                    walls.update(a + m * np.spacing(np.float32(a)) for m in (-1, 0, 1, 2))
+    assert len(walls) > 40
+    for a in sorted(walls):
+        rho = np.full((1, 2, 1, nr), 1e-16)
+        rho[0, thick] = 4e-15
+        arr = dict(rw=rw * AU, tw=np.array([0, np.pi]), pw=np.array([0.0, a, 2 * np.pi]), rho=rho,
+                   lam_um=lam, kabs=np.ones((1, 20)), ksca=np.zeros((1, 20)), gsca=None,
+                   stars=np.array([[7e10, 4000.0, 0.0, 0.0, 0.0]]))
+        T = np.full(2 * nr, 100.0)
+        dm = _dev(arr)
+        cam = dm.camera(npix, pix * AU, **kw)
+        img = dm.image(cam, torch.tensor(T, dtype=torch.float32, device="cuda"))
+        ref = oracle.image(arr, T, [1.0], npix, pix * AU, **kw)
+        err = np.abs(img.double().cpu().numpy() - ref)
+        err[npix // 2, npix // 2] = 0.0  # along the axis of the spheres
+        assert err.max() <= 2e-5 * ref.max(), (a, np.argwhere(err > 2e-5 * ref.max()).tolist())
+
