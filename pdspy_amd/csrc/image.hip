@@ -1261,8 +1261,9 @@ static int setup_camera(rt_model *m, const rt_camera *cam, CamParams &C, KapArg 
     C.ny = cam->ny;
     C.nsub = cam->nsub > 0 ? cam->nsub : 1;
     C.mode = cam->mode;
-    // ray tile: neighbouring rays run in tile_w x tile_h pixels (default 8 x 8)
-    C.tw = cam->tile_w > 0 ? cam->tile_w : 8;
+    // ray tile: neighbouring rays run in tile_w x tile_h pixels (default 8 x 8; 64
+    // wide if only the height is given)
+    C.tw = cam->tile_w > 0 ? cam->tile_w : (cam->tile_h > 0 ? 64 : 8);
     C.th = cam->tile_h > 0 ? cam->tile_h : 64 / C.tw;
     if (C.th < 1) C.th = 1;
     if (C.tw * C.th > 256 || (C.tw * C.th) % 64)

@@ -988,3 +988,17 @@ def test_share_that_begins_at_the_wall_of_a_wide_phi_cell(incl, wide, thick):
         err[npix // 2, npix // 2] = 0.0  # along the axis of the spheres
         assert err.max() <= 2e-5 * ref.max(), (a, np.argwhere(err > 2e-5 * ref.max()).tolist())
 
+
+def test_ray_tile_of_a_height_alone():
+    """64 pixels wide: heights 1 to 4 are accepted, more are not (256 pixels)."""
+    print("case: tile heights", flush=True)
+    arr, T = _disk_setup(nr=16, nt=8)
+    dm = _dev(arr)
+    Td = torch.tensor(T, dtype=torch.float32, device="cuda")
+    cam = lambda h: dm.camera(72, 4.0 * AU, 1300.0, incl=50.0, tile=(0, h))
+    ref = dm.image(cam(0), Td)
+    for h in (1, 2, 3, 4):
+        assert torch.equal(dm.image(cam(h), Td), ref)
+    for h in (5, 8, 16, 32):
+        with pytest.raises(RTError):
+            dm.image(cam(h), Td)
