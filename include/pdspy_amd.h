@@ -134,7 +134,8 @@ typedef struct {
     int incl_star;      /* 1: add stars as point sources (pdspy nostar=False) */
     double tau_stop;    /* stop a ray once tau exceeds this (0 = 40) */
     int tile_w, tile_h; /* ray tile of one thread block, a multiple of 64 pixels
-                           up to 256 (0, 0: 8 x 8; a height alone: 64 wide; a width
+                           up to 256 (0, 0: 8 x 8, or 64 x 1 where a sub-pixelled image then
+                           has fewer nodes; a height alone: 64 wide; a width
                            alone: 64 pixels); results do not depend on it */
     const float *d_jscat; /* scattering source: mean intensity J_nu[cells] at lam_um
                              from rt_scattering_source; the extinction is then

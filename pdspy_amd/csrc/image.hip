@@ -1262,8 +1262,14 @@ static int setup_camera(rt_model *m, const rt_camera *cam, CamParams &C, KapArg 
     C.nsub = cam->nsub > 0 ? cam->nsub : 1;
     C.mode = cam->mode;
     // ray tile: neighbouring rays run in tile_w x tile_h pixels (default 8 x 8; 64
-    // wide if only the height is given)
+    // wide if only the height is given).  Sub-pixelled images keep every tile's pixels
+    // in their node pool, which is as large as its caller made it under capture: theirs
+    // is 64 x 1 where that takes fewer (64 x 1 pixels: 64 nodes, 512 with 8 x 8 tiles)
     C.tw = cam->tile_w > 0 ? cam->tile_w : (cam->tile_h > 0 ? 64 : 8);
+    if (cam->tile_w <= 0 && cam->tile_h <= 0 && cam->nrefine > 0) {
+        auto up = [](int n, int t) { return (size_t)((n + t - 1) / t) * t; };
+        if (up(C.nx, 64) * C.ny < up(C.nx, 8) * up(C.ny, 8)) C.tw = 64;
+    }
     C.th = cam->tile_h > 0 ? cam->tile_h : 64 / C.tw;
     if (C.th < 1) C.th = 1;
     if (C.tw * C.th > 256 || (C.tw * C.th) % 64)

@@ -124,3 +124,30 @@ def test_subpixel_pool_grows_and_cap_of_levels():
     dm.image(one, Td)
     n1, _ = dm.refine_stats()
     assert 48 * 48 < n1 <= 5 * 48 * 48
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 1), (128, 129), (192, 30), (72, 72)])
+def test_capture_in_a_pool_of_twice_the_pixels(nx, ny):
+    """A pool of two nodes per pixel (rows padded to 64) is enough to capture an image
+    that splits none of its pixels; every replay is the eager image bit for bit."""
+    print("case: captured sub-pixels, %dx%d" % (nx, ny), flush=True)
+    from pdspy_amd import _lib
+    arr, T = _disk_setup(nr=16, nt=8)
+    Td = torch.tensor(T, dtype=torch.float32, device="cuda")
+    eager = rt.DeviceModel(arr)
+    ctx = _lib.Context(0)
+    dm = rt.DeviceModel(arr, ctx=ctx)
+    cam = dm.camera(nx, 4.0 * AU, 1300.0, ny=ny, incl=50.0, nrefine=1, refine_crit=1e9)
+    want = eager.image(cam, Td)
+    dm.image(dm.camera(8, 4.0 * AU, 1300.0, incl=50.0), Td)  # the model's own buffers
+    ctx.check(ctx.L.rt_refine_reserve(ctx.h, 2 * ((nx + 63) // 64 * 64) * ny))
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = dm.image(cam, Td)
+    for _ in range(3):
+        out.fill_(-1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
