@@ -313,7 +313,7 @@ int rt_vis_dft(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy,
                const double *d_u, const double *d_v, int K, double dra, double ddec,
                float *d_re, float *d_im);
 /* Transpose: d_g_img[j][k] = dL/dI given dL/dRe, dL/dIm at each point.  Many points
- * use device scratch of the context (at most 64 MiB, allocated at the first such
+ * use device scratch of the context (at most 48 MiB, allocated at the first such
  * call, freed with the context; in a stream capture none is used). */
 int rt_vis_dft_adjoint(rt_ctx *ctx, const float *d_gre, const float *d_gim, int nx,
                        int ny, double dxy, const double *d_u, const double *d_v, int K,

@@ -85,8 +85,8 @@ struct rt_ctx {
     int n_cu = 0;
     int wallclock_khz = 0;
     RefinePool ref;
-    // scratch of the transposed DFT's partial sums: at most 64 KiB for each of 4 x CUs
-    // workgroups, kept between calls
+    // scratch of the transposed DFT's partial sums: 64 KiB for each of at most
+    // 3 x CUs workgroups, kept between calls
     SharedScratch<HipMem> vis_ws;
     // cells crossed by camera rays since the last read: [0] image rays
     // (sub-pixels included), [1] adjoint sweeps

@@ -164,11 +164,16 @@ __global__ void __launch_bounds__(VIS_BS) k_vis(const float *img, int nx, int ny
 // and a share of the points, 32 at a time: their cosines and sines go through
 // LDS once (16 entries per lane, exact every 8, rotated in between) and serve
 // 64 x 64 x 4 products, so the matrix cores set the pace.  The folded image has
-// few such tiles, so the points are split over two workgroups per CU;
+// few such tiles, so the points are split over the CUs (adj_split);
 // their partial planes are added in order by k_vis_adj_sum.
 // 256 x 256 pixels, 5e4 points: 467 us with k_vis_adj, 111 now; 1024 x 1024: 7446
-// and 1241.
-#define VA_CH 32  // points per chunk
+// and 1219.
+// An accumulator takes 64 chunks and is then added to the share's sum: a large
+// image has few shares (8 at 1024 x 1024, one from about 2450 x 2450 on), and the
+// rounding of an FP32 sum grows with the root of its number of terms.  2048 x 2048, 1e6
+// points, rms error over rms gradient: 1.3e-5 in one sum per share, 9e-7 now.
+#define VA_CH 32   // points per chunk
+#define VA_SUM 64  // chunks per accumulator
 // below this many pixel x point products k_vis_adj, which needs no scratch and one
 // launch, is the faster one: 22 against 27 us at 256 x 256 and 2e3 points, 51
 // against 31 at 5e3 (smaller images count as 256 x 256: they take as long)
@@ -176,15 +181,30 @@ __global__ void __launch_bounds__(VIS_BS) k_vis(const float *img, int nx, int ny
 
 struct AdjSplit {
     int tx, ty, splits, per;  // tiles, shares of the points, chunks per share
+    int wpc;                  // workgroups per CU (2 or 3)
 };
 
+// Shares that fill two workgroups per CU, which is what the registers allow at full
+// speed, or three, 5 % slower each (some are spilled), where that comes out
+// ahead: a launch takes its rounds of them.  2300 x 2300 pixels (324 tiles): two shares
+// at three per CU 4.1 ms, one at two 5.8; 300 x 300 (9 tiles): 56 shares, 504
+// workgroups at two per CU, 0.38 ms, 57 shares 0.44.
 static AdjSplit adj_split(const rt_ctx *ctx, int nx, int ny, int K) {
     AdjSplit a;
     a.tx = (fold_n(nx) + 63) / 64;
     a.ty = (fold_n(ny) + 63) / 64;
     const long tiles = (long)a.tx * a.ty, chunks = ((long)K + VA_CH - 1) / VA_CH;
-    long s = (2l * ctx->n_cu + tiles - 1) / tiles;
-    s = std::max(1l, std::min(s, (chunks + 3) / 4));
+    double best = 0.0;
+    long s = 1;
+    for (int wpc = 2; wpc <= 3; ++wpc) {
+        const long c = (long)wpc * ctx->n_cu, n = std::max(1l, std::min(c / tiles, (chunks + 3) / 4));
+        const double cost = (double)((tiles * n + c - 1) / c) * wpc / n * (wpc == 3 ? 1.05 : 1.0);
+        if (wpc == 2 || cost < best) {
+            best = cost;
+            s = n;
+            a.wpc = wpc;
+        }
+    }
     a.per = (int)((chunks + s - 1) / s);
     a.splits = (int)((chunks + a.per - 1) / a.per);
     return a;
@@ -194,7 +214,7 @@ static bool adj_tiled(int nx, int ny, int K) {
     return std::max(65536.0, (double)nx * ny) * K >= VIS_ADJ_MIN;
 }
 
-// at most (2 n_cu + tiles) planes' worth: 64 MiB on 256 CUs
+// at most 3 n_cu workgroups' planes: 48 MiB on 256 CUs
 size_t vis_adjoint_workspace(const rt_ctx *ctx, int nx, int ny, int K) {
     if (nx < 1 || ny < 1 || !adj_tiled(nx, ny, K)) return 0;
     const AdjSplit a = adj_split(ctx, nx, ny, K);
@@ -212,7 +232,9 @@ __device__ __forceinline__ void unfold_pixels(int l, int m, int nx, int ny, floa
     if (jm != jp && km != kp) gimg[(size_t)jm * nx + km] = (p1 - p2) - (p3 + p4);
 }
 
-__global__ void __launch_bounds__(256) k_vis_adj_part(const float *gre, const float *gim, int nx,
+// WPC: workgroups per CU the registers are kept for
+template <int WPC>
+__global__ void __launch_bounds__(256, WPC) k_vis_adj_part(const float *gre, const float *gim, int nx,
                                                       int ny, const double *u, const double *v,
                                                       int K, double dxy, double dra, double ddec,
                                                       int per, float *part, float *gimg) {
@@ -222,7 +244,7 @@ __global__ void __launch_bounds__(256) k_vis_adj_part(const float *gre, const fl
     const int i32 = lane & 31, kh = lane >> 5, wr = (w >> 1) * 32, wc = (w & 1) * 32;
     const int l0 = blockIdx.y * 64, m0 = blockIdx.x * 64;
     const double ox = fold_off(nx), oy = fold_off(ny);
-    vf16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
+    vf16 p1 = {}, p2 = {}, p3 = {}, p4 = {}, t1 = {}, t2 = {}, t3 = {}, t4 = {};
     // table: lane of point tp, 16 rows (tg < 4) or columns
     const int tp = threadIdx.x >> 3, tg = threadIdx.x & 7;
     const int c0 = blockIdx.z * per, c1 = min(c0 + per, (K + VA_CH - 1) / VA_CH);
@@ -271,12 +293,19 @@ __global__ void __launch_bounds__(256) k_vis_adj_part(const float *gre, const fl
             p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.x, h.y * a.y, p3, 0, 0, 0);
             p4 = __builtin_amdgcn_mfma_f32_32x32x2f32(r.y, h.y * a.x, p4, 0, 0, 0);
         }
+        if ((c - c0) % VA_SUM == VA_SUM - 1 || c == c1 - 1) {
+            t1 += p1;
+            t2 += p2;
+            t3 += p3;
+            t4 += p4;
+            p1 = p2 = p3 = p4 = vf16{};
+        }
     }
     if (!part) {  // one share: no planes
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            unfold_pixels(l0 + wr + 8 * (r >> 2) + 4 * kh + (r & 3), m0 + wc + i32, nx, ny, p1[r],
-                          p2[r], p3[r], p4[r], gimg);
+            unfold_pixels(l0 + wr + 8 * (r >> 2) + 4 * kh + (r & 3), m0 + wc + i32, nx, ny, t1[r],
+                          t2[r], t3[r], t4[r], gimg);
         return;
     }
     // [share][tile][plane][64][64]
@@ -285,10 +314,10 @@ __global__ void __launch_bounds__(256) k_vis_adj_part(const float *gre, const fl
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int at = (wr + 8 * (r >> 2) + 4 * kh + (r & 3)) * 64 + wc + i32;
-        o[at] = p1[r];
-        o[at + 4096] = p2[r];
-        o[at + 2 * 4096] = p3[r];
-        o[at + 3 * 4096] = p4[r];
+        o[at] = t1[r];
+        o[at + 4096] = t2[r];
+        o[at + 2 * 4096] = t3[r];
+        o[at + 3 * 4096] = t4[r];
     }
 }
 
@@ -815,9 +844,9 @@ int vis_adjoint_run(rt_ctx *ctx, const float *d_gre, const float *d_gim, int nx,
     const size_t need = vis_adjoint_workspace(ctx, nx, ny, K);
     auto tiled = [&](void *part) {
         const AdjSplit a = adj_split(ctx, nx, ny, K);
-        hipLaunchKernelGGL(k_vis_adj_part, dim3(a.tx, a.ty, a.splits), dim3(256), 0, sm, d_gre,
-                           d_gim, nx, ny, d_u, d_v, K, dxy, dra, ddec, a.per, (float *)part,
-                           d_g_img);
+        hipLaunchKernelGGL(a.wpc == 3 ? k_vis_adj_part<3> : k_vis_adj_part<2>,
+                           dim3(a.tx, a.ty, a.splits), dim3(256), 0, sm, d_gre, d_gim, nx, ny, d_u,
+                           d_v, K, dxy, dra, ddec, a.per, (float *)part, d_g_img);
         if (part)
             hipLaunchKernelGGL(k_vis_adj_sum, dim3(a.tx, a.ty, 16), dim3(256), 0, sm,
                                (const float *)part, a.splits, nx, ny, d_g_img);
