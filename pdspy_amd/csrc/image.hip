@@ -105,18 +105,30 @@ __device__ __forceinline__ double sqrt_d(double x) {
     return fma(fma(-g, g, x), h, g);
 }
 
-// 1 - e^-x for x >= 0: its series up to x^8 / 8! below 0.5 (the rest is below
-// 1e-8 of it), the difference above
+// e^-x = s (1 + m) for x >= 0: s a power of two, m = e^r - 1 of the rest r of the
+// division by ln 2 (in two parts), |r| < 0.36, or of -x itself below 0.5, by its series
+// up to r^8 / 8!
+__device__ __forceinline__ void exp_parts(float x, float &s, float &m) {
+    const float y = x > 1000.f ? 1000.f : x;  // (NaN stays)
+    const float n = y < 0.5f ? 0.f : rintf(y * -1.44269504f);
+    float r = fmaf(n, -0.693145751953125f, -y);
+    r = fmaf(n, -1.42860682e-6f, r);
+    float p = 1.f / 40320.f;
+    p = fmaf(p, r, 1.f / 5040.f);
+    p = fmaf(p, r, 1.f / 720.f);
+    p = fmaf(p, r, 1.f / 120.f);
+    p = fmaf(p, r, 1.f / 24.f);
+    p = fmaf(p, r, 1.f / 6.f);
+    p = fmaf(p, r, 0.5f);
+    m = fmaf(r, p * r, r);
+    s = ldexpf(1.f, (int)n);
+}
+
+// 1 - e^-x to 7.2e-8 (rounding alone: 6e-8)
 __device__ __forceinline__ float one_minus_exp(float x) {
-    float p = -1.f / 40320.f;
-    p = fmaf(p, x, 1.f / 5040.f);
-    p = fmaf(p, x, -1.f / 720.f);
-    p = fmaf(p, x, 1.f / 120.f);
-    p = fmaf(p, x, -1.f / 24.f);
-    p = fmaf(p, x, 1.f / 6.f);
-    p = fmaf(p, x, -0.5f);
-    p = fmaf(p, x, 1.f);
-    return x < 0.5f ? p * x : 1.f - __expf(-x);
+    float s, m;
+    exp_parts(x, s, m);
+    return fmaf(-s, m, 1.f - s);
 }
 
 // cells of the unfolded theta axis, its walls' cosines (descending) and the
@@ -416,10 +428,10 @@ struct RaySum {
 
 // 1 - e^-dtau and e^-dtau as two numbers that sum to 1
 __device__ __forceinline__ void absorb(float dtau, double &om, double &e) {
-    const bool thin = dtau < 0.5f;
-    const double x = thin ? (double)one_minus_exp(dtau) : (double)__expf(-dtau);
-    om = thin ? x : 1.0 - x;
-    e = thin ? 1.0 - x : x;
+    float s, m;
+    exp_parts(dtau, s, m);
+    om = fma(-(double)s, (double)m, 1.0 - (double)s);
+    e = fma((double)s, (double)m, (double)s);
 }
 
 // The formal solution along the ray by L neighbouring lanes; every lane gets the

@@ -1032,3 +1032,33 @@ def test_vis_adjoint_of_large_images_keeps_its_digits(ny, nx, K):
     err = float(((got - ref).pow(2).mean() / ref.pow(2).mean()).sqrt())
     print("rms error / rms gradient %.2e" % err, flush=True)
     assert err <= 1.1e-6
+
+
+@pytest.mark.parametrize("rho", [1e-16, 1e-15, 1e-14, 5e-14])
+def test_emission_of_one_segment_keeps_its_digits(rho):
+    """Rays through one cell, tau 0.01 to 60: intensity over source against
+    1 - e^-tau of the tau the same ray has.  The factor is good to 7.2e-8 (its
+    series and reduction evaluated in FP32 steps over all arguments), its product
+    with the source rounds to 6e-8."""
+    print("case: one segment, rho %g" % rho, flush=True)
+    npix, pix = 256, 201.0 / 256
+    lam = np.logspace(-1, 4, 20)
+    arr = dict(rw=np.array([1.0, 100.0]) * AU, tw=np.array([0, np.pi]), pw=np.array([0, 2 * np.pi]),
+               rho=np.full((1, 1, 1, 1), rho), lam_um=lam, kabs=np.ones((1, 20)),
+               ksca=np.zeros((1, 20)), gsca=None, stars=np.array([[7e10, 4000.0, 0.0, 0.0, 0.0]]))
+    T = torch.full((1,), 100.0, device="cuda")
+
+    def image(arr, mode):
+        dm = _dev(arr)
+        cam = dm.camera(npix, pix * AU, 500.0, mode=mode, incl=30.0, incl_star=False,
+                        tau_stop=1e30)
+        return dm.image(cam, T).double().cpu().numpy()
+
+    tau, I = image(arr, 1), image(arr, 0)
+    S = image(dict(arr, rho=np.full((1, 1, 1, 1), 1e-9)), 0)[npix // 2 + 20, npix // 2]
+    x = (np.arange(npix) - npix // 2) * pix
+    sel = (np.hypot(x[:, None], x[None]) > 1.01) & (tau > 0)  # beside the hole
+    want = -np.expm1(-tau[sel])
+    err = np.abs(I[sel] / S - want) / want
+    print("largest error %.2e over tau %.2g..%.2g" % (err.max(), tau[sel].min(), tau[sel].max()))
+    assert sel.sum() > 20000 and err.max() <= 1.32e-7
