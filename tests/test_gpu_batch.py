@@ -122,3 +122,34 @@ def test_batch_step_graph_replays_match_eager():
             assert _close(got[2][i], exp[2][i], 1e-6), (k, i)
             assert _close(got[3][i], exp[3][i], 1e-4), (k, i)
             assert _close(got[4][i], exp[4][i], 1e-4), (k, i)
+
+
+def test_batch_gradients_with_the_tiled_transpose_and_growing_scratch():
+    """Five models on four chain streams, 4000 points (above the line from which the
+    transposed DFT splits its points and needs scratch): gradients as by the
+    single-model calls.  The same batch then takes 9000 points, eagerly and
+    captured, and 4000 again: its scratch grows in between, and every result is bit
+    for bit that of a batch made for those points."""
+    print("case: tiled transpose in a batch, K=4000, 9000, 4000", flush=True)
+    params = _small_params() + _small_params()[:2]
+    for k, p in enumerate(params):
+        p.update(incl=20.0 + 13.0 * k, nphot=8000)
+    kw = dict(npix=32, max_events=100000)
+    a = SamplerStep(params, K=4000, **kw)
+    b = SamplerStep(params, K=9000, **kw)
+
+    def run(batch, items, graph):
+        for x in items.img + items.g_T + items.g_logrho + items.chi2:
+            x.fill_(-1.0)
+        batch.step(items.items(), a.nphot, np.arange(a.n) + 5000, use_graph=graph, **a.opts)
+        return [x.cpu().numpy().copy() for x in items.img + items.g_T + items.g_logrho + items.chi2]
+
+    want = {4000: run(a.batch, a, False), 9000: run(b.batch, b, False)}
+    for i in range(a.n):
+        img, c2, glr, gT = a.single_model(i, 5000 + i)
+        assert float(c2.item()) == pytest.approx(float(want[4000][3 * a.n + i][0]), rel=1e-5)
+        for x, y in ((gT, want[4000][a.n + i]), (glr, want[4000][2 * a.n + i])):
+            assert np.abs(y).max() > 0 and _close(x.cpu().numpy(), y, 1e-4)
+    for items, graph in ((b, False), (a, True), (b, True), (b, True), (a, True), (a, False)):
+        for x, y in zip(run(a.batch, items, graph), want[items.u.numel()]):
+            assert np.array_equal(x, y)

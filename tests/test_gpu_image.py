@@ -1062,3 +1062,36 @@ def test_emission_of_one_segment_keeps_its_digits(rho):
     err = np.abs(I[sel] / S - want) / want
     print("largest error %.2e over tau %.2g..%.2g" % (err.max(), tau[sel].min(), tau[sel].max()))
     assert sel.sum() > 20000 and err.max() <= 1.32e-7
+
+
+@pytest.mark.parametrize("nr,nt,pw,full", [
+    (1, 1, [0, 2 * np.pi], False), (1, 1, [0, 2 * np.pi], True), (2, 1, [0, 2 * np.pi], False),
+    (3, 5, [0, np.pi, 2 * np.pi], False), (6, 7, [0, 2 * np.pi], True),
+    (6, 8, [0, 1.0, 2.5, 4.0, 2 * np.pi], True)])
+@pytest.mark.parametrize("npix,nsub", [(1, 1), (1, 2), (3, 1)])
+def test_central_rays_match_oracle(nr, nt, pw, full, npix, nsub):
+    """The smallest images, whose central ray passes through the origin (moved off
+    it by 1e-12 of the radius) in none of these grids' walls, or whose four rays
+    pass beside it: image and gradients, no pixel left out.  Optical depths up to
+    4: at 20 and more the oracle's own gradient, a difference of intensities in
+    FP64, begins to lose its digits."""
+    print("case: central ray %dx%dx%d full=%s npix=%d nsub=%d" % (nr, nt, len(pw) - 1, full, npix,
+                                                                  nsub), flush=True)
+    arr, T = _small_grid(nr, nt, pw, full, 7 * nr + npix)
+    arr["rho"] = 0.05 * arr["rho"]
+    dm = _dev(arr)
+    kaps = [rt._loglog_interp(np.array([500.0]), arr["lam_um"], k)[0] for k in arr["kabs"]]
+    kw = dict(incl=53.0, phi=23.0, lam_um=500.0, incl_star=False, nsub=nsub)
+    pix = 60.0 * AU
+    cam = dm.camera(npix, pix, pa=17.0, **kw)
+    Td = torch.tensor(T, dtype=torch.float32, device="cuda")
+    img = dm.image(cam, Td).double().cpu().numpy()
+    ref = oracle.image(arr, T, kaps, npix, pix, posang=17.0, **kw)
+    assert ref.min() > 0
+    assert np.abs(img - ref).max() <= 2e-5 * ref.max()
+    dimg = np.random.default_rng(1).uniform(0.5, 1.5, (npix, npix)).astype(np.float32)
+    glr, gT = dm.image_adjoint(cam, Td, None, torch.tensor(dimg, device="cuda"))
+    rlr, rT = oracle.image_adjoint(arr, T, kaps, dimg, npix, pix, posang=17.0, **kw)
+    assert np.abs(rT).max() > 0 and np.abs(rlr).max() > 0
+    assert np.abs(glr.double().cpu().numpy() - rlr).max() <= 5e-5 * np.abs(rlr).max()
+    assert np.abs(gT.double().cpu().numpy() - rT).max() <= 5e-5 * np.abs(rT).max()

@@ -249,3 +249,34 @@ def test_walks_leave_a_run_as_it_is(model):
                                                        "n_escape", "n_killed", "n_mrw")]))
     assert out[0][1] == out[1][1]
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("model", ["one group", "two groups", "forward"])
+@pytest.mark.parametrize("max_events", [69, 133, 1000, 20000])
+def test_walk_inside_a_thick_cell_tallies_what_the_loop_does(model, max_events):
+    """A walk needs more than eight interactions left in the packet's slice, so with
+    slices of eight there are none.  In a run's first epoch a slice only decides
+    which slot a deposit goes to: the temperatures, which come from every deposit of
+    two packets in cells of optical depth 1e6, and the counts are equal bit for bit
+    with walks and without."""
+    print("case: thick cell against the loop, %s, max_events %d" % (model, max_events), flush=True)
+    if model == "forward":
+        arr = oracle_arrays(configs.spiral_3d(nr=4, nt=4, nphi=3))
+    else:
+        arr = oracle_arrays(configs.disk_envelope(nr=4, nt=2))
+    if model == "two groups":
+        lam = arr["lam_um"]
+        arr["kabs"] = np.array(arr["kabs"], dtype=float)
+        arr["kabs"][0] = np.where(lam > 1.0, 1e3 * lam ** -0.6, 1e3)
+    # (at 1e9 the adds, in units of 2^-28 of the largest, would round to 0)
+    k = np.asarray(arr["kabs"]).max()
+    arr["rho"] = np.broadcast_to(1e6 / (k * np.diff(arr["rw"])), arr["rho"].shape).copy()
+    out = []
+    for slice_events in (8, 10000):
+        dm = rt.DeviceModel(arr)
+        st = dm.thermal(2, 5, max_events=max_events, slice_events=slice_events)
+        assert st["n_epochs"] == 1 and st["n_killed"] == 2
+        assert st["n_events"] == 2 * max_events == st["n_abs"] + st["n_scat"]
+        out.append((dm.temperature(), [st[k] for k in ("n_cross", "n_abs", "n_scat")]))
+    assert out[0][1] == out[1][1] and np.array_equal(out[0][0], out[1][0])
+    assert out[0][0].max() > 0
