@@ -300,7 +300,11 @@ int rt_get_temperature_device(rt_model *m, float *d_T);
 int rt_image(rt_model *m, const rt_camera *cam, const float *d_T, const float *d_rho,
              float *d_img);
 /* Adjoint of rt_image: given d_dimg = dL/dimg, writes dL/dlog(rho)
- * [nspec][cells] and dL/dT [cells].  tau is recomputed, not stored. */
+ * [nspec][cells] and dL/dT [cells].  tau is recomputed, not stored.  Not the
+ * transpose of rt_image to the last digit: the image crosses the cells in closed
+ * form (FP64), the adjoint marches in FP32 from wall to wall, and where a ray
+ * grazes a cone for long the two charge its path to the neighbouring cells
+ * differently, by up to 1.1e-3 of the largest gradient in such cells. */
 int rt_image_adjoint(rt_model *m, const rt_camera *cam, const float *d_T,
                      const float *d_rho, const float *d_dimg, float *d_g_logrho,
                      float *d_g_T);
@@ -308,7 +312,10 @@ int rt_image_adjoint(rt_model *m, const rt_camera *cam, const float *d_T,
 /* Visibilities of an image at K (u,v) points (wavelengths):
  * V = sum_jk I[j][k] exp(-2 pi i (u x_k + v y_j)), x_k = (k - nx/2) dxy,
  * y_j = (j - ny/2) dxy (rad), phase centre shifted by (dra, ddec) rad.
- * On the FFT grid this equals imtovis (imtovis.py:13-24). */
+ * On the FFT grid this equals imtovis (imtovis.py:13-24).  ny <= 1024.  The sums are
+ * of the differences of mirrored pixels: with a pixel that is not finite (or
+ * above FLT_MAX / 4) the visibilities are NaN or infinite, which of the two is not
+ * defined; so it is for the transpose and the gridded sampler. */
 int rt_vis_dft(rt_ctx *ctx, const float *d_img, int nx, int ny, double dxy,
                const double *d_u, const double *d_v, int K, double dra, double ddec,
                float *d_re, float *d_im);

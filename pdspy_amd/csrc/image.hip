@@ -87,6 +87,7 @@ struct RayGeo {
     bool flip;     // z reflected
 };
 
+// reciprocal: two Newton steps on the hardware's estimate
 __device__ __forceinline__ double rcp_d(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(fma(-x, r, 1.0), r, r);
@@ -94,7 +95,8 @@ __device__ __forceinline__ double rcp_d(double x) {
 }
 
 // square root to a few ulp (positive arguments far from the ends of the range;
-// anything below counts as 1e-280), without the library's scaling
+// anything below counts as 1e-280): Goldschmidt's iteration on the hardware's estimate
+// of 1 / sqrt(x) and a last Newton step, without the library's scaling
 __device__ __forceinline__ double sqrt_d(double x) {
     x = fmax(x, 1e-280);
     const double y = __builtin_amdgcn_rsq(x);
@@ -329,7 +331,7 @@ __device__ __forceinline__ void walk_ray(const CamParams &C, const RayGeo &q, in
 // gradient to its neighbour, and either is as good.  The adjoint keeps the FP32
 // march from wall to wall (next_wall) that defines those gradients, and takes
 // from the sequences above only where a lane's share begins: at a radial
-// crossing, where the march sets its position on the line again (cross_cam) and
+// crossing, where the march sets its position on the line again (put_on_sphere) and
 // so depends on nothing before it.
 struct CamRay {
     float x0, y0, z0;  // p0 (au)
@@ -709,9 +711,9 @@ __global__ void __launch_bounds__(IMG_BS) k_image_adj(CamParams C, const float *
 // as pdspy leaves them at RADMC-3D's defaults): a (sub)pixel of side d whose
 // central ray crosses a cell of size l with d > crit l is replaced by the mean
 // of its 2 x 2 sub-pixels.  Done breadth first over a node pool: every node of
-// level L is traced by one lane, which hands its four children (at most
-// RT_MAX_REFINE levels deep) their slots in level L + 1 with one atomic per
-// wavefront; the values are then averaged bottom-up, level by level.  Siblings
+// level L is traced by ref_lanes of the level's size, the first of which hands its
+// four children (at most RT_MAX_REFINE levels deep) their slots in level L + 1 with
+// one atomic per wavefront; the values are then averaged bottom-up, level by level.  Siblings
 // are summed in a fixed order, so the image does not depend on the order in
 // which slots were handed out.  The adjoint hands each leaf ray the pixel's
 // cotangent divided by 4 per level and runs the per-ray reverse sweep.

@@ -508,7 +508,8 @@ __device__ __forceinline__ void flush_counts(const ThermParams &R, int lane, uns
 // 3500 clocks, replay 15 000, about 20 interactions; a pass of the loop 8000).
 // Waves with 4 live packets (8: the same, 16: 854 against 786 ms at 5e6 packets; 2:
 // 1e4 packets of disk and envelope 187 against 154); from optical depth 1 (3: 200
-// against 189).
+// against 189).  The instances for more than two species have no walks: which group
+// absorbs is told from the first species' share alone.
 #define RT_WALK_LIVE 4    // waves with at most this many live packets look for walks
 #define RT_WALK_FROM 2    // interactions in the cell before a packet is looked at
 #define RT_WALK_MIN 1.0f  // optical depth to the bound from which a walk is worth its draws

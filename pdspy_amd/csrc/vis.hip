@@ -20,6 +20,8 @@
 #include "rt_internal.h"
 
 #define VIS_BS 256
+// More rows are an error of rt_vis_dft, as they were when its kernel held whole columns
+// in LDS; this one has no such bound, but a call that was refused stays refused
 #define VIS_MAXROWS 1024
 #define VIS_TK 32  // columns (of the folded image) per staged tile
 #define VIS_REF 8  // matrix-core steps between exact phasors
