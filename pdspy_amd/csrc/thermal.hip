@@ -594,6 +594,28 @@ __device__ __forceinline__ float lanef(float v, int src) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
 }
 
+// A lane's packet while the wave replays walks.  The replay wants most of the registers
+// for itself.  In the batched (2, 1) instance 41 of them were spilled, in the loop that
+// crosses cells too: 64 models with 2.8e8 packets 25.1 s, no faster than before there
+// were walks (25.0).  With the packets put into memory for the replay and read back
+// from there the loop has none: 22.9 s.  The other instances (18 spilled around the
+// replay in the plain one, none) keep them where the compiler has them: in memory the
+// walks of the longest packets take 2 % longer.
+template <int MS, int MG>
+struct WalkState {
+    float x, y, z, dx, dy, dz, tau, aRc, rcache[MS], xcache[MG];
+    int ir, it, ip, hemi, ifr, ps;
+    uint32_t krng, nev, nstep, nev_cell, nzero, slice_left, ovf;
+    uint64_t pid;
+    unsigned long long acc[MG];
+    double ssum;
+};
+// what lies at w may have been read and written: it is there and nowhere else
+template <class W>
+__device__ __forceinline__ void in_memory(W &w) {
+    __asm__ volatile("" : : "v"(&w) : "memory");
+}
+
 // One persistent launch for a batch of runs (one model each).  Each wavefront
 // serves one run at a time: its LDS slice holds that run's opacities and
 // walls; when it has no packet left and the run has none to hand out (all
@@ -863,30 +885,48 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                         const CellWalls w = cell_walls(g, p.ir, p.it, p.ip);
                         el = a * walk_bound(w, p.x, p.y, p.z) > RT_WALK_MIN;
                     }
-                    for (uint64_t todo = __ballot(el); todo; todo &= todo - 1ull) {
+                    const uint64_t walkers = __ballot(el);
+                    constexpr bool MEM = BATCH && MG == 1;  // the packets in memory meanwhile
+#define RT_WALK(f, reg) (MEM ? ws.f : (reg))
+                    WalkState<MS, MG> ws;
+                    if (MEM && walkers) {
+                        ws.x = p.x, ws.y = p.y, ws.z = p.z;
+                        ws.dx = p.dx, ws.dy = p.dy, ws.dz = p.dz;
+                        ws.ir = p.ir, ws.it = p.it, ws.ip = p.ip, ws.hemi = p.hemi;
+                        ws.tau = tau, ws.aRc = aRc, ws.ifr = ifr, ws.ps = ps;
+                        ws.krng = krng, ws.nev = nev, ws.nstep = nstep, ws.nev_cell = nev_cell;
+                        ws.nzero = nzero, ws.slice_left = slice_left, ws.ovf = ovf;
+                        ws.pid = pid, ws.ssum = ssum;
+#pragma unroll
+                        for (int s = 0; s < MS; ++s) ws.rcache[s] = rcache[s];
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) ws.xcache[q] = xcache[q], ws.acc[q] = acc[q];
+                    }
+                    for (uint64_t todo = walkers; todo; todo &= todo - 1ull) {
+                        if (MEM) in_memory(ws);
                         const int L = (int)uniform32(
                             (unsigned)(__ffsll((unsigned long long)todo) - 1));
                         // the packet of lane L, the same in every lane
-                        const uint64_t w_pid = lane64(pid, L);
-                        const uint32_t k0 = (uint32_t)__builtin_amdgcn_readlane((int)krng, L);
-                        const uint32_t w_nev = (uint32_t)__builtin_amdgcn_readlane((int)nev, L);
-                        const uint32_t w_nc = (uint32_t)__builtin_amdgcn_readlane((int)nev_cell, L);
-                        const uint32_t w_sl = (uint32_t)__builtin_amdgcn_readlane((int)slice_left, L);
+                        const uint64_t w_pid = lane64(RT_WALK(pid, pid), L);
+                        const uint32_t k0 = (uint32_t)__builtin_amdgcn_readlane((int)RT_WALK(krng, krng), L);
+                        const uint32_t w_nev = (uint32_t)__builtin_amdgcn_readlane((int)RT_WALK(nev, nev), L);
+                        const uint32_t w_nc = (uint32_t)__builtin_amdgcn_readlane((int)RT_WALK(nev_cell, nev_cell), L);
+                        const uint32_t w_sl = (uint32_t)__builtin_amdgcn_readlane((int)RT_WALK(slice_left, slice_left), L);
                         uint32_t nmax = min(64u, w_sl - 1u);
                         if (P.max_events)
                             nmax = min(nmax, (uint32_t)std::min<uint64_t>(
                                                  64u, P.max_events - 1u - std::min<uint64_t>(
                                                           P.max_events - 1u, w_nev)));
-                        const int w_ir = __builtin_amdgcn_readlane(p.ir, L);
+                        const int w_ir = __builtin_amdgcn_readlane(RT_WALK(ir, p.ir), L);
                         const CellWalls w =
-                            cell_walls(g, w_ir, __builtin_amdgcn_readlane(p.it, L),
-                                       __builtin_amdgcn_readlane(p.ip, L));
+                            cell_walls(g, w_ir, __builtin_amdgcn_readlane(RT_WALK(it, p.it), L),
+                                       __builtin_amdgcn_readlane(RT_WALK(ip, p.ip), L));
                         const float inv = s_invdr[w_ir];
                         float rho[MS], xr[MG];
 #pragma unroll
-                        for (int s = 0; s < MS; ++s) rho[s] = lanef(rcache[s], L);
+                        for (int s = 0; s < MS; ++s) rho[s] = lanef(RT_WALK(rcache[s], rcache[s]), L);
 #pragma unroll
-                        for (int q = 0; q < MG; ++q) xr[q] = lanef(xcache[q], L);
+                        for (int q = 0; q < MG; ++q) xr[q] = lanef(RT_WALK(xcache[q], xcache[q]), L);
                         // this lane's interaction of the next 64
                         float u[8];
                         rng8(P.seed, w_pid, k0 + (uint32_t)lane, u);
@@ -921,10 +961,12 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                                 ek[q][t] = (MG == 1 || (q < G && t < G)) ? s_gka[t * NL + ec[q]] : 0.f;
                         }
                         // the packet's own state
-                        int f = __builtin_amdgcn_readlane(ifr, L);
-                        float x = lanef(p.x, L), y = lanef(p.y, L), z = lanef(p.z, L);
-                        float dx = lanef(p.dx, L), dy = lanef(p.dy, L), dz = lanef(p.dz, L);
-                        float tl = lanef(tau, L), aR = lanef(aRc, L);
+                        int f = __builtin_amdgcn_readlane(RT_WALK(ifr, ifr), L);
+                        float x = lanef(RT_WALK(x, p.x), L), y = lanef(RT_WALK(y, p.y), L),
+                              z = lanef(RT_WALK(z, p.z), L);
+                        float dx = lanef(RT_WALK(dx, p.dx), L), dy = lanef(RT_WALK(dy, p.dy), L),
+                              dz = lanef(RT_WALK(dz, p.dz), L);
+                        float tl = lanef(RT_WALK(tau, tau), L), aR = lanef(RT_WALK(aRc, aRc), L);
                         float cabs = 0.f, csca = 0.f, c0 = 0.f, ck[MG];
 #pragma unroll
                         for (int s = 0; s < MS; ++s)
@@ -1146,26 +1188,35 @@ k_thermal(BatchArgs A, const ThermParams *__restrict__ runs, ThermParams P1) {
                             }
                         }
                         if (lane == L) {
-                            p.x = x;
-                            p.y = y;
-                            p.z = z;
-                            p.dx = dx;
-                            p.dy = dy;
-                            p.dz = dz;
-                            tau = tl;
-                            ifr = f;
-                            aRc = aR;
-                            krng += n;
-                            nev += n;
-                            nev_cell += n;
-                            slice_left -= n;
-                            if (n) nzero = 0;
+                            RT_WALK(x, p.x) = x, RT_WALK(y, p.y) = y, RT_WALK(z, p.z) = z;
+                            RT_WALK(dx, p.dx) = dx, RT_WALK(dy, p.dy) = dy, RT_WALK(dz, p.dz) = dz;
+                            RT_WALK(tau, tau) = tl, RT_WALK(ifr, ifr) = f, RT_WALK(aRc, aRc) = aR;
+                            RT_WALK(krng, krng) += n;
+                            RT_WALK(nev, nev) += n;
+                            RT_WALK(nev_cell, nev_cell) += n;
+                            RT_WALK(slice_left, slice_left) -= n;
+                            if (n) RT_WALK(nzero, nzero) = 0;
 #pragma unroll
-                            for (int q = 0; q < MG; ++q) acc[q] += add[q];
+                            for (int q = 0; q < MG; ++q) RT_WALK(acc[q], acc[q]) += add[q];
                             crow[5] += n;
                             crow[2] += nsc;
                             crow[1] += n - nsc;
                         }
+                    }
+#undef RT_WALK
+                    if (MEM && walkers) {
+                        in_memory(ws);
+                        p.x = ws.x, p.y = ws.y, p.z = ws.z;
+                        p.dx = ws.dx, p.dy = ws.dy, p.dz = ws.dz;
+                        p.ir = ws.ir, p.it = ws.it, p.ip = ws.ip, p.hemi = ws.hemi;
+                        tau = ws.tau, aRc = ws.aRc, ifr = ws.ifr, ps = ws.ps;
+                        krng = ws.krng, nev = ws.nev, nstep = ws.nstep, nev_cell = ws.nev_cell;
+                        nzero = ws.nzero, slice_left = ws.slice_left, ovf = ws.ovf;
+                        pid = ws.pid, ssum = ws.ssum;
+#pragma unroll
+                        for (int s = 0; s < MS; ++s) rcache[s] = ws.rcache[s];
+#pragma unroll
+                        for (int q = 0; q < MG; ++q) xcache[q] = ws.xcache[q], acc[q] = ws.acc[q];
                     }
                 }
             }

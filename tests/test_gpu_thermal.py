@@ -280,3 +280,9 @@ def test_walk_inside_a_thick_cell_tallies_what_the_loop_does(model, max_events):
         out.append((dm.temperature(), [st[k] for k in ("n_cross", "n_abs", "n_scat")]))
     assert out[0][1] == out[1][1] and np.array_equal(out[0][0], out[1][0])
     assert out[0][0].max() > 0
+    # the batched instances' walks (the one-group one has its packets in memory meanwhile)
+    dms = [rt.DeviceModel(arr) for _ in range(2)]
+    st = rt.Batch(dms).thermal([2, 2], [5, 5], max_events=max_events)
+    for dm, s in zip(dms, st):
+        assert [s[k] for k in ("n_cross", "n_abs", "n_scat")] == out[0][1]
+        assert np.array_equal(dm.temperature(), out[0][0])
